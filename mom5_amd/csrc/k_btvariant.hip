@@ -7,7 +7,9 @@
 //   <CG=true,  PR=true>  pred_corr_tropic_press_cgrid :4355-4693
 // followed by the tail of update_ocean_barotropic (:2846-2894).
 //
-// Two launches per subcycle, each over the data domain:
+// Blocked in time where the domain allows it (k_btv_block, several subcycles a
+// launch); otherwise, and with barotropic_subcycles_per_launch = 0, two
+// launches per subcycle, each over the data domain:
 //   k_btv_velocity  udrho_bt(fstaup1) at every point.  The predicted x
 //                   (eta_t_bt or anompb_bt) is recomputed at the points the
 //                   pressure gradient needs instead of being stored; the
@@ -245,6 +247,370 @@ __global__ void k_btv_corrector(BtvArgs<CG, PR> a, int fstau, int fstaup1, doubl
   }
 }
 
+// ---- temporally blocked subcycles -----------------------------------------
+// The two-launch form above moves every plane through memory twice a subcycle.
+// Here one work-group owns a 64 x 32 region of the data domain and advances it
+// nsub subcycles with its state in registers, reading and writing the planes
+// once a launch.  80 C-grid pressure subcycles at 1440x1080: 11.4 ms with two
+// launches each (112 + 43 us), 2.2 ms in sixteen launches of five.
+//
+// A wavefront holds two neighbouring rows, so x neighbours are DPP lane shifts
+// and half of the y neighbours the thread's own registers; the other half goes
+// through LDS, one row a wavefront and quantity.  The forcing and the thickness
+// are read once a subcycle and lie in LDS too, which keeps a thread within the
+// 128 registers that 16 wavefronts a CU allow.
+//
+// Dependencies: a transport needs the transports one point away in each
+// direction, x also those of one point west and south.  After nsub subcycles a
+// region is exact from nsub + 1 points above its low edges to nsub points below
+// its high ones.  On a cyclic-x domain the reference keeps a halo column's own
+// values and only overwrites what its halo update covers (B-grid: the predicted
+// x, C-grid: the transports, compute rows), so the region runs over the data
+// columns 0 .. NI-1, 0, 1, .. and column 0 (NI-1) takes the updated quantity
+// from column NI-2 (1), two lanes to the left (right): two more halo lanes a
+// side.  A chain of dependencies crosses that seam once if ni > nsub, so
+// domains narrower than MIN_NI, and cyclic-y ones, keep the two launches.
+constexpr int VX = 64, VW = 16, VY = 2 * VW;
+constexpr int MIN_NI = 16;             // > the most subcycles a launch takes (12)
+
+__host__ __device__ constexpr int btv_lo(int nsub, bool cyc) { return nsub + 1 + (cyc ? 2 : 0); }
+__host__ __device__ constexpr int btv_tx(int nsub, bool cyc) {
+  return VX - 2 * nsub - 1 - (cyc ? 4 : 0);
+}
+__host__ __device__ constexpr int btv_ty(int nsub) { return VY - 2 * nsub - 1; }
+
+struct BtvBlk {
+  const double *xs, *us, *fs;          // state read: x, transports (2), force at two levels (4)
+  double *xd, *ud, *fd;                // state written
+  const unsigned char *mask;           // bit 0 tmask(k=1), bit 1 umask(k=1)
+  int s0, nsub, nts, step_a, ntx, ntiles;
+};
+
+// sf and the masks, constant over the subcycles
+template <bool CG, bool PR>
+__global__ void k_btv_sfmask(BtvArgs<CG, PR> a, unsigned char *__restrict__ mask) {
+  const int ii = blockIdx.x * blockDim.x + threadIdx.x, jj = blockIdx.y;
+  if (ii >= a.d.NI) return;
+  const int o = ii + a.d.NI * jj;
+  const double tm = tm1(a.kmt, o);
+  const double s = a.pme[o] + a.river[o] + a.source[o] - a.smooth[o];
+  a.sf[o] = PR ? tm * (a.grav * s + a.dpatm_dt[o]) : tm * s;
+  mask[o] = (unsigned char)((1 <= a.kmt[o] ? 1 : 0) | (1 <= a.kmu[o] ? 2 : 0));
+}
+
+template <bool CG, bool PR>
+__global__ __launch_bounds__(VX *VW) void k_btv_block(BtvArgs<CG, PR> a, BtvBlk J, int per_xcd) {
+  const int b = blockIdx.x;
+  const int t0 = (b & 7) * per_xcd + (b >> 3);
+  if (t0 >= J.ntiles) return;                  // the whole block
+  const int tile = strip_tile<8>(t0, J.ntx, J.ntiles / J.ntx);
+  const KDom d = a.d;
+  const int P2 = d.P2, nsub = J.nsub;
+  const bool cyc = d.cyclic_x != 0;
+  __shared__ double s_p[VW][VX], s_v[VW][VX];             // p of the low rows, vh of the high
+  __shared__ double s_u1[VW][VX], s_u2[VW][VX];           // C: u1 of the low rows, u2 of the high
+  // forcing (2), thickness (C: 2); C-grid depth: rho_g, patm
+  constexpr bool PL = CG && !PR;
+  __shared__ double s_c[PL ? 6 : (CG ? 4 : 3)][2][VW][VX];
+  const int lane = threadIdx.x & (VX - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / VX);
+  const int wm = max(wave - 1, 0), wp = min(wave + 1, VW - 1);
+  const int LX = btv_lo(nsub, cyc), LY = btv_lo(nsub, false);
+  const int TX = btv_tx(nsub, cyc), TY = btv_ty(nsub);
+  const int seq = (tile % J.ntx) * TX - LX + lane;        // position in the column sequence
+  const int col = cyc ? wrapi(seq, d.NI) : seq;
+  const int row0 = (tile / J.ntx) * TY - LY + 2 * wave;
+  const bool colok = cyc || (seq >= 0 && seq < d.NI);
+  // a region that holds the seam of a cyclic-x domain (uniform)
+  const int seq0 = (tile % J.ntx) * TX - LX;
+  const bool seam = cyc && (seq0 <= 0 || seq0 + VX > d.NI - 2);
+  const bool first = J.s0 == 1;
+
+  int off[2];
+  bool in[2], tmb[2], umb[2], div0[2], grad0[2], comp[2], fromw[2], frome[2];
+  double x[2], u1[2], u2[2], fa1[2], fa2[2], fb1[2], fb2[2], sx[2], su1[2], su2[2];
+  double datr[2], m1[2], m2[2], g1c[2], g2c[2], k1[2], k2[2], f[2], sf[2], rg[2], pa[2];
+  double fS = 0.0;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int j = row0 + q;
+    const bool present = colok && j >= 0 && j < d.NJ;
+    const bool crow = j >= 1 && j <= d.nj;
+    const int o = present ? col + d.NI * j : 0;
+    off[q] = o;
+    in[q] = present && lane >= LX && lane < LX + TX && seq < d.NI && 2 * wave + q >= LY &&
+            2 * wave + q < LY + TY;
+    div0[q] = col == 0 || j == 0;
+    grad0[q] = col == d.NI - 1 || j == d.NJ - 1;
+    comp[q] = crow && col >= 1 && col <= d.ni;
+    fromw[q] = cyc && crow && col == 0;
+    frome[q] = cyc && crow && col == d.NI - 1;
+    double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
+    tmb[q] = umb[q] = false;
+    x[q] = u1[q] = u2[q] = fa1[q] = fa2[q] = fb1[q] = fb2[q] = sx[q] = su1[q] = su2[q] = 0.0;
+    datr[q] = m1[q] = m2[q] = g1c[q] = g2c[q] = k1[q] = k2[q] = f[q] = sf[q] = rg[q] = pa[q] = 0.0;
+    if (present) {
+      const unsigned char mb = J.mask[o];
+      tmb[q] = (mb & 1) != 0;
+      umb[q] = (mb & 2) != 0;
+      x[q] = J.xs[o]; u1[q] = J.us[o]; u2[q] = J.us[o + P2];
+      sf[q] = a.sf[o]; datr[q] = a.datr[o]; f[q] = a.f[o];
+      c0 = a.forcing[o]; c1 = a.forcing[o + P2];
+      c2 = a.thick[o];
+      if (!PR) { rg[q] = a.rho_g[o]; pa[q] = a.patm[o]; }
+      if (CG) {
+        c3 = a.thick[o + P2];
+        m1[q] = a.dat[o];
+        g1c[q] = 1.0 / (a.dxte[o] + kEpsln);
+        g2c[q] = 1.0 / (a.dytn[o] + kEpsln);
+        k1[q] = a.tmasken[o]; k2[q] = a.tmasken[o + P2];
+        if (!first) {
+          fa1[q] = J.fs[o]; fa2[q] = J.fs[o + P2];
+          fb1[q] = J.fs[o + 2 * (size_t)P2]; fb2[q] = J.fs[o + 3 * (size_t)P2];
+        }
+        if (q == 0) fS = j >= 1 ? a.f[o - d.NI] : 0.0;
+      } else {
+        m1[q] = a.dyu[o]; m2[q] = a.dxu[o];
+        g1c[q] = a.dxur[o]; g2c[q] = a.dyur[o];
+        k1[q] = 0.5 * a.dtbt * f[q];             // cori1, cori2 (:1285-1286)
+        k2[q] = 1.0 / (1.0 + k1[q] * k1[q]);
+      }
+      if (in[q]) {
+        if (first) {
+          sx[q] = a.initsum ? a.xbar_tau[o] : a.x_tau[o];
+        } else {
+          sx[q] = a.accx[o]; su1[q] = a.accu[o]; su2[q] = a.accu[o + P2];
+        }
+      }
+    }
+    s_c[0][q][wave][lane] = c0;
+    s_c[1][q][wave][lane] = c1;
+    s_c[2][q][wave][lane] = c2;
+    if constexpr (CG) s_c[3][q][wave][lane] = c3;
+    if constexpr (PL) {
+      s_c[4][q][wave][lane] = rg[q];
+      s_c[5][q][wave][lane] = pa[q];
+    }
+  }
+  const double fW0 = lane_prev(f[0]), fW1 = lane_prev(f[1]);
+
+  // the transports through a cell's edges of both rows, those other rows read to LDS
+  double uh[2], vh[2], dv[2];
+  auto share = [&]() {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (CG) {      // DIV_UD, C-grid (ocean_operators.F90:526-536)
+        uh[q] = u1[q] * m1[q] * g1c[q];
+        vh[q] = u2[q] * m1[q] * g2c[q];
+      } else {
+        uh[q] = u1[q] * m1[q];
+        vh[q] = u2[q] * m2[q];
+      }
+    }
+    s_v[wave][lane] = vh[1];
+    if (CG) {
+      s_u1[wave][lane] = u1[0];
+      s_u2[wave][lane] = u2[1];
+    } else {
+      s_u1[wave][lane] = uh[1];
+    }
+  };
+  auto diverge = [&]() {
+    const double vs = s_v[wm][lane];
+    if (CG) {
+      dv[0] = ((uh[0] - lane_prev(uh[0])) + (vh[0] - vs)) * datr[0];
+      dv[1] = ((uh[1] - lane_prev(uh[1])) + (vh[1] - vh[0])) * datr[1];
+    } else {         // B-grid (:570-605)
+      const double us = s_u1[wm][lane];
+      const double bay0 = 0.5 * (uh[0] + us), bay1 = 0.5 * (uh[1] + uh[0]);
+      const double baxs = 0.5 * (vs + lane_prev(vs));
+      const double bax0 = 0.5 * (vh[0] + lane_prev(vh[0]));
+      const double bax1 = 0.5 * (vh[1] + lane_prev(vh[1]));
+      dv[0] = ((bay0 - lane_prev(bay0)) + (bax0 - baxs)) * datr[0];
+      dv[1] = ((bay1 - lane_prev(bay1)) + (bax1 - bax0)) * datr[1];
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      if (div0[q]) dv[q] = 0.0;
+  };
+  share();
+  __syncthreads();
+  diverge();
+
+  for (int t = 0; t < nsub; ++t) {
+    const int itime = J.s0 + t;
+    // A: the prediction and the pressure; C-grid: the Coriolis force, from
+    // the transports that the phases B before wrote
+    double F1[2], F2[2], p[2];
+    if constexpr (CG) {
+      const double u2s = s_u2[wm][lane], u1n = s_u1[wp][lane];
+      const double e0 = u2[0] + lane_next(u2[0]), e1 = u2[1] + lane_next(u2[1]);
+      const double es = u2s + lane_next(u2s);
+      F1[0] = 0.25 * (f[0] * e0 + fS * es);
+      F1[1] = 0.25 * (f[1] * e1 + f[0] * e0);
+      const double n0 = u1[0] + u1[1], n1 = u1[1] + u1n;
+      F2[0] = -(0.25 * (f[0] * n0 + fW0 * lane_prev(n0)));
+      F2[1] = -(0.25 * (f[1] * n1 + fW1 * lane_prev(n1)));
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        if (!comp[q]) F1[q] = F2[q] = 0.0;
+        if (itime == 1) {                     // all three levels (:3711-3730)
+          fa1[q] = fb1[q] = F1[q];
+          fa2[q] = fb2[q] = F2[q];
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      double e = x[q];
+      if (a.predict) {
+        const double tmp = PR ? -a.grav * dv[q] : (tmb[q] ? -dv[q] : -dv[q] * 0.0);
+        e = x[q] + a.c_pred * (tmp + sf[q]);
+      }
+      if (!CG && seam) {                      // the legacy halo update (:3383, :4140)
+        const double w = lane_prev(lane_prev(e)), n = lane_next(lane_next(e));
+        e = fromw[q] ? w : (frome[q] ? n : e);
+      }
+      if constexpr (PR)
+        p[q] = tmb[q] ? e : e * 0.0;
+      else if constexpr (PL)
+        p[q] = s_c[4][q][wave][lane] * e + s_c[5][q][wave][lane];
+      else
+        p[q] = rg[q] * e + pa[q];
+    }
+    s_p[wave][lane] = p[0];
+    __syncthreads();
+    // B: pressure gradient and transports
+    {
+      const double pn1 = s_p[wp][lane];
+      double n1[2], n2[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const double pn = q == 0 ? p[1] : pn1;
+        const double pe = lane_next(p[q]), pne = CG ? 0.0 : lane_next(pn);
+        double h1 = 0.0, h2 = 0.0;
+        if (!grad0[q]) {
+          if (CG) {    // GRAD_BAROTROPIC_P, C-grid (ocean_operators.F90:664-669)
+            h1 = (pe - p[q]) * g1c[q] * k1[q];
+            h2 = (pn - p[q]) * g2c[q] * k2[q];
+          } else {     // B-grid (:651-660)
+            const double p_fay = 0.5 * (p[q] + pn);
+            const double p_fax = 0.5 * (p[q] + pe);
+            const double pip_fay = 0.5 * (pe + pne);
+            const double pjp_fax = 0.5 * (pn + pne);
+            const double y1 = (pip_fay - p_fay) * g1c[q], y2 = (pjp_fax - p_fax) * g2c[q];
+            h1 = umb[q] ? y1 : y1 * 0.0;
+            h2 = umb[q] ? y2 : y2 * 0.0;
+          }
+        }
+        const double th1 = s_c[2][q][wave][lane], th2 = CG ? s_c[CG ? 3 : 2][q][wave][lane] : th1;
+        const double pf1 = PR ? -(a.rho0r * th1 * h1) : -(th1 * h1);
+        const double pf2 = PR ? -(a.rho0r * th2 * h2) : -(th2 * h2);
+        const double fo1 = s_c[0][q][wave][lane], fo2 = s_c[1][q][wave][lane];
+        if (CG) {
+          constexpr double ab0 = 23.0 / 12.0, ab1 = -16.0 / 12.0, ab2 = 5.0 / 12.0;  // :617-619
+          double acc1 = 0.0, acc2 = 0.0;
+          if (comp[q]) {
+            acc1 = ab0 * F1[q] + ab1 * fa1[q] + ab2 * fb1[q];
+            acc2 = ab0 * F2[q] + ab1 * fa2[q] + ab2 * fb2[q];
+          }
+          const double s1 = acc1 + pf1 + fo1, s2 = acc2 + pf2 + fo2;
+          n1[q] = u1[q] + a.dtbt * k1[q] * (PR ? s1 : s1 + 0.0);
+          n2[q] = u2[q] + a.dtbt * k2[q] * (PR ? s2 : s2 + 0.0);
+          if (seam) {                         // the halo update of udrho_bt (:3895-3897)
+            const double w1 = lane_prev(lane_prev(n1[q])), w2 = lane_prev(lane_prev(n2[q]));
+            const double e1 = lane_next(lane_next(n1[q])), e2 = lane_next(lane_next(n2[q]));
+            n1[q] = fromw[q] ? w1 : (frome[q] ? e1 : n1[q]);
+            n2[q] = fromw[q] ? w2 : (frome[q] ? e2 : n2[q]);
+          }
+          fb1[q] = fa1[q]; fb2[q] = fa2[q];
+          fa1[q] = F1[q]; fa2[q] = F2[q];
+        } else {
+          const double fo = f[q], v1 = u1[q], v2 = u2[q];
+          double r1, r2;
+          if (PR) {
+            r1 = v1 + a.dtbt * (0.5 * fo * v2 + pf1 + fo1);
+            r2 = v2 + a.dtbt * (-(0.5 * fo * v1) + pf2 + fo2);
+          } else {
+            r1 = v1 + a.dtbt * (0.5 * fo * v2 + pf1 + fo1 + 0.0);
+            r2 = v2 + a.dtbt * (-(0.5 * fo * v1) + pf2 + fo2 + 0.0);
+          }
+          n1[q] = k2[q] * (r1 + k1[q] * r2);
+          n2[q] = k2[q] * (r2 - k1[q] * r1);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) { u1[q] = n1[q]; u2[q] = n2[q]; }
+      // the reads of s_v, s_u1, s_u2 of phases C and A are behind the barrier above
+      share();
+    }
+    __syncthreads();
+    // C: corrector and time sums
+    diverge();
+    const double wgt = (double)(J.nts - itime + 1);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const double tmp = PR ? -a.grav * dv[q] : (tmb[q] ? -dv[q] : -dv[q] * 0.0);
+      x[q] = x[q] + a.c_corr * (tmp + sf[q]);
+      sx[q] = sx[q] + x[q];
+      su1[q] = su1[q] + (J.step_a ? u1[q] : wgt * u1[q]);
+      su2[q] = su2[q] + (J.step_a ? u2[q] : wgt * u2[q]);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    if (!in[q]) continue;
+    const int o = off[q];
+    J.xd[o] = x[q];
+    J.ud[o] = u1[q];
+    J.ud[o + P2] = u2[q];
+    if (CG) {
+      J.fd[o] = fa1[q];
+      J.fd[o + P2] = fa2[q];
+      J.fd[o + 2 * (size_t)P2] = fb1[q];
+      J.fd[o + 3 * (size_t)P2] = fb2[q];
+    }
+    a.accx[o] = sx[q];
+    a.accu[o] = su1[q];
+    a.accu[o + P2] = su2[q];
+  }
+}
+
+// nsub = hsub subcycles a launch; the state alternates between two sets of
+// planes of ctx->btv (a region reads its neighbours' points).
+template <bool CG, bool PR>
+int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a, int hsub) {
+  const KDom &d = a.d;
+  const size_t P2 = (size_t)d.P2;
+  hipStream_t s = ctx->stream;
+  double *w = ctx->btv;
+  unsigned char *mask = (unsigned char *)(w + 7 * P2);    // the place of cori1
+  double *xb[2] = {w, w + P2}, *ub[2] = {w + 2 * P2, w + 4 * P2};
+  double *fb[2] = {w + 8 * P2, w + 18 * P2};              // 4 planes each: 8-11, 18-21
+  hipLaunchKernelGGL((k_btv_sfmask<CG, PR>), dim3((d.NI + 255) / 256, d.NJ), dim3(256), 0, s, a,
+                     mask);
+  MOM_LAUNCHED(ctx, "k_btv_sfmask");
+  BtvBlk J{a.xbar_tau, a.ud_tau, nullptr, nullptr, nullptr, nullptr, mask, 1, 0, nts, step_a, 0, 0};
+  const bool cyc = d.cyclic_x != 0;
+  for (int which = 0; J.s0 <= nts; J.s0 += hsub, which ^= 1) {
+    J.nsub = min(hsub, nts - J.s0 + 1);
+    const int TX = btv_tx(J.nsub, cyc), TY = btv_ty(J.nsub);
+    J.ntx = (d.NI + TX - 1) / TX;
+    J.ntiles = J.ntx * ((d.NJ + TY - 1) / TY);
+    J.xd = xb[which];
+    J.ud = ub[which];
+    J.fd = fb[which];
+    const int per_xcd = (J.ntiles + 7) / 8;
+    hipLaunchKernelGGL((k_btv_block<CG, PR>), dim3(8 * per_xcd), dim3(VX * VW), 0, s, a, J,
+                       per_xcd);
+    MOM_LAUNCHED(ctx, "k_btv_block");
+    J.xs = J.xd;
+    J.us = J.ud;
+    J.fs = J.fd;
+  }
+  return MOM_GPU_OK;
+}
+
 // Tail (:2846-2894): the time means, each halo-updated, and
 // conv_rho_ud_t = -DIV_UD(udrho(taup1)) halo-updated.
 template <bool CG, bool PR>
@@ -339,19 +705,24 @@ int run_variant(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p, const mom_gpu_bt
   a.initsum = p->initsum_with_bar ? 1 : 0;
   hipStream_t s = ctx->stream;
   const dim3 grid((d.NI + 63) / 64, d.NJ), block(64);
-  hipLaunchKernelGGL((k_btv_init<CG, PR>), grid, block, 0, s, a);
-  MOM_LAUNCHED(ctx, "k_btv_init");
-  const int nts = p->nts;
-  for (int itime = 1; itime <= nts; ++itime) {
-    const int fstau = itime % 2 + 1, fstaup1 = (itime + 1) % 2 + 1;
-    const int m2 = itime % 3 + 1, m1 = (itime + 1) % 3 + 1, m0 = (itime + 2) % 3 + 1;
-    hipLaunchKernelGGL((k_btv_velocity<CG, PR>), grid, block, 0, s, a, fstau, fstaup1,
-                       m0, m1, m2);
-    const double wgt = p->stepping_a ? 0.0 : (double)(nts - itime + 1);
-    hipLaunchKernelGGL((k_btv_corrector<CG, PR>), grid, block, 0, s, a, fstau, fstaup1,
-                       wgt);
+  const int nts = p->nts, hsub = ctx->tune.bt_subcycles_per_launch;
+  if (hsub > 0 && !d.cyclic_y && (!d.cyclic_x || d.ni >= MIN_NI)) {
+    const int rc = run_blocked(ctx, a, nts, p->stepping_a, hsub);
+    if (rc) return rc;
+  } else {
+    hipLaunchKernelGGL((k_btv_init<CG, PR>), grid, block, 0, s, a);
+    MOM_LAUNCHED(ctx, "k_btv_init");
+    for (int itime = 1; itime <= nts; ++itime) {
+      const int fstau = itime % 2 + 1, fstaup1 = (itime + 1) % 2 + 1;
+      const int m2 = itime % 3 + 1, m1 = (itime + 1) % 3 + 1, m0 = (itime + 2) % 3 + 1;
+      hipLaunchKernelGGL((k_btv_velocity<CG, PR>), grid, block, 0, s, a, fstau, fstaup1,
+                         m0, m1, m2);
+      const double wgt = p->stepping_a ? 0.0 : (double)(nts - itime + 1);
+      hipLaunchKernelGGL((k_btv_corrector<CG, PR>), grid, block, 0, s, a, fstau, fstaup1,
+                         wgt);
+    }
+    MOM_LAUNCHED(ctx, "k_btv_velocity/k_btv_corrector");
   }
-  MOM_LAUNCHED(ctx, "k_btv_velocity/k_btv_corrector");
   const double rntsp1 = 1.0 / ((double)nts + 1.0);          // :2804
   const double rnts = p->stepping_a ? 1.0 / (double)nts      // :2807-2811
                                     : 2.0 / ((double)nts * (double)(nts + 1));
@@ -372,7 +743,7 @@ int launch_bt_variant(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p,
       return mom_fail(ctx, MOM_GPU_ERR_ARG,
                       "update_ocean_barotropic_variant: the first call allocates its state; "
                       "call it once before capturing a graph");
-    MOM_HIP(ctx, hipMalloc((void **)&ctx->btv, 18 * (size_t)ctx->kd.P2 * sizeof(double)));
+    MOM_HIP(ctx, hipMalloc((void **)&ctx->btv, 22 * (size_t)ctx->kd.P2 * sizeof(double)));
   }
   if (v->cgrid)
     return v->pressure_based ? run_variant<true, true>(ctx, p, v) : run_variant<true, false>(ctx, p, v);

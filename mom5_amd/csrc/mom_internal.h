@@ -154,7 +154,7 @@ struct mom_gpu_ctx {
   double bt_cori_dtbt;
   // REMAP_BT_TO_BU metrics dte, dtw, dus, dun, daur (5 planes, optional)
   double *remap;
-  // state of the barotropic variants (18 planes, allocated on first use)
+  // state of the barotropic variants (22 planes, allocated on first use)
   double *btv;
   // invtri work (e coefficients), one 3-D plane set
   double *tri_e;

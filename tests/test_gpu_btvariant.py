@@ -98,3 +98,42 @@ def test_bgrid_depth_variant_equals_blocked_path():
                           (xb.to_host(), ud.to_host(), cv.to_host())):
         assert np.array_equal(_bits(a), _bits(b)), name
     g.close()
+
+
+# The variants blocked in time: several tiles a side (odd sizes, seam of the
+# cyclic axis inside a tile's halo), every count of subcycles a launch, a last
+# launch with fewer, and halo columns that hold no wrap.
+@pytest.mark.parametrize("cyclic", [True, False])
+@pytest.mark.parametrize("cgrid,press", [(False, False), (True, False), (False, True),
+                                         (True, True)])
+def test_variant_blocked_bitwise(cyclic, cgrid, press):
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    for ni, nj, hsubs, nts in ((131, 67, (1, 2, 5, 7), 9), (16, 30, (5, 12), 13),
+                               (64, 33, (4,), 6)):
+        kw = {} if cyclic else dict(cyclic_x=False, lat_s=20.0, lat_n=50.0, lon_span=30.0)
+        c = make_case(ni, nj, 3, seed=62, land_frac=0.3, barotropic=True, **kw)
+        fl = _inputs(c, cgrid, press, seed=11)
+        H = DeviceArray.from_host
+        g = OceanGPU(c.dom, c.grid)
+        sh = fl["patm"].shape
+        kw = {k: H(v) for k, v in fl.items() if v is not None and k not in ("udrho", "xbar_tau")}
+        xbar, ud = H(fl["xbar_tau"]), H(fl["udrho"])
+        want = None
+        for stepping_a, initsum in ((False, True), (True, False)):
+            for hsub in (0,) + hsubs:
+                print(f"[barotropic variant {ni}x{nj} cyclic={cyclic} cgrid={cgrid} press={press} "
+                      f"{hsub} subcycles a launch stepping_a={stepping_a}]", flush=True)
+                g.set_tuning("barotropic_subcycles_per_launch", hsub)
+                out = DeviceArray(sh), DeviceArray((2,) + sh), DeviceArray(sh)
+                g.update_ocean_barotropic_variant(
+                    cgrid=cgrid, pressure_based=press, nts=nts, dtbt=c.dtbt, x_bar_tau=xbar,
+                    udrho_tau=ud, x_bar_taup1=out[0], udrho_taup1=out[1], conv_rho_ud_t=out[2],
+                    stepping_a=stepping_a, initsum_with_bar=initsum, **kw)
+                g.sync()
+                got = [a.to_host() for a in out]
+                if hsub == 0:
+                    want = got
+                for name, a, b in zip(("x_bar", "udrho", "conv_rho_ud_t"), got, want):
+                    assert np.array_equal(_bits(a), _bits(b)), (name, hsub)
+        g.close()
