@@ -62,3 +62,29 @@ def test_barotropic_forcing_bitwise(oracle_lib, cyclic):
     g.sync()
     assert np.array_equal(out.to_host(), ref)
     g.close()
+
+
+# Edges of the kernel's 63 x 15 regions: data domains (ni + 2) x (nj + 2) of
+# exactly one region, one point less and more, and the smallest.
+@pytest.mark.parametrize("ni,nj,nk", [(61, 13, 2), (60, 12, 3), (62, 14, 3), (124, 28, 2),
+                                      (3, 3, 2)])
+def test_advection_velocity_region_edges(oracle_lib, ni, nj, nk):
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    c = make_case(ni, nj, nk, seed=33, land_frac=0.2, barotropic=False)
+    print(f"[advection velocity {ni}x{nj}x{nk}]", flush=True)
+    NJ, NI = nj + 2, ni + 2
+    rng = np.random.default_rng(8)
+    u = rng.standard_normal((2, nk, NJ, NI)) * 0.2
+    rdu = 1035.0 * c.grid["dzt"][:, None, None] * (1.0 + 0.01 * rng.random((nk, NJ, NI)))
+    pme = 1e-4 * rng.standard_normal((NJ, NI))
+    river = 1e-4 * rng.random((NJ, NI))
+    ref = oracle_lib.Oracle(c).advection_velocity(u, rdu, pme, river)
+    g = OceanGPU(c.dom, c.grid)
+    H = DeviceArray.from_host
+    ue, vn, wb = g.field3(), g.field3(), DeviceArray((nk + 1, NJ, NI))
+    g.advection_velocity(H(u), H(rdu), H(pme), H(river), ue, vn, wb)
+    g.sync()
+    for name, got, want in zip(("uhrho_et", "vhrho_nt", "wrho_bt"), (ue, vn, wb), ref):
+        assert np.array_equal(got.to_host(), want), name
+    g.close()
