@@ -115,6 +115,28 @@ __host__ __device__ inline double fmx(double a, double b) { return (b > a) ? b :
 __host__ __device__ inline float fmnf(float a, float b) { return (b < a) ? b : a; }
 __host__ __device__ inline float fmxf(float a, float b) { return (b > a) ? b : a; }
 
+// Level-sliced addressing: a buffer descriptor of the level (the array plus
+// the level's offset, in scalar registers) and a 32-bit byte offset of the
+// point within the level, so that no lane carries a 64-bit address.  A level
+// of the largest domain is far below 4 GiB.
+__device__ inline __amdgpu_buffer_rsrc_t lvl_rsrc(const void *p) {
+  // raw buffer: stride 0, 4 GiB of records, 32-bit data format (CDNA)
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, -1, 0x00020000);
+}
+__device__ inline float ld_lv(const float *base, unsigned boff) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(lvl_rsrc(base), (int)boff, 0, 0));
+}
+__device__ inline double ld_lv(const double *base, unsigned boff) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(lvl_rsrc(base), (int)boff, 0, 0));
+}
+__device__ inline void st_lv(float *base, unsigned boff, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), lvl_rsrc(base), (int)boff, 0, 0);
+}
+__device__ inline void st_lv(double *base, unsigned boff, double v) {
+  using V2 = unsigned __attribute__((ext_vector_type(2)));
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), lvl_rsrc(base), (int)boff, 0, 0);
+}
+
 struct mom_gpu_ctx {
   mom_gpu_domain_t dom;
   KDom kd;

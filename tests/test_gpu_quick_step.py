@@ -134,3 +134,51 @@ def test_update_domains_matches_single_pe_halo_update(oracle_lib, cyclic):
                                      ref.ctypes.data_as(C.POINTER(C.c_double)), 5, 3)
     assert np.array_equal(got, ref)
     assert cyclic == (not np.array_equal(ref, a))
+
+
+# Pairs that share a pass: regions of 60 x 8 (two tracers) and 60 x 12 (one)
+# cells exactly, one more and one less, two and three levels; flags OR'ed or
+# not; other th_tendency terms on none, one or both of a pair.
+@pytest.mark.parametrize("ni,nj,nk", [(60, 8, 2), (61, 9, 3), (59, 7, 4), (121, 25, 5)])
+@pytest.mark.parametrize("schemes,ts_same,with_th", [
+    (["quicker"] * 4, True, (0, 2, 3)), (["quicker"] * 4, False, ()),
+    (["quicker", "mdfl_sweby", "quicker", "mdfl_sweby"], True, (0,)),
+    (["mdfl_sweby", "quicker", "quicker", "quicker"], False, (1, 2))])
+def test_quicker_pairs_equal_oracle(oracle_lib, ni, nj, nk, schemes, ts_same, with_th):
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    from _cases import assert_close_cells, oracle_tracer_step
+    c = make_case(ni, nj, nk, land_frac=0.2, nts=10, seed=63, n_passive=2, stf_scale=1e-3)
+    print(f"[quicker pairs {ni}x{nj}x{nk} {schemes} ts_same={ts_same} th={with_th}]", flush=True)
+    rng = np.random.default_rng(9)
+    tm = c.grid["tmask"]
+    names = [n for n, _ in c.tracers]
+    mins, maxs = _limits(names)
+    Ts = [np.asarray(t, np.float64) for _, t in c.tracers]
+    wet = np.argwhere(tm[:, 1:-1, 1:-1] > 0)
+    for n in range(4):
+        for k, j, i in wet[rng.choice(len(wet), 12, replace=False)]:
+            Ts[n][k, j + 1, i + 1] = maxs[n] + 0.5
+        Ts[n][..., 0], Ts[n][..., -1] = Ts[n][..., -2].copy(), Ts[n][..., 1].copy()
+    ths = [1e-4 * rng.standard_normal(tm.shape) * tm if n in with_th else None for n in range(4)]
+    f = c.fields
+    gpu = OceanGPU(c.dom, c.grid)
+    H = DeviceArray.from_host
+    dev = {k: H(v) for k, v in f.items() if isinstance(v, np.ndarray)}
+    tin, tout = [H(t) for t in Ts], [DeviceArray(t.shape, np.float64) for t in Ts]
+    thd = [H(t) if t is not None else None for t in ths]
+    for t in tout:
+        t.zero()
+    gpu.step_tracers(tin, tout, uhrho_et=dev["uhrho_et"], vhrho_nt=dev["vhrho_nt"],
+                     wrho_bt=dev["wrho_bt"], rho_dzt_tau=dev["rho_dzt"],
+                     rho_dztr=dev["rho_dztr"], dtime=c.dt, stfs=[H(s) for s in f["stf"]],
+                     btfs=[H(b) for b in f["btf"]], dzwt=dev["dzwt"], diff_cbt=dev["diff_cbt"],
+                     schemes=schemes, min_limits=mins, max_limits=maxs, ts_same=ts_same,
+                     th_tendencies=thd)
+    gpu.sync()
+    want = oracle_tracer_step(oracle_lib.Oracle(c), Ts, f["stf"], f["btf"], c.dt, ths=ths,
+                              schemes=schemes, mins=mins, maxs=maxs, ts_same=ts_same)
+    for n in range(4):
+        assert_close_cells(tout[n].to_host()[:, 1:-1, 1:-1], want[n][:, 1:-1, 1:-1],
+                           what=f"{names[n]} ({schemes[n]})")
+    gpu.close()
