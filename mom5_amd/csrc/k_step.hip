@@ -121,7 +121,13 @@ struct StepJob {
 
 // One 64-wide tile of one job, marched through all levels.  Every thread of
 // the block calls it with the same job and tile.
-template <typename TT, int G, int RPW, int NW>
+// TH: some FP64 tracer of the group has other th_tendency terms.  A pass without
+// them must not hold their load: at the join of the branch around it the wait is
+// for every load in flight, the next level's too.  (Only the shapes with loads
+// in flight there, one row a wavefront and up to two tracers, have both forms.)
+template <typename TT, int G, int RPW>
+constexpr bool both_th() { return sizeof(TT) == 8 && RPW == 1 && G <= 2; }
+template <typename TT, int G, int RPW, int NW, bool TH>
 __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
   const KDom d = J.d;
   const StepTab<TT> &tab = J.tab;
@@ -145,19 +151,30 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
   constexpr int RY = NW * RPW;
   // FP64 groups of one row a wavefront and at most two tracers (registers to
   // spare) issue the tracers of level k+3 right after the z sweep (EARLYT;
-  // the others load them at the end of the level), keep two copies of the
+  // the others load them at the end of the level) and keep two copies of the
   // x-swept values and of the y fluxes, by level parity, where the LDS holds
   // them (ONEB: one barrier a level, the update of a level done after the
-  // next level's barrier), and issue a level's w and rho_dzt during the level
-  // before (PREWR).  FP32 groups of one row a wavefront take PREWR only, and
-  // with it the loads of the east face (u and its two rho_dzt).
+  // next level's barrier).
+  // ONEB shapes and FP32 groups of one row a wavefront issue each of a level's
+  // inputs during the level before, when the sweep that reads it is done with
+  // the last one's (PRE), so that no sweep waits for loads issued just before
+  // it.  What makes room for them: the rho_dzt of the faces is one value a point
+  // (at its own place in the data domain, halo included), the other sides of
+  // the east and north faces come from the next lane and, through LDS, the next
+  // row; five loads of rho_dzt a level become two.  Domains that are cyclic in y
+  // take other shapes (their halo rows' x and y faces read different rows).
+  // With the loads at the level's start two FP64 tracers took 1.75 ms at
+  // 1440x1080x50; so, and without branches, 1.50 ms, now bound by vector
+  // instructions: 347 a level and wavefront, issued 82% of the time (ten FP32
+  // tracers: 752, 91%).
   constexpr bool EARLYT = RPW == 1 && EXACT && G <= 2;
   constexpr bool ONEB = EARLYT &&
                         2 * 2 * G * RY * RX * sizeof(TT) + RY * RX * sizeof(int) <= 160 * 1024;
-  constexpr bool PREWR = EXACT ? ONEB : RPW == 1;
+  constexpr bool PRE = EXACT ? ONEB : RPW == 1;
   constexpr int NB = ONEB ? 2 : 1;
   __shared__ TT s_tx[NB][G][RY][RX];
   __shared__ TT s_fy[NB][G][RY][RX];
+  __shared__ TT s_r[PRE ? NB : 1][PRE ? RY : 1][RX];   // rho_dzt at the points' own places
   __shared__ int s_km[RY][RX];
 
   constexpr int TY = RY - 4;
@@ -256,16 +273,14 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
     }
   }
 
-  // FP64 groups issue all of a level's 3-D loads when the level starts (w
-  // and rho_dzt of the point during the level before, PREWR): u and the two
-  // rho_dzt of its east face, v and the two of its north face,
-  // rho_dzt(taum1) and 1/rho_dzt(taup1) (or rho_dzt(taup1); with ONEB those
-  // of the level before, for its deferred update), so that the x, y and
-  // update phases (each after a barrier) do not each wait for their own loads
-  // with every wavefront of the work-group at once.  The loads are
-  // unconditional, from offset 0 where the face or point does not exist (the
-  // value is then unused).  The face metrics stay in registers as for FP32
-  // groups.
+  // A level's 3-D inputs: w and rho_dzt of the point, u and the two rho_dzt of
+  // its east face, v and the two of its north face, rho_dzt(taum1) and
+  // 1/rho_dzt(taup1) (or rho_dzt(taup1)).  Shapes other than PRE issue them when
+  // the level starts, so that the x, y and update phases (each after a barrier)
+  // do not each wait for their own loads with every wavefront of the work-group
+  // at once.  The loads are unconditional, from offset 0 where the face or point
+  // does not exist (the value is then unused).  The face metrics stay in
+  // registers as for FP32 groups.
   struct LvIn {
     double w, r, u, rw, re, v, rs, rn, rm1, rr;
   };
@@ -300,44 +315,38 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
     by[q] = (unsigned)oyq[q] * 8u;
   }
   const double *Rx = Rr ? Rr : R;
-  // PREWR shapes issue a level's w and rho_dzt (FP32: and the east face's
-  // u and rho_dzt) during the level before, after its z sweep: the sweeps
-  // that start a level then wait for nothing
-  double nw[RPW], nr[RPW], nu[RPW], nrw[RPW], nre[RPW];
-  if constexpr (PREWR) {
+  // PRE shapes: the next level's inputs (nh: rho_dzt at the point's own place;
+  // nm, nx: the update's)
+  double nw[RPW], nr[RPW], nu[RPW], nh[RPW], nv[RPW], nm[RPW], nx[RPW];
+  unsigned bh[RPW];
+  if constexpr (PRE) {
 #pragma unroll
     for (int q = 0; q < RPW; ++q) {
+      bh[q] = gi >= -1 && gi <= d.ni && gjr[q] >= -1 && gjr[q] <= d.nj
+                  ? (unsigned)d2(d, gi, gjr[q]) * 8u : 0u;
       nw[q] = ld_lv(W + P2, bz[q]);
       nr[q] = ld_lv(R, bz[q]);
-      if constexpr (!EXACT) {
-        nu[q] = ld_lv(U, bx[q]);
-        nrw[q] = ld_lv(R, bx[q]);
-        nre[q] = ld_lv(R + 1, bx[q]);
-      }
+      nu[q] = ld_lv(U, bx[q]);
+      nh[q] = ld_lv(R, bh[q]);
+      nv[q] = ld_lv(V, by[q]);
     }
   }
   auto lv_load = [&](int k, LvIn *L) {
     const size_t pk = (size_t)P2 * (k - 1);
-    // the update's rho_dzt(taum1) and 1/rho_dzt(taup1): of the level before
-    // when the update is deferred (unused at the first level)
-    const size_t pu = ONEB ? (size_t)P2 * max(k - 2, 0) : pk;
 #pragma unroll
     for (int q = 0; q < RPW; ++q) {
-      if constexpr (PREWR) {
-        L[q].w = nw[q];
-        L[q].r = nr[q];
-      } else {
-        L[q].w = ld_lv(W + pk + P2, bz[q]);
-        L[q].r = ld_lv(R + pk, bz[q]);
-      }
+      L[q].w = ld_lv(W + pk + P2, bz[q]);
+      L[q].r = ld_lv(R + pk, bz[q]);
       L[q].u = ld_lv(U + pk, bx[q]);
       L[q].rw = ld_lv(R + pk, bx[q]);
       L[q].re = ld_lv(R + pk + 1, bx[q]);
       L[q].v = ld_lv(V + pk, by[q]);
       L[q].rs = ld_lv(R + pk, by[q]);
       L[q].rn = ld_lv(R + pk + d.NI, by[q]);
-      L[q].rm1 = ld_lv(Rm1 + pu, bz[q]);
-      L[q].rr = ld_lv(Rx + pu, bz[q]);
+      if constexpr (EXACT) {
+        L[q].rm1 = ld_lv(Rm1 + pk, bz[q]);
+        L[q].rr = ld_lv(Rx + pk, bz[q]);
+      }
     }
   };
 
@@ -346,7 +355,7 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
   // from level kf in pf_*.  The arithmetic is that of the in-level update.
   double pf_xf[RPW], pf_dtr[RPW], pf_r[RPW], pf_brk[RPW];
   TT pf_tx[G][RPW];
-  auto update_deferred = [&](int kf, const LvIn *L) {
+  auto update_deferred = [&](int kf) {
     const int bp = kf & 1;
 #pragma unroll
     for (int q = 0; q < RPW; ++q) {
@@ -357,11 +366,12 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
       if (cell) {
         const size_t pk = (size_t)P2 * (kf - 1);
         const double mi = mk<double>(kf, km[q]);
-        const double rm1 = L[q].rm1;
-        const double rr = Rr ? L[q].rr : 1.0 / (L[q].rr + EPSLN);
+        const double rm1 = nm[q];
+        const double rr = Rr ? nx[q] : 1.0 / (nx[q] + EPSLN);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-          const double thin = tab.th[g] ? ld_lv(tab.th[g] + pk, bz[q]) : 0.0;
+          double thin = 0.0;
+          if constexpr (TH) thin = tab.th[g] ? ld_lv(tab.th[g] + pk, bz[q]) : 0.0;
           const double Tc = t0[g][q];
           double tr = pf_tx[g][q] + pf_xf[q] * (s_fy[bp][g][ry - 1][lane] - s_fy[bp][g][ry][lane]);
           tr = tr + pf_dtr[q] * Tc * pf_brk[q];
@@ -375,34 +385,15 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
   auto level = [&](const int k) {
     const int bb = ONEB ? (k & 1) : 0;
     LvIn cur[RPW];
-    if constexpr (EXACT) {
-      lv_load(k, cur);
-    } else {
-      // FP32 groups (registers for eight more values, not ten): the z, x and
-      // y phases' loads
-      const size_t pk = (size_t)P2 * (k - 1);
+    if constexpr (PRE) {
 #pragma unroll
       for (int q = 0; q < RPW; ++q) {
-        if constexpr (PREWR) {
-          cur[q].w = nw[q];
-          cur[q].r = nr[q];
-        } else {
-          cur[q].w = ld_lv(W + pk + P2, bz[q]);
-          cur[q].r = ld_lv(R + pk, bz[q]);
-        }
-        if constexpr (PREWR) {
-          cur[q].u = nu[q];
-          cur[q].rw = nrw[q];
-          cur[q].re = nre[q];
-        } else {
-          cur[q].u = ld_lv(U + pk, bx[q]);
-          cur[q].rw = ld_lv(R + pk, bx[q]);
-          cur[q].re = ld_lv(R + pk + 1, bx[q]);
-        }
-        cur[q].v = ld_lv(V + pk, by[q]);
-        cur[q].rs = ld_lv(R + pk, by[q]);
-        cur[q].rn = ld_lv(R + pk + d.NI, by[q]);
+        cur[q].w = nw[q];
+        cur[q].r = nr[q];
       }
+    } else {
+      // FP32 groups load the update's inputs later (registers for eight, not ten)
+      lv_load(k, cur);
     }
     const int k0 = k - 1;
     const int kp1 = min(k + 1, nk), kp2 = min(k + 2, nk);
@@ -417,9 +408,10 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
 #pragma unroll
     for (int q = 0; q < RPW; ++q) {
       rhov[q] = 1.0; wv[q] = RT(0); rinv[q] = 1.0f; dtrv[q] = 0.0;
-      // mk(km1)*mk(k) = mk(k), mk(k)*mk(kp1) = mk(kp1), mk(kp1)*mk(kp2) =
-      // mk(kp2): km1 <= k <= kp1 <= kp2 and masks in {0, 1}
-      const TT mA = mk<TT>(k, km[q]), mB = mk<TT>(kp1, km[q]), mC = mk<TT>(kp2, km[q]);
+      // mk(k)*mk(kp1) = mk(kp1), mk(kp1)*mk(kp2) = mk(kp2) (k <= kp1 <= kp2, masks
+      // in {0, 1}).  Where the face is wet (mB = 1) so is the cell above; where it
+      // is dry its weight is 0: only mC needs applying to a difference
+      const TT mB = mk<TT>(kp1, km[q]), mC = mk<TT>(kp2, km[q]);
       if constexpr (!EXACT) {
         // FP32 groups take no branch: at a point outside the domain (t, dat,
         // datr and the masks 0) w = 0 and rho_dzt = 1 keep every value
@@ -435,8 +427,6 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
         const float dtrf = (float)dtime * ri, datrf = (float)datrv[q];
         const float wdiff = (float)wkm1[q] - wf;
 #pragma unroll
-        // where the face is wet (mB = 1) so is the cell above (mA = 1);
-        // where it is dry its weights are 0: only mC needs applying
         for (int g = 0; g < G; ++g) {
           const float Rjp = t0[g][q] - t1[g][q];
           const float Rj = t1[g][q] - t2[g][q];
@@ -445,8 +435,10 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
           tz[g][q] = fmaf(dtrf, fmaf(datrf, fbt - ftp[g][q], t1[g][q] * wdiff), t1[g][q]);
           fbtv[g][q] = fbt;
         }
-      } else if (ok[q]) {
-        const double w = cur[q].w, r = cur[q].r;
+      } else {
+        // no branch: a point outside the domain (t, dat, datr and the masks 0)
+        // takes w = 0 and rho_dzt = 1, and gets tz = 0 and a zero flux
+        const double w = ok[q] ? cur[q].w : 0.0, r = ok[q] ? cur[q].r : 1.0;
         rhov[q] = r; wv[q] = (RT)w;
         const double dtr = dtime * mdfl64::rcp64(r);
         dtrv[q] = dtr;
@@ -454,16 +446,13 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
         const double wdiff = wkm1[q] - w;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-          const double Rjp = (t0[g][q] - t1[g][q]) * mA;
-          const double Rj = (t1[g][q] - t2[g][q]) * mB;
+          const double Rjp = t0[g][q] - t1[g][q];
+          const double Rj = t1[g][q] - t2[g][q];
           const double Rjm = (t2[g][q] - t3[g][q]) * mC;
           const double fbt = mdfl64::flux(cz, Rjm, Rj, Rjp, t2[g][q], t1[g][q]);
           tz[g][q] = t1[g][q] + dtr * (datrv[q] * (fbt - ftp[g][q]) + t1[g][q] * wdiff);
           fbtv[g][q] = fbt;
         }
-      } else {
-#pragma unroll
-        for (int g = 0; g < G; ++g) { tz[g][q] = TT(0); fbtv[g][q] = TT(0); }
       }
     }
 
@@ -480,18 +469,19 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
         }
       }
     }
-    if constexpr (PREWR) {
-      // w and rho_dzt of level k+1 (the last level reloads its own)
-      const size_t pw = (size_t)P2 * min(k + 1, nk), pr = (size_t)P2 * min(k, nk - 1);
+    // the next level's (the last level loads its own again)
+    const size_t pw = (size_t)P2 * min(k + 1, nk), pr = (size_t)P2 * min(k, nk - 1);
+    if constexpr (PRE) {
 #pragma unroll
       for (int q = 0; q < RPW; ++q) {
         nw[q] = ld_lv(W + pw, bz[q]);
         nr[q] = ld_lv(R + pr, bz[q]);
-        if constexpr (!EXACT) {
-          nu[q] = ld_lv(U + pr, bx[q]);
-          nrw[q] = ld_lv(R + pr, bx[q]);
-          nre[q] = ld_lv(R + pr + 1, bx[q]);
-        }
+        // the x and y faces of this level
+        cur[q].u = nu[q];
+        cur[q].rw = nh[q];
+        cur[q].v = nv[q];
+        if constexpr (EXACT) cur[q].re = lane_next(nh[q]);
+        s_r[bb][wave + NW * q][lane] = (TT)nh[q];
       }
     }
 
@@ -509,16 +499,18 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
       if constexpr (!EXACT) {
         // FP32 groups take no branch: where there is no face its metrics
         // are 0, so its mass flux is 0 and its CFL number is set to 0
-        const float uf = (float)cur[q].u;
+        const float uf = (float)cur[q].u, rwf = (float)cur[q].rw;
+        const float rsum = rwf + (PRE ? lane_next(rwf) : (float)cur[q].re);
         const float cfl = fabsf(uf * (float)(dtime * 2.0) *
-                                rcpf(((float)cur[q].rw + (float)cur[q].re) * mdxte[q]));
+                                rcpf(rsum * mdxte[q]));
         cxf = face_coef_f(mdyte[q] * uf, face ? cfl : 0.0f);
-      } else if (face) {
-        const double u = cur[q].u, rw = cur[q].rw, re = cur[q].re;
+      } else {
+        // no branch: where there is no face u and the Courant number are set to 0
+        const double u = face ? cur[q].u : 0.0, rw = cur[q].rw, re = cur[q].re;
         Mx = hdyte[q] * u;
-        cx = mdfl64::face(Mx, mdfl64::cfl_h(u, dtime, rw + re, hdxte[q]), (double)mX1);
+        const double cf = mdfl64::cfl_h(u, dtime, rw + re, hdxte[q]);
+        cx = mdfl64::face(Mx, face ? cf : 0.0, (double)mX1);
       }
-      const bool cell = rowok[q] && lane >= 2 && lane < RX - 2 && gi < d.ni;
       double mw64 = 0.0;
       if constexpr (EXACT) {
         mw64 = lane_prev(Mx);
@@ -552,7 +544,7 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
         TT fx = TT(0);
         if constexpr (!EXACT)
           fx = flux_fast(cxf, wx, Rjm, Rjl, Rjp, tz[g][q], tzp1);
-        else if (face)
+        else
           fx = mdfl64::flux(cx, Rjm, Rjl, Rjp, tz[g][q], tzp1);
         const TT fxw = lane_prev(fx);
         if constexpr (EXACT) {
@@ -568,15 +560,35 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
         TT tx = TT(0);
         if constexpr (!EXACT)
           tx = fmaf(xfac[q], fmaf(t1[g][q], mfe[q] - mfw[q], fxw - fx), tz[g][q]);
-        else if (cell)
+        else
           tx = tz[g][q] + xf64v[q] * (fxw - fx + t1[g][q] * (Mx - mw64));
         s_tx[bb][g][ry][lane] = tx;
         txv[g][q] = tx;
       }
     }
+    if constexpr (PRE) {
+#pragma unroll
+      for (int q = 0; q < RPW; ++q) {
+        nu[q] = ld_lv(U + pr, bx[q]);
+        nh[q] = ld_lv(R + pr, bh[q]);
+      }
+    }
     __syncthreads();
     if constexpr (ONEB) {
-      if (k > 1) update_deferred(k - 1, cur);
+      if (k > 1) update_deferred(k - 1);
+#pragma unroll
+      for (int q = 0; q < RPW; ++q) {
+        nm[q] = ld_lv(Rm1 + (size_t)P2 * k0, bz[q]);
+        nx[q] = ld_lv(Rx + (size_t)P2 * k0, bz[q]);
+      }
+    }
+    if constexpr (PRE) {
+#pragma unroll
+      for (int q = 0; q < RPW; ++q) {
+        const int ry = wave + NW * q;
+        cur[q].rs = s_r[bb][ry][lane];
+        cur[q].rn = s_r[bb][min(ry + 1, RY - 1)][lane];
+      }
     }
 
     // ---- Y ----------------------------------------------------------------
@@ -632,7 +644,7 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
             const TT tjm1 = s_tx[bb][g][ry - 1][lane], tj = s_tx[bb][g][ry][lane];
             const TT tjp1 = s_tx[bb][g][ry + 1][lane], tjp2 = s_tx[bb][g][ry + 2][lane];
             const TT Rjp = (tjp2 - tjp1) * mY2;
-            const TT Rj = (tjp1 - tj) * mY1;
+            const TT Rj = tjp1 - tj;   // the face's weight carries mY1
             const TT Rjm = (tj - tjm1) * mY0;
             fy = mdfl64::flux(cy, Rjm, Rj, Rjp, tj, tjp1);
           }
@@ -640,6 +652,10 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
           fyv[g][q] = fy;
         }
       }
+    }
+    if constexpr (PRE) {
+#pragma unroll
+      for (int q = 0; q < RPW; ++q) nv[q] = ld_lv(V + pr, by[q]);
     }
     if constexpr (ONEB) {
       // keep what the deferred update of this level needs
@@ -723,34 +739,27 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
   };
   for (int k = 1; k <= nk; ++k) level(k);
   if constexpr (ONEB) {
-    LvIn last[RPW];
-    const size_t pk = (size_t)P2 * (nk - 1);
-#pragma unroll
-    for (int q = 0; q < RPW; ++q) {
-      last[q].rm1 = ld_lv(Rm1 + pk, bz[q]);
-      last[q].rr = ld_lv(Rx + pk, bz[q]);
-    }
     __syncthreads();
-    update_deferred(nk, last);
+    update_deferred(nk);
   }
 }
 
 
-template <typename TT, int G, int RPW, int NW>
+template <typename TT, int G, int RPW, int NW, bool TH>
 __global__ __launch_bounds__(RX * NW) void k_step(StepJob<TT> J, int per_xcd) {
   const int b = blockIdx.x;
   // XCD-aware: each XCD takes per_xcd consecutive positions of the order of
   // 8-wide strips, so x- and y-neighbours share their halo in one L2
   const int t = (b & 7) * per_xcd + (b >> 3);
   if (t >= J.ntiles) return;
-  step_tile<TT, G, RPW, NW>(J, strip_tile<8>(t, J.ntx, J.ntiles / J.ntx));
+  step_tile<TT, G, RPW, NW, TH>(J, strip_tile<8>(t, J.ntx, J.ntiles / J.ntx));
 }
 
 // Ensemble pass: a persistent grid takes (job, tile) items from a device-side
 // counter in order (jobs sorted largest first) until none is left.  first[j]
 // is the index of job j's first item; total = sum of the jobs' tiles.  Every
 // block leaves the loop once the counter passes total.
-template <typename TT, int G, int RPW, int NW>
+template <typename TT, int G, int RPW, int NW, bool TH>
 __global__ __launch_bounds__(RX * NW) void k_step_queue(const StepJob<TT> *__restrict__ jobs,
                                                         const int *__restrict__ first, int njobs,
                                                         int total, int *__restrict__ counter) {
@@ -766,7 +775,7 @@ __global__ __launch_bounds__(RX * NW) void k_step_queue(const StepJob<TT> *__res
       const int mid = (lo + hi + 1) >> 1;
       if (first[mid] <= item) lo = mid; else hi = mid - 1;
     }
-    step_tile<TT, G, RPW, NW>(jobs[lo], item - first[lo]);
+    step_tile<TT, G, RPW, NW, TH>(jobs[lo], item - first[lo]);
   }
 }
 
@@ -782,8 +791,10 @@ struct Shape {
   int rpw, nw;
 };
 
+// cyc_y: a domain cyclic in y, which one-row shapes do not take
 template <typename TT>
-static Shape shape_of(int rpw, int waves) {
+static Shape shape_of(int rpw, int waves, bool cyc_y) {
+  if (cyc_y && rpw == 1) return {2, 8};
   if (sizeof(TT) == 4) {
     if (rpw == 1 && waves == 16) return {1, 16};
     if (rpw == 2 && waves == 16) return {2, 16};
@@ -895,6 +906,13 @@ static void add_th_f32(hipStream_t s, const KDom &d, float *out, const double *t
 }
 
 template <typename TT>
+static bool any_th(const StepTab<TT> &t, int n) {
+  for (int g = 0; g < n; ++g)
+    if (t.th[g]) return true;
+  return false;
+}
+
+template <typename TT>
 struct GroupLaunch {
   mom_gpu_ctx *ctx;
   const StepTab<TT> &tab;
@@ -910,8 +928,15 @@ struct GroupLaunch {
     const int per = (ntiles + 7) / 8;
     const StepJob<TT> J{d, tab, u, v, w, rho, rm1, rr, ctx->kmt, ctx->dat, ctx->datr,
                         ctx->dxte, ctx->dyte, ctx->dxtn, ctx->dytn, dtime, ntx, ntiles};
-    hipLaunchKernelGGL((k_step<TT, G, RPW, NW>), dim3(8 * per), dim3(RX * NW), 0, ctx->stream,
-                       J, per);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(8 * per), dim3(RX * NW), 0, ctx->stream, J, per);
+    };
+    if constexpr (both_th<TT, G, RPW>()) {
+      if (any_th(tab, G)) go(k_step<TT, G, RPW, NW, true>);
+      else go(k_step<TT, G, RPW, NW, false>);
+    } else {
+      go(k_step<TT, G, RPW, NW, true>);
+    }
     return MOM_GPU_OK;
   }
 };
@@ -922,7 +947,7 @@ static void launch_all(mom_gpu_ctx *ctx, int gmax, int rpw, int waves, int ntr,
                        const double *const *th_in, int want, const double *u, const double *v,
                        const double *w, const double *rho, const double *rm1, const double *rr,
                        double dtime) {
-  const Shape sh = shape_of<TT>(rpw, waves);
+  const Shape sh = shape_of<TT>(rpw, waves, ctx->kd.cyclic_y != 0);
   std::vector<int> idx;
   for (int n = 0; n < ntr; ++n)
     if (dtype[n] == want) idx.push_back(n);
@@ -971,9 +996,19 @@ static int queue_launch(mom_gpu_ensemble *e, std::vector<StepJob<TT>> &jobs, int
   if (!dev) return MOM_GPU_ERR_HIP;
   // enough persistent groups to fill the device; late ones find the queue empty
   const int grid = std::min(total, 2048);
-  hipLaunchKernelGGL((k_step_queue<TT, G, RPW, NW>), dim3(grid), dim3(RX * NW), 0,
-                     e->lead->stream, (const StepJob<TT> *)dev, (const int *)(dev + jbytes),
-                     (int)nj, total, e->counters + slot);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(RX * NW), 0, e->lead->stream,
+                       (const StepJob<TT> *)dev, (const int *)(dev + jbytes), (int)nj, total,
+                       e->counters + slot);
+  };
+  bool th = !both_th<TT, G, RPW>();
+  for (const StepJob<TT> &J : jobs) th = th || any_th(J.tab, G);
+  if constexpr (both_th<TT, G, RPW>()) {
+    if (th) go(k_step_queue<TT, G, RPW, NW, true>);
+    else go(k_step_queue<TT, G, RPW, NW, false>);
+  } else {
+    go(k_step_queue<TT, G, RPW, NW, true>);
+  }
   MOM_LAUNCHED(e->lead, "k_step_queue");
   return MOM_GPU_OK;
 }
@@ -991,7 +1026,9 @@ template <typename TT>
 static int ensemble_type(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *steps, int want,
                          int gmax, int rpw, int waves, int &slot) {
   // jobs bucketed by group size (the shape's sizes no larger than gmax), per domain
-  const Shape sh = shape_of<TT>(rpw, waves);
+  bool cyc_y = false;
+  for (const mom_gpu_ctx *c : e->ctx) cyc_y = cyc_y || c->kd.cyclic_y;
+  const Shape sh = shape_of<TT>(rpw, waves, cyc_y);
   constexpr int GMAX = 12;
   std::vector<StepJob<TT>> by[GMAX + 1];
   const int TY = sh.nw * sh.rpw - 4;

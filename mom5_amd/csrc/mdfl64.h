@@ -68,19 +68,19 @@ __device__ __forceinline__ double flip(double x, unsigned long long sgn) {
   return __builtin_bit_cast(double, __builtin_bit_cast(unsigned long long, x) ^ sgn);
 }
 
-// psi*Rj for the neighbouring difference Rn; d0a = d0*Rj, sgn the sign bit
-// of Rj.  With s = -1 where Rj's
-// sign bit is set and +1 elsewhere (exact sign flips),
-//   psi*Rj = s*max(0, min(|Rj|, s*lin, s*kr)),
-// which is max(0, min(Rj, lin, kr)) for Rj >= 0 and min(0, max(Rj, lin, kr))
-// for Rj < 0 without a branch.
-__device__ __forceinline__ double psi_r(const Face &f, double d0a, double Rj,
-                                        unsigned long long sgn, double Rn) {
-  const double lin = fma(f.d1, Rn, d0a);
-  const double kr = f.kk * Rn;
-  const double m = __builtin_fmin(flip(lin, sgn), flip(kr, sgn));
-  const double t = __builtin_fmax(0.0, __builtin_fmin(fabs(Rj), m));
-  return flip(t, sgn);
+// psi*Rj for the neighbouring difference Rn, up to the sign of Rj.  With s = -1
+// where Rj's sign bit (sgn) is set and +1 elsewhere (exact sign flips),
+//   s*psi*Rj = max(0, min(|Rj|, s*lin, s*kr)),
+//   s*lin = d1*(s*Rn) + d0*|Rj|,  s*kr = kk*(s*Rn)
+// (rounding is symmetric in the sign), which is max(0, min(Rj, lin, kr)) for
+// Rj >= 0 and min(0, max(Rj, lin, kr)) for Rj < 0 without a branch.  Flipping Rn,
+// not lin and kr, keeps the minimum's operands results of arithmetic: no
+// canonicalising v_max_f64 before it.
+__device__ __forceinline__ double psi_s(const Face &f, double Rj, unsigned long long sgn,
+                                        double Rn) {
+  const double a = fabs(Rj), rn = flip(Rn, sgn);
+  const double m = __builtin_fmin(fma(f.d1, rn, f.d0 * a), f.kk * rn);
+  return __builtin_fmax(0.0, __builtin_fmin(a, m));
 }
 
 // The limited flux: Tpos is upstream for M > 0, Tneg for M < 0; Rjm, Rj, Rjp
@@ -89,11 +89,10 @@ __device__ __forceinline__ double psi_r(const Face &f, double d0a, double Rj,
 // the M < 0 term.
 __device__ __forceinline__ double flux(const Face &f, double Rjm, double Rj, double Rjp,
                                        double Tpos, double Tneg) {
-  const double d0a = f.d0 * Rj;
   const unsigned long long sgn = __builtin_bit_cast(unsigned long long, Rj) & (1ull << 63);
   const double Rn = f.pos ? Rjm : Rjp;
   const double Tu = f.pos ? Tpos : Tneg;
-  return f.wm * (Tu + flip(psi_r(f, d0a, Rj, sgn, Rn), f.nsg));
+  return f.wm * (Tu + flip(psi_s(f, Rj, sgn, Rn), sgn ^ f.nsg));
 }
 
 // Courant numbers: |w*dtime/rho_dzt| of a bottom face (dtr = dtime/rho_dzt)

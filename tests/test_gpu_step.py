@@ -384,3 +384,60 @@ def test_shallow_domains_default_shapes(oracle_lib, nk):
         err = np.abs(got[n].astype(np.float64) - ref[n]).max() / np.abs(ref[n]).max()
         assert err <= 1e-5, (n, err)
     gpu.close()
+
+
+@pytest.mark.parametrize("cyc", [(1, 0), (0, 0), (1, 1)])
+@pytest.mark.parametrize("ni,nj,nk", [(61, 25, 4), (60, 12, 2), (125, 11, 7)])
+def test_step_reads_the_halo_as_given(cyc, ni, nj, nk):
+    """Halo values of the transports and of rho_dzt that hold no wrap: the
+    one-row shapes (which take a face's rho_dzt from the neighbouring lane and
+    row) equal the per-tracer path (FP64) and the two-row shapes (FP32, FP64)
+    bit for bit, on cyclic, closed and doubly cyclic domains, at sizes about a
+    region's, with other th_tendency terms on one tracer of a pair."""
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    print(f"[step {ni}x{nj}x{nk} cyclic x, y = {cyc}, halos without a wrap]", flush=True)
+    case = make_case(ni, nj, nk, land_frac=0.2, nts=8, seed=71, n_passive=5, barotropic=False,
+                     cyclic_x=bool(cyc[0]),
+                     **({} if cyc[0] else dict(lat_s=20.0, lat_n=50.0, lon_span=30.0)))
+    g = OceanGPU(dict(case.dom, cyclic_y=cyc[1]), case.grid)
+    rng = np.random.default_rng(3)
+    H = DeviceArray.from_host
+    f = {k: np.array(case.fields[k]) for k in ("uhrho_et", "vhrho_nt", "wrho_bt", "rho_dzt")}
+    for name, a in f.items():
+        old = a.copy()
+        scale = np.abs(a).max()
+        noise = rng.random(a.shape) if name == "rho_dzt" else rng.standard_normal(a.shape)
+        a[:] = (0.5 + noise) * a.mean() if name == "rho_dzt" else 0.1 * scale * noise
+        a[:, 1:-1, 1:-1] = old[:, 1:-1, 1:-1]
+    d = {k: H(v) for k, v in f.items()}
+    rhor = H(1.0 / f["rho_dzt"])
+    dtypes = [np.float64] * 3 + [np.float32] * 4
+    Ts = [H(np.asarray(t, dt)) for (_, t), dt in zip(case.tracers, dtypes)]
+    th = H(1e-4 * rng.standard_normal(f["rho_dzt"].shape))
+
+    def step():
+        outs = [g.field3(dtype=dt) for dt in dtypes]
+        g.step_tracers(Ts, outs, uhrho_et=d["uhrho_et"], vhrho_nt=d["vhrho_nt"],
+                       wrho_bt=d["wrho_bt"], rho_dzt_tau=d["rho_dzt"], rho_dztr=rhor,
+                       dtime=case.dt, th_tendencies=[None, th] + [None] * 5)
+        g.sync()
+        return [o.to_host()[:, 1:-1, 1:-1] for o in outs]
+
+    got = step()
+    g.set_tuning("step_rows_per_wave", 2)
+    g.set_tuning("step_rows_per_wave_f32", 2)
+    for n, (a, b) in enumerate(zip(got, step())):
+        assert np.isfinite(a).all(), n
+        assert np.array_equal(a, b), n
+    for n in range(3):
+        tend, out = g.field3(), g.field3()
+        if n == 1:
+            g.copy(tend, th)
+        g.horz_advect_tracer("mdfl_sweby", Ts[n], tend, uhrho_et=d["uhrho_et"],
+                             vhrho_nt=d["vhrho_nt"], wrho_bt=d["wrho_bt"],
+                             rho_dzt_tau=d["rho_dzt"], dtime=case.dt)
+        g.update_tracer_explicit(Ts[n], tend, d["rho_dzt"], rhor, case.dt, out)
+        g.sync()
+        assert np.array_equal(got[n], out.to_host()[:, 1:-1, 1:-1]), n
+    g.close()
