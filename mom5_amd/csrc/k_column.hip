@@ -1187,6 +1187,215 @@ void k_vdiff_twin64(VdJob<double> J, int per_xcd) {
   twin64_tile<H, 2>(J, min(tile, J.nblocks - 1), tile < J.nblocks);
 }
 
+// Several FP64 tracers of one mixing class: k_vdiff_twin64's elimination with the
+// factorisation formed once a column instead of once a tracer.  Its p and bet
+// of every slot lie in LDS (own lane, no exchange), q bet in registers, and the
+// tracers then stream through, each read while the one before is solved and
+// written once.  The same expressions in the same order as k_vdiff_twin64: a
+// tracer's result does not depend on the group it is solved in.  (A dry level's
+// value is multiplied by bet = 0 instead of by the mask and bet.)
+//
+// Bound by HBM: 16 B a cell and tracer, and 24 B a cell once a class, which
+// k_vdiff_twin64 reads again for each tracer: T, S and six more at 1440x1080x50
+// 4.42 ms with that, 3.04 ms so (12.4 GB: 4.1 TB/s), at 75 levels 6.46 and 4.69.
+// One tile (64 columns, two wavefronts) a block: the factors of two tiles fill a
+// CU's LDS at 76 levels.  (Two tiles a block: the same within 4%.)
+constexpr int SHARE_NT = 32;
+struct ShareJob {
+  KDom d;
+  double *z[SHARE_NT];
+  const double *stf[SHARE_NT], *btf[SHARE_NT];
+  int n, n2;                 // tracers; the first of class 2
+  const double *dcb[2];      // diff_cbt planes of the two classes
+  double rho0;
+  const int *kmt;
+  const double *dh, *dhw;
+  double tdt, aidif;
+  int nbx, nblocks;
+};
+
+template <int H>
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(H > 20 ? 1 : 2)))
+void k_vdiff_share(ShareJob J, int per_xcd) {
+  const int blk = blockIdx.x;
+  const int tile = (blk & 7) * per_xcd + (blk >> 3);
+  if (tile >= J.nblocks) return;               // the whole block
+  __shared__ double s_p[2][H][64], s_b[2][H][64];
+  __shared__ double xv[2][2][64], xq[2][64];   // [parity][half][column]
+  const KDom d = J.d;
+  const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool top = half == 0;
+  const int lane = threadIdx.x & 63;
+  const int col = (tile % J.nbx) * 64 + lane;
+  const bool valid = col < d.ni;
+  const int nk = d.nk;
+  const int nt = (nk + 1) >> 1;
+  const int nact = top ? nt : nk - nt;
+  const int ph = H - nact;
+  const long P2 = d.P2;
+  const long step = top ? P2 : -P2;
+  const long p0 = top ? 0 : (long)(nk - 1) * P2;
+  const unsigned o = (unsigned)d2(d, valid ? col : d.ni - 1, tile / J.nbx);
+  const unsigned ob8 = o * 8u;
+  const int kmo = ld_at(J.kmt, o * 4u);
+  const int kb = max(2, kmo);
+  const double tda = J.tdt * J.aidif;
+  double A[H], B[H], qs[H];
+
+  // a tracer's active levels, slot ph's plane first (k_vdiff_twin64)
+  auto load = [&](int n, double *v) {
+    const double *z = J.z[n];
+    long pl = p0;
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+      v[j] = 0.0;
+      int phj = ph;
+      asm volatile("" : "+s"(phj));
+      if (j < phj) continue;           // inert slot (wavefront-uniform)
+      asm volatile("" : "+s"(pl));
+      v[j] = ld_at(z + pl, ob8);
+      pl += step;
+    }
+  };
+  double dh1 = 1.0, dhkb = 1.0;        // dh of level 1 and of level kb
+  auto factor = [&](const double *dcbase) {
+    constexpr int CH = 4, NCH = (H + CH - 1) / CH;
+    const long dwo = top ? P2 : 0, dco = top ? 0 : -P2;
+    double Ldh[NCH * CH], Ldw[NCH * CH], Ldc[NCH * CH];
+    auto cload = [&](int c) {
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int j = c * CH + u;
+        if (j >= H) break;
+        int phj = ph;
+        asm volatile("" : "+s"(phj));
+        long plj = p0 + (long)max(j - phj, 0) * step;
+        asm volatile("" : "+s"(plj));
+        Ldh[j] = ld_at(J.dh + plj, ob8);
+        Ldw[j] = ld_at(J.dhw + plj + dwo, ob8);
+        Ldc[j] = ld_at(dcbase + plj + dco, ob8);
+      }
+    };
+    const double dhw_first = ld_at(J.dhw + p0 + (top ? 0 : P2), ob8);
+    const double dcb_first = top ? 0.0 : J.rho0 * ld_at(dcbase + p0, ob8);
+    double bet = 0.0, qprev = 0.0, dcb_c = 0.0, dhw_c = 0.0;
+    cload(0);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      if (c + 1 < NCH) cload(c + 1);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int j = c * CH + u;
+        if (j >= H) break;
+        qs[j] = 0.0;
+        int phj = ph;
+        asm volatile("" : "+s"(phj));
+        if (j < phj) continue;
+        const int r = j - phj;
+        const int k = top ? r + 1 : nk - r;
+        const double dhk = Ldh[j];
+        const double dcb_new = J.rho0 * Ldc[j];
+        // dzwt plane k-1 is the interface above level k, plane k the one below
+        double dcb_km1, dcb_k, dhw_km1, dhw_k;
+        if (top) {
+          dcb_k = dcb_new;
+          dhw_k = Ldw[j];
+          dcb_km1 = (r == 0) ? dcb_k : dcb_c;
+          dhw_km1 = (r == 0) ? dhw_first : dhw_c;
+          dcb_c = dcb_k;
+          dhw_c = dhw_k;
+        } else {
+          dcb_k = (r == 0) ? dcb_first : dcb_c;
+          dhw_k = (r == 0) ? dhw_first : dhw_c;
+          dcb_km1 = dcb_new;
+          dhw_km1 = Ldw[j];
+          dcb_c = dcb_km1;
+          dhw_c = dhw_km1;
+        }
+        const int kp1 = min(k + 1, nk);
+        const double factu = tda / (dhw_km1 * dhk);
+        const double factl = tda / (dhw_k * dhk);
+        const double mkk = (k <= kmo) ? 1.0 : 0.0;
+        const double mkp1 = (kp1 <= kmo) ? 1.0 : 0.0;
+        double a = -dcb_km1 * factu * mkk;
+        double c2 = -dcb_k * factl * mkp1;
+        if (k == 1) a = 0.0;
+        if (k == nk) c2 = 0.0;
+        const double b = 1.0 - a - c2;
+        const double p = top ? a : c2, q = top ? c2 : a;
+        if (r == 0) {
+          bet = mkk / (b + EPS_TRI);
+        } else {
+          const double e = qprev * bet;
+          bet = mkk / (b - p * e + EPS_TRI);
+        }
+        s_p[half][j][lane] = p;
+        s_b[half][j][lane] = bet;
+        qs[j] = q * bet;
+        qprev = q;
+        if (k == 1) dh1 = dhk;
+        if (k == kb) dhkb = dhk;
+        __builtin_amdgcn_sched_barrier(0);   // one slot at a time
+      }
+    }
+    xq[half][lane] = qs[H - 1];
+  };
+  const double m1 = (1 <= kmo) ? 1.0 : 0.0, mkb = (kb <= kmo) ? 1.0 : 0.0;
+  // tracer n, its levels in v; the next one's go to w meanwhile
+  auto solve = [&](int n, int last, double *v, double *w) {
+    const double stf = ld_at(J.stf[n], ob8), btf = ld_at(J.btf[n], ob8);
+    if (n + 1 < last) load(n + 1, w);
+    const double fs = stf * tda * m1 / dh1, fb = btf * tda * mkb / dhkb;
+    double vprev = 0.0;
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+      int phj = ph;
+      asm volatile("" : "+s"(phj));
+      if (j < phj) continue;
+      const int r = j - phj, k = top ? r + 1 : nk - r;
+      double f = v[j];
+      if (k == 1) f = f + fs;
+      f = (k == kb) ? f - fb : f;
+      vprev = (f - s_p[half][j][lane] * vprev) * s_b[half][j][lane];
+      v[j] = vprev;
+    }
+    // the meeting: x_t + Qt x_b = Vt (top's last level), x_b + Qb x_t = Vb
+    xv[n & 1][half][lane] = vprev;
+    lds_barrier();
+    const double Vo = xv[n & 1][1 - half][lane], Qo = xq[1 - half][lane];
+    const double Vt = top ? vprev : Vo, Qt = top ? qs[H - 1] : Qo;
+    const double Vb = top ? Vo : vprev, Qb = top ? Qo : qs[H - 1];
+    const double xt = (Vt - Qt * Vb) / (1.0 - Qt * Qb);
+    double x = top ? xt : Vb - Qb * xt;
+    double *z = J.z[n];
+    long pl = p0 + (long)(nact - 1) * step;
+#pragma unroll
+    for (int j = H - 1; j >= 0; --j) {
+      int phj = ph;
+      asm volatile("" : "+s"(phj));
+      if (j < phj) continue;
+      if (j < H - 1) x = v[j] - qs[j] * x;
+      asm volatile("" : "+s"(pl));
+      if (valid) st_at(z + pl, ob8, x);
+      pl -= step;
+    }
+  };
+  for (int c = 0; c < 2; ++c) {
+    const int first = c == 0 ? 0 : J.n2, last = c == 0 ? J.n2 : J.n;
+    if (first >= last) continue;
+    load(first, A);
+    // the other half's reads of the last class's xq are over
+    if (c == 1) lds_barrier();
+    factor(J.dcb[c]);
+    for (int n = first; n < last; n += 2) {
+      solve(n, last, A, B);
+      if (n + 1 < last) solve(n + 1, last, B, A);
+    }
+  }
+}
+
 // Ensemble: every FP64 group of every domain whose nk the register solver
 // takes, in one launch; tiles in XCD-aware order over the whole table.
 template <int H>
@@ -1480,6 +1689,7 @@ int launch_invtri(mom_gpu_ctx *ctx, double *z, const double *topbc, const double
 
 static int twin_slots(int nk);
 static void launch_twin64(mom_gpu_ctx *ctx, VdJob<double> J);
+static void launch_share(mom_gpu_ctx *ctx, const ShareJob &J);
 
 // FP64 tracers take the register-resident solver (k_vdiff_twin64) whenever nk
 // is in its range (2..80), whatever the knobs, so that FP64 results never
@@ -1521,6 +1731,28 @@ static int twin64_groups(mom_gpu_ctx *ctx, int ntr, void *const *T, const int *d
   const int n1 = (int)c1.size();
   std::vector<int> all(c1);
   all.insert(all.end(), c2.begin(), c2.end());
+  // Three tracers of class 1 or more share its factorisation (class 2 is salt
+  // alone).  With two the one factorisation saved is what fewer wavefronts in
+  // flight cost: T, S and one more tracer at 1440x1080, 41 levels 1.49 ms with
+  // k_vdiff_twin64 against 1.57, 50 levels 1.84 against 1.75; with two more 2.46
+  // against 2.04 at 50 levels.
+  if (c1.size() >= 3) {
+    for (size_t at = 0; at < all.size(); at += SHARE_NT) {
+      ShareJob J{};
+      J.d = d; J.dcb[0] = diff_cbt; J.dcb[1] = diff_cbt + p3; J.rho0 = rho0; J.kmt = ctx->kmt;
+      J.dh = dh; J.dhw = dhw; J.tdt = dt; J.aidif = aidif;
+      J.nbx = nbx; J.nblocks = nbx * d.nj;
+      J.n = (int)std::min((size_t)SHARE_NT, all.size() - at);
+      for (int q = 0; q < J.n; ++q) {
+        const int n = all[at + q];
+        J.z[q] = (double *)T[n]; J.stf[q] = stf[n]; J.btf[q] = btf[n];
+      }
+      J.n2 = std::max(0, std::min(J.n, n1 - (int)at));
+      launch_share(ctx, J);
+      MOM_LAUNCHED(ctx, "k_vdiff_share");
+    }
+    return MOM_GPU_OK;
+  }
   for (size_t at = 0; at < all.size(); at += NT) {
     const int cnt = (int)std::min((size_t)NT, all.size() - at);
     VdJob<double> J = job();
@@ -1723,6 +1955,22 @@ static void launch_twin64(mom_gpu_ctx *ctx, VdJob<double> J) {
     case 32: hipLaunchKernelGGL(k_vdiff_twin64<32>, grid, block, 0, ctx->stream, J, per_xcd); break;
     default: hipLaunchKernelGGL(k_vdiff_twin64<40>, grid, block, 0, ctx->stream, J, per_xcd); break;
   }
+}
+
+static void launch_share(mom_gpu_ctx *ctx, const ShareJob &J) {
+  const int per_xcd = (J.nblocks + 7) / 8, h = (J.d.nk + 1) / 2;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(8 * per_xcd), dim3(128), 0, ctx->stream, J, per_xcd);
+  };
+  if (h <= 8) go(k_vdiff_share<8>);
+  else if (h <= 12) go(k_vdiff_share<12>);
+  else if (h <= 16) go(k_vdiff_share<16>);
+  else if (h <= 20) go(k_vdiff_share<20>);
+  else if (h <= 25) go(k_vdiff_share<25>);
+  else if (h <= 30) go(k_vdiff_share<30>);
+  else if (h <= 34) go(k_vdiff_share<34>);
+  else if (h <= 38) go(k_vdiff_share<38>);
+  else go(k_vdiff_share<40>);
 }
 
 static void launch_twin(mom_gpu_ctx *ctx, VdJobF J) {

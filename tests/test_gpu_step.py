@@ -441,3 +441,32 @@ def test_step_reads_the_halo_as_given(cyc, ni, nj, nk):
         g.sync()
         assert np.array_equal(got[n], out.to_host()[:, 1:-1, 1:-1]), n
     g.close()
+
+
+@pytest.mark.parametrize("nk", [2, 3, 16, 17, 24, 25, 39, 50, 51, 60, 67, 75, 76, 77, 80])
+def test_shared_factorisation_equals_single_tracers(nk):
+    """vert_diffuse_implicit of T, S and 2..34 more FP64 tracers, which share a
+    factorisation, is bit for bit that of each tracer alone, around every
+    count of register slots (and past one launch's table of 32 tracers)."""
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    print(f"[shared factorisation 70x9x{nk}]", flush=True)
+    case = make_case(70, 9, nk, land_frac=0.3, nts=8, seed=81, barotropic=False)
+    g = OceanGPU(case.dom, case.grid)
+    H = DeviceArray.from_host
+    rng = np.random.default_rng(nk)
+    f = case.fields
+    tm = case.grid["tmask"]
+    dcb, dh, dhw = H(f["diff_cbt"]), H(f["rho_dzt"]), H(f["dzwt"])
+    for ntr in (4, 5) + ((36,) if nk == 3 else ()):
+        Ts = [tm * (1.0 + rng.random(tm.shape)) for _ in range(ntr)]
+        st = [H(1e-2 * rng.standard_normal(tm[0].shape)) for _ in range(2 * ntr)]
+        group = [H(t) for t in Ts]
+        g.vert_diffuse_implicit(group, st[:ntr], st[ntr:], dcb, dh, dhw, 1800.0, index_salt=1)
+        for n in range(ntr):
+            one = H(Ts[n])
+            g.vert_diffuse_implicit([one], [st[n]], [st[ntr + n]], dcb, dh, dhw, 1800.0,
+                                    index_salt=0 if n == 1 else -1)
+            g.sync()
+            assert np.array_equal(group[n].to_host(), one.to_host()), (ntr, n)
+    g.close()
