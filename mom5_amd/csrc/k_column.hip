@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -548,6 +549,10 @@ template <int H, int NP = 1>
 __device__ __forceinline__ void twin_tile(const VdJobF &J, int tile, bool live = true) {
   __shared__ float xch_all[NP][2][2][64];    // [pair][tracer parity][half][column]
   __shared__ double ech_all[NP][2][64];
+  // the multipliers of the forward sweep, own lane, where they would not fit the
+  // registers (they spilled 220 B a lane at 40 slots)
+  constexpr bool PLDS = H > 32;
+  __shared__ float pm_all[PLDS ? NP : 1][PLDS ? 2 : 1][PLDS ? H : 1][64];
   const int pr = NP > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 7) : 0;
   float (*xch)[2][64] = xch_all[pr];
   double (*ech)[64] = ech_all[pr];
@@ -555,6 +560,7 @@ __device__ __forceinline__ void twin_tile(const VdJobF &J, int tile, bool live =
   const int half = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 1);
   const bool top = half == 0;
   const int lane = threadIdx.x & 63;
+  float (*pm)[64] = pm_all[PLDS ? pr : 0][PLDS ? half : 0];
   const int col = (tile % J.nbx) * 64 + lane;
   const bool valid = live && col < d.ni;
   const int nk = d.nk;
@@ -589,7 +595,7 @@ __device__ __forceinline__ void twin_tile(const VdJobF &J, int tile, bool live =
       Ldw[j] = ld_at(dwp + r * step, ob8);
     }
   };
-  float P[H], E[H];
+  float P[PLDS ? 1 : H], E[H];
   double Dp = 0.0, Wp = 1.0, mdp = 0.0, Eprev = 0.0;
   // bet and dh of the surface row (top) and of row kb (bottom flux)
   double bet1 = 0.0, dh1 = 1.0, betkb = 0.0, dhkb = 1.0;
@@ -624,7 +630,7 @@ __device__ __forceinline__ void twin_tile(const VdJobF &J, int tile, bool live =
       // that only they, not their FP64 sources, stay in registers
       float pj = (float)(p * bet), ej = (float)Eprev;
       asm volatile("" : "+v"(pj), "+v"(ej));
-      P[j] = pj;
+      if constexpr (PLDS) pm[j][lane] = pj; else P[j] = pj;
       E[j] = ej;
       if (real && lev == 1) { bet1 = bet; dh1 = dhk; }
       const bool atkb = real && lev == kb;
@@ -678,7 +684,9 @@ __device__ __forceinline__ void twin_tile(const VdJobF &J, int tile, bool live =
     for (int j = 0; j < H; ++j) {
       const float t1 = (j > 0 ? T[j - 1] - T[j] : 0.0f) + dprev;
       const float t2 = T[j + 1] - T[j];
-      float dj = fmaf(-P[j], t1, -(E[j] * t2));
+      float pj;
+      if constexpr (PLDS) pj = pm[j][lane]; else pj = P[j];
+      float dj = fmaf(-pj, t1, -(E[j] * t2));
       dj += (j == jsl) ? inj0 : 0.0f;
       dj += (j == jkb_l) ? injb : 0.0f;
       dv[j] = dj;
@@ -1941,20 +1949,38 @@ static int vdiff_mix_one(mom_gpu_ctx *ctx, int ntr, void *const *T, const int *d
 static int twin_slots(int nk) {
   if (nk < 2 || nk > 80) return 0;
   const int h = (nk + 1) / 2;
-  return h <= 8 ? 8 : h <= 16 ? 16 : h <= 24 ? 24 : h <= 32 ? 32 : 40;
+  for (int slots : {8, 12, 16, 20, 23, 26, 29, 32, 35, 38, 40})
+    if (h <= slots) return slots;
+  return 0;
+}
+
+// f(integral constant) for a count of slots that twin_slots returns.  Fine
+// steps: an unused slot costs its registers, and FP32 columns its arithmetic (T, S
+// at 1440x1080x50 in 26 slots instead of 32: SLOTNUM)
+template <typename F>
+static void with_slots(int h, F &&f) {
+  switch (h) {
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 12: f(std::integral_constant<int, 12>{}); break;
+    case 16: f(std::integral_constant<int, 16>{}); break;
+    case 20: f(std::integral_constant<int, 20>{}); break;
+    case 23: f(std::integral_constant<int, 23>{}); break;
+    case 26: f(std::integral_constant<int, 26>{}); break;
+    case 29: f(std::integral_constant<int, 29>{}); break;
+    case 32: f(std::integral_constant<int, 32>{}); break;
+    case 35: f(std::integral_constant<int, 35>{}); break;
+    case 38: f(std::integral_constant<int, 38>{}); break;
+    default: f(std::integral_constant<int, 40>{}); break;
+  }
 }
 
 static void launch_twin64(mom_gpu_ctx *ctx, VdJob<double> J) {
   const KDom &d = J.d;
   const int per_xcd = ((J.nblocks + 1) / 2 + 7) / 8;   // tile pairs per XCD
   const dim3 grid(8 * per_xcd), block(256);
-  switch (twin_slots(d.nk)) {
-    case 8: hipLaunchKernelGGL(k_vdiff_twin64<8>, grid, block, 0, ctx->stream, J, per_xcd); break;
-    case 16: hipLaunchKernelGGL(k_vdiff_twin64<16>, grid, block, 0, ctx->stream, J, per_xcd); break;
-    case 24: hipLaunchKernelGGL(k_vdiff_twin64<24>, grid, block, 0, ctx->stream, J, per_xcd); break;
-    case 32: hipLaunchKernelGGL(k_vdiff_twin64<32>, grid, block, 0, ctx->stream, J, per_xcd); break;
-    default: hipLaunchKernelGGL(k_vdiff_twin64<40>, grid, block, 0, ctx->stream, J, per_xcd); break;
-  }
+  with_slots(twin_slots(d.nk), [&](auto H) {
+    hipLaunchKernelGGL(k_vdiff_twin64<H.value>, grid, block, 0, ctx->stream, J, per_xcd);
+  });
 }
 
 static void launch_share(mom_gpu_ctx *ctx, const ShareJob &J) {
@@ -1979,13 +2005,9 @@ static void launch_twin(mom_gpu_ctx *ctx, VdJobF J) {
   J.nblocks = J.nbx * d.nj;
   const int per_xcd = ((J.nblocks + 1) / 2 + 7) / 8;   // tile pairs per XCD
   const dim3 grid(8 * per_xcd), block(256);
-  switch (twin_slots(d.nk)) {
-    case 8: hipLaunchKernelGGL(k_vdiff_twin<8>, grid, block, 0, ctx->stream, J, per_xcd); break;
-    case 16: hipLaunchKernelGGL(k_vdiff_twin<16>, grid, block, 0, ctx->stream, J, per_xcd); break;
-    case 24: hipLaunchKernelGGL(k_vdiff_twin<24>, grid, block, 0, ctx->stream, J, per_xcd); break;
-    case 32: hipLaunchKernelGGL(k_vdiff_twin<32>, grid, block, 0, ctx->stream, J, per_xcd); break;
-    default: hipLaunchKernelGGL(k_vdiff_twin<40>, grid, block, 0, ctx->stream, J, per_xcd); break;
-  }
+  with_slots(twin_slots(d.nk), [&](auto H) {
+    hipLaunchKernelGGL(k_vdiff_twin<H.value>, grid, block, 0, ctx->stream, J, per_xcd);
+  });
 }
 
 bool vdiff_fp32_scratch(const mom_gpu_ctx *c) {
@@ -2279,13 +2301,9 @@ int launch_vdiff_ensemble(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *step
       const dim3 grid(8 * per_xcd), block(128);
       hipStream_t st = e->lead->stream;
       const VdJob<double> *jt = (const VdJob<double> *)dev;
-      switch (h64) {
-        case 8: hipLaunchKernelGGL(k_vdiff_twin64_ens<8>, grid, block, 0, st, jt, L, per_xcd); break;
-        case 16: hipLaunchKernelGGL(k_vdiff_twin64_ens<16>, grid, block, 0, st, jt, L, per_xcd); break;
-        case 24: hipLaunchKernelGGL(k_vdiff_twin64_ens<24>, grid, block, 0, st, jt, L, per_xcd); break;
-        case 32: hipLaunchKernelGGL(k_vdiff_twin64_ens<32>, grid, block, 0, st, jt, L, per_xcd); break;
-        default: hipLaunchKernelGGL(k_vdiff_twin64_ens<40>, grid, block, 0, st, jt, L, per_xcd); break;
-      }
+      with_slots(h64, [&](auto H) {
+        hipLaunchKernelGGL(k_vdiff_twin64_ens<H.value>, grid, block, 0, st, jt, L, per_xcd);
+      });
       MOM_LAUNCHED(e->lead, "k_vdiff_twin64_ens");
     }
   }
@@ -2310,13 +2328,9 @@ int launch_vdiff_ensemble(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *step
     const int per_xcd = (total + 7) / 8;
     const dim3 grid(8 * per_xcd), block(128);
     hipStream_t st = e->lead->stream;
-    switch (hmax) {
-      case 8: hipLaunchKernelGGL(k_vdiff_twin_ens<8>, grid, block, 0, st, (const VdJobF *)dev, L, per_xcd); break;
-      case 16: hipLaunchKernelGGL(k_vdiff_twin_ens<16>, grid, block, 0, st, (const VdJobF *)dev, L, per_xcd); break;
-      case 24: hipLaunchKernelGGL(k_vdiff_twin_ens<24>, grid, block, 0, st, (const VdJobF *)dev, L, per_xcd); break;
-      case 32: hipLaunchKernelGGL(k_vdiff_twin_ens<32>, grid, block, 0, st, (const VdJobF *)dev, L, per_xcd); break;
-      default: hipLaunchKernelGGL(k_vdiff_twin_ens<40>, grid, block, 0, st, (const VdJobF *)dev, L, per_xcd); break;
-    }
+    with_slots(hmax, [&](auto H) {
+      hipLaunchKernelGGL(k_vdiff_twin_ens<H.value>, grid, block, 0, st, (const VdJobF *)dev, L, per_xcd);
+    });
     MOM_LAUNCHED(e->lead, "k_vdiff_twin_ens");
   }
   return MOM_GPU_OK;
