@@ -115,7 +115,8 @@ int mom_gpu_copy(mom_gpu_ctx_t *ctx, double *dst, const double *src, size_t n);
  * results on vdiff_solver).  Knobs:
  *   "barotropic_subcycles_per_launch"  0: three launches per subcycle (two for
  *                                      the variants); n>0: n subcycles per
- *                                      launch (1..12)
+ *                                      launch (1..12).  Until it is set (5 is
+ *                                      read back) it is chosen from the size
  *   "mdfl_rows_per_wave"               1, 2 or 4: rows a wavefront of the MDFL kernel
  *                                      (16 wavefronts with 1 row, 8 otherwise)
  *   "step_group_f64"                   1, 2 or 4 FP64 tracers per batched pass

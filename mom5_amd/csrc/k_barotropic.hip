@@ -11,8 +11,7 @@
 
 #include <algorithm>
 #include <cstring>
-
-#include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -206,13 +205,15 @@ __host__ __device__ constexpr int bt_lo(int nsub) { return nsub + 1; }
 __host__ __device__ constexpr int bt_interior(int n, int nsub) { return n - 2 * nsub - 1; }
 
 // sf: tmask * (pme + river + source - eta_smooth) and mask: bit 0 tmask(k=1),
-// bit 1 umask(k=1), formed once per call by k_bt_sfmask (constant over the
+// bit 1 umask(k=1), formed once per call by k_bt_prep (constant over the
 // subcycles) instead of being re-read from their six sources by every launch
 struct BtIn {
   const double *rho_g, *patm, *thicku, *forcing, *f;
   const double *dxu, *dyu, *datr, *dxur, *dyur;
   const double *sf;
   const unsigned char *mask;
+  const double *rowc;   // per row: datr, dyu/2, dxu/2, dxur/2, dyur/2, cori1, cori2,
+                         // f/2 (or null)
   int recip;   // dxur, dyur formed as 1/(dxu + epsln), 1/(dyu + epsln), not loaded
 };
 
@@ -221,13 +222,17 @@ constexpr double EPSLN_GRID = 1.0e-40;   // shared/constants/constants.F90:123
 // Per data-domain point: bit 0 where dxur or dyur is not, bit for bit, the
 // reciprocal ocean_grids.F90:949-951 forms; bit 1 where a metric the blocked
 // barotropic multiplies is outside LAND_BOUND in magnitude (or not a number)
-// or dxu, dyu, datr carries a sign bit.  The host ORs them up.
+// or dxu, dyu, datr carries a sign bit; bit 2 where a metric bt_rows_tile takes from
+// its row differs from the row's first point.  The host ORs them up.
 constexpr double LAND_BOUND = 1.0e100;
 __device__ inline bool bounded(double x) { return fabs(x) <= LAND_BOUND; }
 __global__ void k_check_recip(KDom d, const double *__restrict__ dxu,
                               const double *__restrict__ dxur, const double *__restrict__ dyu,
                               const double *__restrict__ dyur, const double *__restrict__ datr,
                               const double *__restrict__ f, int *__restrict__ bad) {
+  auto differ = [](double a, double b) {
+    return __builtin_bit_cast(unsigned long long, a) != __builtin_bit_cast(unsigned long long, b);
+  };
   const int ii = blockIdx.x * blockDim.x + threadIdx.x;
   const int o = ii + d.NI * blockIdx.y;
   if (ii >= d.NI) return;
@@ -239,7 +244,11 @@ __global__ void k_check_recip(KDom d, const double *__restrict__ dxu,
   const bool grid_bad = !(bounded(dxu[o]) && bounded(dyu[o]) && bounded(datr[o]) &&
                           bounded(dxur[o]) && bounded(dyur[o]) && bounded(f[o]) &&
                           !signbit(dxu[o]) && !signbit(dyu[o]) && !signbit(datr[o]));
-  bad[o] = (recip_bad ? 1 : 0) | (grid_bad ? 2 : 0);
+  const int r = d.NI * blockIdx.y;
+  const bool row_bad = differ(dxu[o], dxu[r]) || differ(dyu[o], dyu[r]) ||
+                       differ(dxur[o], dxur[r]) || differ(dyur[o], dyur[r]) ||
+                       differ(datr[o], datr[r]) || differ(f[o], f[r]);
+  bad[o] = (recip_bad ? 1 : 0) | (grid_bad ? 2 : 0) | (row_bad ? 4 : 0);
 }
 
 // The per-call inputs that decide whether a point is inert under the
@@ -247,18 +256,27 @@ __global__ void k_check_recip(KDom d, const double *__restrict__ dxu,
 struct Inert {
   const double *eta, *ud, *forcing, *rho_g, *patm, *thicku;
 };
-__global__ void k_bt_sfmask(KDom d, const double *__restrict__ pme,
-                            const double *__restrict__ river, const double *__restrict__ source,
-                            const double *__restrict__ eta_smooth, const int *__restrict__ kmt,
-                            const int *__restrict__ kmu, double *__restrict__ sf,
-                            unsigned char *__restrict__ mask, Inert x) {
-  const int ii = blockIdx.x * blockDim.x + threadIdx.x, jj = blockIdx.y;
-  if (ii >= d.NI) return;
+// What a call forms once: sf and the masks of every point and, for domains whose
+// rows are uniform in x (rowc not null), each row's constants.
+struct BtPrep {
+  KDom d;
+  const double *pme, *river, *source, *eta_smooth;
+  const int *kmt, *kmu;
+  double *sf;
+  unsigned char *mask;
+  Inert x;
+  const double *datr, *dyu, *dxu, *dxur, *dyur, *f;
+  double dtbt;
+  double *rowc;
+};
+__device__ __forceinline__ void bt_prep(const BtPrep &P, int ii, int jj) {
+  const KDom &d = P.d;
+  const Inert &x = P.x;
   const int o = ii + d.NI * jj;
-  const double tm = (1 <= kmt[o]) ? 1.0 : 0.0;
-  const double s = tm * (pme[o] + river[o] + source[o] - eta_smooth[o]);
-  sf[o] = s;
-  const bool t = 1 <= kmt[o], u = 1 <= kmu[o];
+  const double tm = (1 <= P.kmt[o]) ? 1.0 : 0.0;
+  const double s = tm * (P.pme[o] + P.river[o] + P.source[o] - P.eta_smooth[o]);
+  P.sf[o] = s;
+  const bool t = 1 <= P.kmt[o], u = 1 <= P.kmu[o];
   // inert: both masks 0, forcing and velocity zeros (either sign), sf a
   // zero, the fields multiplied into the pressure bounded
   const size_t P2 = (size_t)d.P2;
@@ -266,7 +284,24 @@ __global__ void k_bt_sfmask(KDom d, const double *__restrict__ pme,
                      x.forcing[o + P2] == 0.0 && x.ud[o] == 0.0 && x.ud[o + P2] == 0.0 &&
                      bounded(x.eta[o]) && bounded(x.rho_g[o]) && bounded(x.patm[o]) &&
                      bounded(x.thicku[o]);
-  mask[o] = (unsigned char)((t ? 1 : 0) | (u ? 2 : 0) | (inert ? 4 : 0));
+  P.mask[o] = (unsigned char)((t ? 1 : 0) | (u ? 2 : 0) | (inert ? 4 : 0));
+  if (P.rowc && ii == 0) {
+    double *r = P.rowc + (size_t)8 * jj;
+    const double fo = P.f[o], c1 = 0.5 * P.dtbt * fo;     // cori1, cori2 (:1285-1286)
+    r[0] = P.datr[o]; r[1] = 0.5 * P.dyu[o]; r[2] = 0.5 * P.dxu[o];
+    r[3] = 0.5 * P.dxur[o]; r[4] = 0.5 * P.dyur[o];
+    r[5] = c1; r[6] = 1.0 / (1.0 + c1 * c1); r[7] = 0.5 * fo;
+  }
+}
+__global__ void k_bt_prep(BtPrep P) {
+  const int ii = blockIdx.x * blockDim.x + threadIdx.x;
+  if (ii < P.d.NI) bt_prep(P, ii, blockIdx.y);
+}
+// ensembles: blockIdx.z is the domain
+__global__ void k_bt_prep_ens(const BtPrep *__restrict__ Ps) {
+  const BtPrep &P = Ps[blockIdx.z];
+  const int ii = blockIdx.x * blockDim.x + threadIdx.x, jj = blockIdx.y;
+  if (ii < P.d.NI && jj < P.d.NJ) bt_prep(P, ii, jj);
 }
 
 // One launch of the blocked subcycle for one domain: nsub subcycles from s0.
@@ -274,12 +309,51 @@ struct BtJob {
   KDom d;
   BtIn in;
   const double *eta_src, *ud_src;
+  const double *eb_src, *ub_src;   // the time sums so far (ub_src null: zero, the first launch)
   double *eta_dst, *ud_dst, *eb, *ub;
   int s0, nsub, nts, step_a;
   double dtbt, cp, cc;
-  int xbase, xcount, ntx, ntiles;
+  int xbase, xcount, ntx, ntiles, rev;
   const int *land;   // per tile: 1 where bt_tile may take its land path (null: none)
 };
+
+// Land path of a tile (a region of ry rows): every point of the region is inert
+// (k_bt_prep, mask bit 2).  There the velocity after each momentum phase is +0
+// (the pressure gradient is x*0.0, the forcing and the old velocity zeros,
+// dtbt > 0, and the Coriolis factors finite), so U*dyu and U*dxu are +0 with
+// dxu, dyu >= +0 and the divergence is +0; the corrector adds
+// cc*(-0*0.0 + sf) = cc*sf, a signed zero, to eta, and the time sums add eta and
+// +0.  The velocity sums start the call at +0 and every subcycle adds +0 to them
+// in either path.  The same values as the full path.
+__device__ __forceinline__ void bt_land_tile(const BtJob &J, int ry, int x_int0, int y_int0) {
+  const KDom d = J.d;
+  const bool cyc = d.cyclic_x != 0;
+  const int TX = bt_interior(BRX, J.nsub), TY = bt_interior(ry, J.nsub), LO = bt_lo(J.nsub);
+  const int lane = threadIdx.x % BRX;
+  const int vi = x_int0 - LO + lane;
+  const int col = cyc ? 1 + wrapi(vi - 1, d.ni) : vi;
+  for (int r = threadIdx.x / BRX; r < ry; r += blockDim.x / BRX) {
+    const int j = y_int0 - LO + r;
+    const bool inside = (cyc || (vi >= 0 && vi < d.NI)) && j >= 0 && j < d.NJ && lane >= LO &&
+                        lane < LO + TX && vi < J.xbase + J.xcount && r >= LO && r < LO + TY;
+    if (!inside) continue;
+    const int o = col + d.NI * j;
+    double e = J.eta_src[o], ebq = J.eb_src[o];
+    const double s = J.in.sf[o];
+    for (int t = 0; t < J.nsub; ++t) {
+      e = e + J.cc * s;
+      ebq = ebq + e;
+    }
+    J.eta_dst[o] = e;
+    J.ud_dst[o] = 0.0;
+    J.ud_dst[o + d.P2] = 0.0;
+    J.eb[o] = ebq;
+    if (!J.ub_src) {
+      J.ub[o] = 0.0;
+      J.ub[o + d.P2] = 0.0;
+    }
+  }
+}
 
 __device__ __forceinline__ void bt_tile(const BtJob &J, int tile) {
   const KDom d = J.d;
@@ -288,8 +362,10 @@ __device__ __forceinline__ void bt_tile(const BtJob &J, int tile) {
   const double *__restrict__ ud_src = J.ud_src;
   double *__restrict__ eta_dst = J.eta_dst;
   double *__restrict__ ud_dst = J.ud_dst;
-  double *__restrict__ eb = J.eb;
-  double *__restrict__ ub = J.ub;
+  // (a launch after the first reads the sums it writes)
+  const double *eb_src = J.eb_src, *ub_src = J.ub_src;
+  double *eb = J.eb;
+  double *ub = J.ub;
   const int s0 = J.s0, nsub = J.nsub, nts = J.nts, step_a = J.step_a;
   const double dtbt = J.dtbt, cp = J.cp, cc = J.cc;
   const int xbase = J.xbase, xcount = J.xcount, ntx = J.ntx;
@@ -304,37 +380,7 @@ __device__ __forceinline__ void bt_tile(const BtJob &J, int tile) {
   const bool cyc = d.cyclic_x != 0;
 
   if (J.land && J.land[tile]) {
-    // Land path: every point of the region is inert (k_bt_sfmask bit 2).
-    // There the velocity after each momentum phase is +0 (the pressure
-    // gradient is x*0.0, the forcing and the old velocity zeros, dtbt > 0,
-    // and the Coriolis factors finite), so U*dyu and U*dxu are +0 with
-    // dxu, dyu >= +0 and the divergence is +0; the corrector adds
-    // cc*(-0*0.0 + sf) = cc*sf, a signed zero, to eta, and the time sums
-    // add eta and +0.  The velocity sums start the call at +0
-    // (k_bt_acc_init) and every subcycle adds +0 to them in either path, so
-    // they are left as they are.  The same values as the full path.
-    const int vi = x_int0 - LO + lane;
-    const int col = cyc ? 1 + wrapi(vi - 1, d.ni) : vi;
-#pragma unroll
-    for (int q = 0; q < BPT; ++q) {
-      const int r = wave + (BNT / BRX) * q;
-      const int j = y_int0 - LO + r;
-      const bool inside = (cyc || (vi >= 0 && vi < d.NI)) && j >= 0 && j < d.NJ &&
-                          lane >= LO && lane < LO + TX && vi < xbase + xcount && r >= LO &&
-                          r < LO + TY;
-      if (!inside) continue;
-      const int o = col + d.NI * j;
-      double e = eta_src[o], ebq = eb[o];
-      const double s = in.sf[o];
-      for (int t = 0; t < nsub; ++t) {
-        e = e + cc * s;
-        ebq = ebq + e;
-      }
-      eta_dst[o] = e;
-      ud_dst[o] = 0.0;
-      ud_dst[o + P2] = 0.0;
-      eb[o] = ebq;
-    }
+    bt_land_tile(J, BRY, x_int0, y_int0);
     return;
   }
 
@@ -381,8 +427,11 @@ __device__ __forceinline__ void bt_tile(const BtJob &J, int tile) {
       }
       umb[q] = (mb & 2) != 0;
       eta[q] = eta_src[o]; u1[q] = ud_src[o]; u2[q] = ud_src[o + P2];
-      if (interior[q]) { ebv[q] = eb[o]; ub1[q] = ub[o]; ub2[q] = ub[o + P2]; }
-      else { ebv[q] = ub1[q] = ub2[q] = 0.0; }
+      ebv[q] = ub1[q] = ub2[q] = 0.0;
+      if (interior[q]) {
+        ebv[q] = eb_src[o];
+        if (ub_src) { ub1[q] = ub_src[o]; ub2[q] = ub_src[o + P2]; }
+      }
     } else {
       tmb[q] = umb[q] = false;
       sf[q] = datr[q] = dyu[q] = dxu[q] = rho_g[q] = patm[q] = thk[q] = 0.0;
@@ -494,11 +543,11 @@ __device__ __forceinline__ void bt_tile(const BtJob &J, int tile) {
 // 1 for a tile of nsub subcycles whose whole region (the points bt_tile
 // loads) is inert, 0 otherwise: one work-group a tile.
 __global__ __launch_bounds__(256) void k_bt_land(KDom d, const unsigned char *__restrict__ mask,
-                                                 int nsub, int xbase, int ntx, int ntiles,
-                                                 int *__restrict__ land) {
+                                                 int ry, int nsub, int xbase, int ntx,
+                                                 int ntiles, int *__restrict__ land) {
   const int tile = blockIdx.x;
   if (tile >= ntiles) return;                  // the whole block
-  const int TX = bt_interior(BRX, nsub), TY = bt_interior(BRY, nsub), LO = bt_lo(nsub);
+  const int TX = bt_interior(BRX, nsub), TY = bt_interior(ry, nsub), LO = bt_lo(nsub);
   const int x_int0 = xbase + (tile % ntx) * TX, y_int0 = (tile / ntx) * TY;
   const int lane = threadIdx.x % BRX;
   const int vi = x_int0 - LO + lane;
@@ -506,7 +555,7 @@ __global__ __launch_bounds__(256) void k_bt_land(KDom d, const unsigned char *__
   const int col = cyc ? 1 + wrapi(vi - 1, d.ni) : vi;
   const bool colok = cyc || (vi >= 0 && vi < d.NI);
   int ok = 1;
-  for (int r = threadIdx.x / BRX; r < BRY; r += 256 / BRX) {
+  for (int r = threadIdx.x / BRX; r < ry; r += 256 / BRX) {
     const int j = y_int0 - LO + r;
     if (colok && j >= 0 && j < d.NJ && !(mask[col + d.NI * j] & 4)) ok = 0;
   }
@@ -514,15 +563,237 @@ __global__ __launch_bounds__(256) void k_bt_land(KDom d, const unsigned char *__
   if (threadIdx.x == 0) land[tile] = ok;
 }
 
+// bt_tile for a domain whose dxu, dyu, datr, dxur, dyur and f are the same, bit for
+// bit, along every row (spherical grids: launch_check_recip).  A row's constants
+// are then wavefront-uniform and lie in scalar registers, x neighbours come by
+// lane shifts, y neighbours from the thread's own rows but for one row a
+// wavefront each way (LDS).  What bounds it: memory a launch (18 planes once, the
+// nine of them that regions share up to twice) against 54 FP64 instructions a
+// point and subcycle, so a region wants many subcycles (fewer launches) and few
+// redundant points, and two blocks share a CU so that one loads while the other
+// steps: 8 wavefronts of 3 rows (64 x 24) or 4 (64 x 32, thickness and forcing in
+// LDS).  3600 x 2700, 120 subcycles, ms at the best depth: bt_tile 13.7 (5); one
+// block of 16 wavefronts, 2 rows 9.8 (6), 3 rows 8.2 (7), 4 rows 8.1 (10); 12
+// wavefronts of 2 rows 11.6 (5), 10 of 3 rows 11.0 (6); 8 of 3 rows 8.4 (6), 8 of
+// 4 rows 8.0 (6), 7.8 with every other launch backwards.  517 x 389, 80
+// subcycles, three states in turn: 241 us (bt_tile) to 121.
+// The same values as bt_tile, instructions saved:
+// - tmask into datr and umask into thicku: x*m is x or a zero of x's sign, as is
+//   the product's (a NaN stays one); the pressure force's zero loses its sign in
+//   the sum with forcing + 0.0, which is never -0;
+// - 0.5*(a + b) and its differences: the halves are in the row constants
+//   (a power of two, exact short of the subnormals);
+// - the corrector's divergence is the next predictor's.
+// Regions inside the domain skip the edge rows' and columns' tests (EDGE).
+// Points outside the domain read a clamped place: no value of theirs reaches a
+// point inside (the divergence is 0 on the first row and column, the gradient on
+// the last).
+template <int R, int NW>
+struct BtRowsLds {
+  // four rows: thickness and forcing in LDS (own lane)
+  static constexpr bool CL = R >= 4;
+  double p[NW][BRX], u[NW][BRX], v[NW][BRX];
+  double c[CL ? 3 : 1][CL ? R : 1][CL ? NW : 1][BRX];
+};
+template <int R, int NW, bool EDGE>
+__device__ __forceinline__ void bt_rows_tile(const BtJob &J, int x_int0, int y_int0,
+                                             BtRowsLds<R, NW> &S) {
+  constexpr int RY = NW * R;
+  constexpr bool CL = BtRowsLds<R, NW>::CL;
+  const KDom d = J.d;
+  const int nsub = J.nsub, P2 = d.P2;
+  const bool cyc = d.cyclic_x != 0;
+  auto &s_p = S.p, &s_u = S.u, &s_v = S.v;
+  auto &s_c = S.c;
+  const int TX = bt_interior(BRX, nsub), TY = bt_interior(RY, nsub), LO = bt_lo(nsub);
+  const int lane = threadIdx.x & (BRX - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / BRX);
+  const int wm = max(wave - 1, 0), wp = min(wave + 1, NW - 1);
+  const int vi = x_int0 - LO + lane;
+  int col;
+  if (!cyc) {
+    col = min(max(vi, 0), d.NI - 1);
+  } else if (d.ni >= 2 * BRX) {
+    int g = vi - 1;
+    g = g < 0 ? g + d.ni : g;
+    col = 1 + (g >= d.ni ? g - d.ni : g);
+  } else {
+    col = 1 + wrapi(vi - 1, d.ni);
+  }
+  const unsigned cb = (unsigned)col * 8u;
+  const bool lin = lane >= LO && lane < LO + TX && vi < J.xbase + J.xcount;
+  const int row0 = y_int0 - LO + R * wave;
+  typedef const __attribute__((address_space(4))) double ConstD;
+  double eta[R], u1[R], u2[R], eb[R], ub1[R], ub2[R], g[R], uh[R], vh[R];
+  double sf[R], rg[R], pa[R], th[CL ? 1 : R], F1[CL ? 1 : R], F2[CL ? 1 : R];
+  double dm[R];                                                       // datr*tmask
+  double hdyu[R], hdxu[R], hdxur[R], hdyur[R], c1[R], c2[R], hf[R];   // uniform
+  auto inside = [&](int q) {
+    const int r = R * wave + q;
+    return lin && row0 + q >= 0 && row0 + q < d.NJ && r >= LO && r < LO + TY;
+  };
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int j = row0 + q, jc = min(max(j, 0), d.NJ - 1);      // uniform
+    const int ro = d.NI * jc;
+    ConstD *rc = (ConstD *)(unsigned long long)(J.in.rowc + (size_t)8 * jc);
+    hdyu[q] = rc[1]; hdxu[q] = rc[2]; hdxur[q] = rc[3]; hdyur[q] = rc[4];
+    c1[q] = rc[5]; c2[q] = rc[6]; hf[q] = rc[7];
+    const unsigned char mb = J.in.mask[ro + col];
+    eta[q] = ld_lv(J.eta_src + ro, cb);
+    u1[q] = ld_lv(J.ud_src + ro, cb);
+    u2[q] = ld_lv(J.ud_src + P2 + ro, cb);
+    sf[q] = ld_lv(J.in.sf + ro, cb);
+    rg[q] = ld_lv(J.in.rho_g + ro, cb);
+    pa[q] = ld_lv(J.in.patm + ro, cb);
+    // datr*tmask; thicku*umask; the forcing + 0.0
+    dm[q] = rc[0] * ((mb & 1) ? 1.0 : 0.0);
+    const double tq = ld_lv(J.in.thicku + ro, cb) * ((mb & 2) ? 1.0 : 0.0),
+                 f1q = ld_lv(J.in.forcing + ro, cb) + 0.0,
+                 f2q = ld_lv(J.in.forcing + P2 + ro, cb) + 0.0;
+    if constexpr (CL) {
+      s_c[0][q][wave][lane] = tq;
+      s_c[1][q][wave][lane] = f1q;
+      s_c[2][q][wave][lane] = f2q;
+    } else {
+      th[q] = tq; F1[q] = f1q; F2[q] = f2q;
+    }
+    eb[q] = ub1[q] = ub2[q] = 0.0;
+    if (inside(q)) {
+      eb[q] = ld_lv(J.eb_src + ro, cb);
+      if (J.ub_src) {
+        ub1[q] = ld_lv(J.ub_src + ro, cb);
+        ub2[q] = ld_lv(J.ub_src + P2 + ro, cb);
+      }
+    }
+  }
+  auto share = [&]() {
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      uh[q] = u1[q] * hdyu[q];
+      vh[q] = u2[q] * hdxu[q];
+    }
+    s_u[wave][lane] = uh[R - 1];
+    s_v[wave][lane] = vh[R - 1];
+  };
+  // g = -DIV_UD*tmask + sf.  bay(row) = (uh(row) + uh(row - 1))/2 and
+  // bax(row) = (vh + vh west)/2; the halves are in dyu and dxu
+  auto diverge = [&]() {
+    double bx = s_v[wm][lane], um = s_u[wm][lane];
+    bx = bx + lane_prev(bx);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const double bay = uh[q] + um, bax = vh[q] + lane_prev(vh[q]);
+      double dv = ((bay - lane_prev(bay)) + (bax - bx)) * dm[q];
+      if (EDGE && (row0 + q == 0 || (!cyc && vi == 0))) dv = 0.0;
+      g[q] = sf[q] - dv;
+      um = uh[q];
+      bx = bax;
+    }
+  };
+  share();
+  __syncthreads();
+  diverge();
+  for (int t = 0; t < nsub; ++t) {
+    // A: predictor and surface pressure
+    double p[R + 1];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const double es = eta[q] + J.cp * g[q];
+      p[q] = rg[q] * es + pa[q];
+    }
+    s_p[wave][lane] = p[0];
+    __syncthreads();
+    // B: pressure gradient (the halves are in dxur and dyur) and momentum with
+    // implicit Coriolis
+    p[R] = s_p[wp][lane];
+    double pe = lane_next(p[0]), fax = p[0] + pe;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const double pne = lane_next(p[q + 1]);
+      const double fay = p[q] + p[q + 1], pip = pe + pne, pjp = p[q + 1] + pne;
+      double g1 = (pip - fay) * hdxur[q], g2 = (pjp - fax) * hdyur[q];
+      if (EDGE && (row0 + q == d.NJ - 1 || (!cyc && vi == d.NI - 1))) g1 = g2 = 0.0;
+      double thq, f1q, f2q;
+      if constexpr (CL) {
+        thq = s_c[0][q][wave][lane]; f1q = s_c[1][q][wave][lane]; f2q = s_c[2][q][wave][lane];
+      } else {
+        thq = th[q]; f1q = F1[q]; f2q = F2[q];
+      }
+      const double t1 = u1[q] + J.dtbt * (hf[q] * u2[q] - thq * g1 + f1q);
+      const double t2 = u2[q] + J.dtbt * (-(hf[q] * u1[q]) - thq * g2 + f2q);
+      u1[q] = c2[q] * (t1 + c1[q] * t2);
+      u2[q] = c2[q] * (t2 - c1[q] * t1);
+      pe = pne;
+      fax = pjp;
+    }
+    share();      // the previous phase C's reads finished before the barrier above
+    __syncthreads();
+    // C: corrector and time-average accumulation
+    diverge();
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      eta[q] = eta[q] + J.cc * g[q];
+      eb[q] = eb[q] + eta[q];
+    }
+    const double wgt = J.step_a ? 1.0 : (double)(J.nts - (J.s0 + t) + 1);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      ub1[q] = ub1[q] + wgt * u1[q];
+      ub2[q] = ub2[q] + wgt * u2[q];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    if (!inside(q)) continue;
+    const int ro = d.NI * (row0 + q);
+    st_lv(J.eta_dst + ro, cb, eta[q]);
+    st_lv(J.ud_dst + ro, cb, u1[q]);
+    st_lv(J.ud_dst + P2 + ro, cb, u2[q]);
+    st_lv(J.eb + ro, cb, eb[q]);
+    st_lv(J.ub + ro, cb, ub1[q]);
+    st_lv(J.ub + P2 + ro, cb, ub2[q]);
+  }
+}
+
+// The tiles: bt_tile, or bt_rows_tile of 8 wavefronts with 3 or 4 rows each
+constexpr int BT_ANY = 0, BT_ROWS3 = 3, BT_ROWS4 = 4;
+__host__ __device__ constexpr int bt_nw(int tile) { return tile == BT_ANY ? BNT / 64 : 8; }
+__host__ __device__ constexpr int bt_ry(int tile) { return tile == BT_ANY ? BRY : 8 * tile; }
+template <int T>
+__device__ __forceinline__ void bt_any_tile(const BtJob &J, int tile) {
+  if constexpr (T == BT_ANY) {
+    bt_tile(J, tile);
+  } else {
+    constexpr int NW = bt_nw(T), RY = bt_ry(T);
+    __shared__ BtRowsLds<T, NW> lds;
+    const KDom &d = J.d;
+    const int LO = bt_lo(J.nsub);
+    const int x0 = J.xbase + (tile % J.ntx) * bt_interior(BRX, J.nsub);
+    const int y0 = (tile / J.ntx) * bt_interior(RY, J.nsub);
+    // a region that meets the first row or column (divergence 0) or the last
+    // (gradient 0)
+    const bool edge = y0 - LO <= 0 || y0 - LO + RY >= d.NJ ||
+                      (!d.cyclic_x && (x0 - LO <= 0 || x0 - LO + BRX >= d.NI));
+    if (J.land && J.land[tile]) bt_land_tile(J, RY, x0, y0);
+    else if (edge) bt_rows_tile<T, NW, true>(J, x0, y0, lds);
+    else bt_rows_tile<T, NW, false>(J, x0, y0, lds);
+  }
+}
+
 // Tiles in XCD-aware order: blocks are dealt to the 8 XCDs round-robin, so
 // each XCD takes per_xcd consecutive positions of the order of 8-wide strips
 // (strip_tile) and the halo rows and columns that neighbouring tiles both
 // read are fetched into one L2.
-__global__ __launch_bounds__(BNT) void k_bt_block(BtJob J, int per_xcd) {
+template <int T>
+__global__ __launch_bounds__(64 * bt_nw(T), 4) void k_bt_block(BtJob J, int per_xcd) {
   const int b = blockIdx.x;
-  const int t = (b & 7) * per_xcd + (b >> 3);
+  // every other launch goes backwards: the planes the last tiles of one launch
+  // wrote are in the cache for the first tiles of the next
+  const int i = J.rev ? per_xcd - 1 - (b >> 3) : b >> 3;
+  const int t = (b & 7) * per_xcd + i;
   if (t >= J.ntiles) return;
-  bt_tile(J, strip_tile<8>(t, J.ntx, J.ntiles / J.ntx));
+  bt_any_tile<T>(J, strip_tile<8>(t, J.ntx, J.ntiles / J.ntx));
 }
 
 // Ensemble: launch ell of every domain that still has subcycles; the static
@@ -531,7 +802,7 @@ constexpr int BT_MAXDOM = 64;
 struct BtDom {
   KDom d;
   BtIn in;
-  const double *eta_bar_tau, *ud_tau;
+  const double *eta_bar_tau, *ud_tau, *eb0;   // the first launch's state and height sum
   double *eta_buf[2], *ud_buf[2];
   double *eb, *ub;
   int nts, step_a;
@@ -540,21 +811,24 @@ struct BtDom {
 };
 struct BtLaunch {
   int first[BT_MAXDOM + 1];   // first tile of each domain in this launch
-  int ndom, ell, hsub;
+  int ndom, ell, hsub, ry;
 };
 
-__device__ __host__ inline void bt_shape(const BtDom &D, int ell, int hsub, int &nsub, int &ntx,
+__device__ __host__ inline void bt_shape(const BtDom &D, const BtLaunch &L, int &nsub, int &ntx,
                                          int &ntiles) {
-  const int left = D.nts - ell * hsub;
-  nsub = left < hsub ? left : hsub;
+  const int left = D.nts - L.ell * L.hsub;
+  nsub = left < L.hsub ? left : L.hsub;
   if (nsub <= 0) { nsub = 0; ntx = 0; ntiles = 0; return; }
-  const int TX = bt_interior(BRX, nsub), TY = bt_interior(BRY, nsub);
+  const int TX = bt_interior(BRX, nsub), TY = bt_interior(L.ry, nsub);
   ntx = (D.xcount + TX - 1) / TX;
   ntiles = ntx * ((D.d.NJ + TY - 1) / TY);
 }
 
-__global__ __launch_bounds__(BNT) void k_bt_block_ens(const BtDom *__restrict__ doms, BtLaunch L) {
-  const int b = blockIdx.x;
+// Every domain's tiles in one order, dealt to the XCDs in contiguous runs.
+template <int T>
+__global__ __launch_bounds__(64 * bt_nw(T), 4) void k_bt_block_ens(const BtDom *__restrict__ doms,
+                                                                   BtLaunch L, int per_xcd) {
+  const int b = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (b >= L.first[L.ndom]) return;
   int lo = 0, hi = L.ndom - 1;
   while (lo < hi) {
@@ -566,9 +840,12 @@ __global__ __launch_bounds__(BNT) void k_bt_block_ens(const BtDom *__restrict__ 
   J.d = D.d;
   J.in = D.in;
   int nsub, ntx, ntiles;
-  bt_shape(D, L.ell, L.hsub, nsub, ntx, ntiles);
-  J.eta_src = L.ell == 0 ? D.eta_bar_tau : D.eta_buf[(L.ell - 1) & 1];
-  J.ud_src = L.ell == 0 ? D.ud_tau : D.ud_buf[(L.ell - 1) & 1];
+  bt_shape(D, L, nsub, ntx, ntiles);
+  const bool first = L.ell == 0;
+  J.eta_src = first ? D.eta_bar_tau : D.eta_buf[(L.ell - 1) & 1];
+  J.ud_src = first ? D.ud_tau : D.ud_buf[(L.ell - 1) & 1];
+  J.eb_src = first ? D.eb0 : D.eb;
+  J.ub_src = first ? nullptr : D.ub;
   J.eta_dst = D.eta_buf[L.ell & 1];
   J.ud_dst = D.ud_buf[L.ell & 1];
   J.eb = D.eb;
@@ -584,71 +861,71 @@ __global__ __launch_bounds__(BNT) void k_bt_block_ens(const BtDom *__restrict__ 
   J.xcount = D.xcount;
   J.ntx = ntx;
   J.ntiles = ntiles;
+  J.rev = 0;
   J.land = nullptr;
-  bt_tile(J, b - L.first[lo]);
+  bt_any_tile<T>(J, strip_tile<8>(b - L.first[lo], ntx, ntiles / ntx));
 }
 
-__global__ void k_bt_acc_init(KDom d, int initsum, const double *__restrict__ eta_t,
-                              const double *__restrict__ eta_bar_tau, double *__restrict__ eta_bar,
-                              double *__restrict__ ud) {
-  const int ii = blockIdx.x * blockDim.x + threadIdx.x, jj = blockIdx.y;
-  if (ii >= d.NI) return;
-  const int o = ii + d.NI * jj;
-  eta_bar[o] = initsum ? eta_bar_tau[o] : eta_t[o];
-  ud[o] = 0.0;
-  ud[o + d.P2] = 0.0;
-}
-
-// Ensemble tails: blockIdx.z is the domain.
+// Tail of update_ocean_barotropic (:2804-2811, :2846-2888) from the time sums of
+// the blocked subcycles (scratch planes, so that a point may read its neighbours'
+// and its cyclic source's): the means, halo columns of the compute rows at
+// their cyclic source, and conv_rho_ud_t = -DIV_UD of them, in one pass.  The
+// halo columns of the first and last row, which no subcycle touches on a
+// cyclic-x domain, hold the initial sums.
 struct BtTail {
   KDom d;
-  int initsum;
-  const double *eta_t, *eta_bar_tau;
+  const double *eb0, *eb, *ub;
   double *eta_bar, *ud, *conv;
   double rntsp1, rnts;
   const double *dxu, *dyu, *datr;
 };
-
-__global__ void k_bt_acc_init_ens(const BtTail *__restrict__ T) {
-  const BtTail &t = T[blockIdx.z];
-  const int ii = blockIdx.x * blockDim.x + threadIdx.x, jj = blockIdx.y;
-  if (ii >= t.d.NI || jj >= t.d.NJ) return;
-  const int o = ii + t.d.NI * jj;
-  t.eta_bar[o] = t.initsum ? t.eta_bar_tau[o] : t.eta_t[o];
-  t.ud[o] = 0.0;
-  t.ud[o + t.d.P2] = 0.0;
-}
-
-__global__ void k_bt_scale_ens(const BtTail *__restrict__ T) {
-  const BtTail &t = T[blockIdx.z];
-  const int ii = blockIdx.x * blockDim.x + threadIdx.x, jj = blockIdx.y;
-  if (ii >= t.d.NI || jj >= t.d.NJ) return;
-  const int o = ii + t.d.NI * jj;
-  t.eta_bar[o] = t.rntsp1 * t.eta_bar[o];
-  t.ud[o] = t.rnts * t.ud[o];
-  t.ud[o + t.d.P2] = t.rnts * t.ud[o + t.d.P2];
-}
-
-// what: 0 = eta_bar and ud (after scaling), 1 = conv
-__global__ void k_bt_wrap_ens(const BtTail *__restrict__ T, int what) {
-  const BtTail &t = T[blockIdx.z];
-  const int jj = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  if (!t.d.cyclic_x || jj > t.d.NJ - 2) return;
-  if (what == 1 && !t.conv) return;
-  double *planes[3] = {what ? t.conv : t.eta_bar, t.ud, t.ud + t.d.P2};
-  const int np = what ? 1 : 3;
-  for (int c = 0; c < np; ++c) {
-    double *p = planes[c] + (size_t)t.d.NI * jj;
-    p[0] = p[t.d.NI - 2];
-    p[t.d.NI - 1] = p[1];
+__device__ __forceinline__ void bt_tail(const BtTail &T, int ii, int jj) {
+  const KDom &d = T.d;
+  const bool crow = jj >= 1 && jj <= d.NJ - 2;
+  // the point whose sums a point takes; -1: none (a halo column the subcycles leave)
+  auto source = [&](int i, int j) {
+    if (!d.cyclic_x || (i >= 1 && i <= d.ni)) return i + d.NI * j;
+    if (j < 1 || j > d.NJ - 2) return -1;
+    return (i == 0 ? d.ni : 1) + d.NI * j;
+  };
+  const int o = ii + d.NI * jj, os = source(ii, jj);
+  T.eta_bar[o] = T.rntsp1 * (os >= 0 ? T.eb[os] : T.eb0[o]);
+  auto mean = [&](int c, int i, int j) {
+    const int q = source(i, j);
+    return T.rnts * (q >= 0 ? T.ub[(size_t)d.P2 * c + q] : 0.0);
+  };
+  const double u = mean(0, ii, jj), v = mean(1, ii, jj);
+  T.ud[o] = u;
+  T.ud[d.P2 + o] = v;
+  if (!T.conv) return;
+  // conv at the point, or at its cyclic source
+  int si = ii;
+  if (d.cyclic_x && crow) si = ii == 0 ? d.ni : (ii == d.NI - 1 ? 1 : ii);
+  double dv = 0.0;
+  if (si != 0 && jj != 0) {
+    const int so = si + d.NI * jj, sm = so - d.NI;
+    const double uh = mean(0, si, jj) * T.dyu[so], vh = mean(1, si, jj) * T.dxu[so];
+    const double uhjm = mean(0, si, jj - 1) * T.dyu[sm], vhjm = mean(1, si, jj - 1) * T.dxu[sm];
+    const double uhim = mean(0, si - 1, jj) * T.dyu[so - 1];
+    const double vhim = mean(1, si - 1, jj) * T.dxu[so - 1];
+    const double uhimjm = mean(0, si - 1, jj - 1) * T.dyu[sm - 1];
+    const double vhimjm = mean(1, si - 1, jj - 1) * T.dxu[sm - 1];
+    const double uh_bay = 0.5 * (uh + uhjm);
+    const double vh_bax = 0.5 * (vh + vhim);
+    const double uhim_bay = 0.5 * (uhim + uhimjm);
+    const double vhjm_bax = 0.5 * (vhjm + vhimjm);
+    dv = ((uh_bay - uhim_bay) + (vh_bax - vhjm_bax)) * T.datr[so];
   }
+  T.conv[o] = -dv;
 }
-
-__global__ void k_bt_conv_ens(const BtTail *__restrict__ T) {
-  const BtTail &t = T[blockIdx.z];
+__global__ void k_bt_tail(BtTail T) {
+  const int ii = blockIdx.x * blockDim.x + threadIdx.x;
+  if (ii < T.d.NI) bt_tail(T, ii, blockIdx.y);
+}
+__global__ void k_bt_tail_ens(const BtTail *__restrict__ Ts) {
+  const BtTail &T = Ts[blockIdx.z];
   const int ii = blockIdx.x * blockDim.x + threadIdx.x, jj = blockIdx.y;
-  if (!t.conv || ii >= t.d.NI || jj >= t.d.NJ) return;
-  t.conv[ii + t.d.NI * jj] = -div_ud(t.d, t.ud, t.ud + t.d.P2, t.dxu, t.dyu, t.datr, ii, jj);
+  if (ii < T.d.NI && jj < T.d.NJ) bt_tail(T, ii, jj);
 }
 
 // ocean_barotropic_forcing (ocean_barotropic.F90:3058-3141, default namelist,
@@ -806,7 +1083,8 @@ __global__ void k_bt_closure(KDom d, ClosureIn c, double *__restrict__ eta_u,
 }  // namespace
 
 // Sets ctx->bt_recip: whether the context's dxur and dyur are the reciprocals
-// the blocked barotropic may form itself (then it loads two planes fewer).
+// the blocked barotropic may form itself (then it loads two planes fewer), and
+// the other checks of the grid.
 int launch_check_recip(mom_gpu_ctx *ctx) {
   const KDom &d = ctx->kd;
   const size_t n = (size_t)d.P2;
@@ -832,8 +1110,83 @@ int launch_check_recip(mom_gpu_ctx *ctx) {
   free(host);
   ctx->bt_recip = (bad & 1) == 0;
   ctx->bt_grid_ok = (bad & 2) == 0;
+  // (the rows' constants lie behind the masks in one plane: 64 B a row)
+  ctx->bt_rows_ok = (bad & 4) == 0 && d.NI >= 16;
   return MOM_GPU_OK;
 }
+
+namespace {
+// The planes of ctx->bt as the blocked subcycles use them: 0-5 the state, two
+// sets; 6 sf; 7 the masks (a byte a point) and behind them the row constants; 8
+// the tiles' land flags (at most one int a point: a tile's interior holds at
+// least one); 9-11 the time sums.
+struct BtBufs {
+  double *eta[2], *ud[2], *sf, *rowc, *eb, *ub;
+  unsigned char *mask;
+  int *land;
+  explicit BtBufs(mom_gpu_ctx *ctx) {
+    const size_t P2 = (size_t)ctx->kd.P2;
+    double *b = ctx->bt;
+    eta[0] = b; eta[1] = b + P2;
+    ud[0] = b + 2 * P2; ud[1] = b + 4 * P2;
+    sf = b + 6 * P2;
+    mask = (unsigned char *)(b + 7 * P2);
+    rowc = b + 7 * P2 + (P2 + 7) / 8;
+    land = (int *)(b + 8 * P2);
+    eb = b + 9 * P2;
+    ub = b + 10 * P2;
+  }
+};
+
+// Tile and subcycles a launch for domains d[0..n) launched together.  Results do
+// not depend on either.  rows: every domain's rows are uniform; h: subcycles asked
+// for, 0 to choose.
+// - While the tiles leave CUs idle a launch's time is its latency, so the deepest
+//   launches win: 90 x 60, 80 subcycles, 5 / 10 a launch: 165 / 120 us (alone),
+//   63 / 50 (three states in turn); 360 x 240, 5 / 7: 178 / 159, 83 / 81; above
+//   one tile a CU, 517 x 389, 5 / 7: 254 / 228 but 126 / 144.  The general tile,
+//   one block a CU: 90 x 60, 5 / 12: 256 / 186 and 95 / 69, 360 x 240, 5 / 8:
+//   268 / 214 and 122 / 120, past 128 tiles 517 x 389, 5 / 7: 286 / 255, 241 / 240.
+// - Three rows a wavefront have the shorter chain (90 x 60, 10 a launch: 120 us
+//   against 186), four the fewer redundant points: they win once the 18 planes are
+//   larger than the 256 MB cache and every launch is paid in memory traffic (1440
+//   x 1080: 933 us with three, 1010 with four; 3600 x 2700: 8404 and 7975), and
+//   at depths that leave the lower region no interior.
+struct BtPlan {
+  int tile, hsub;
+};
+int bt_tiles(const KDom *const *d, int n, int tile, int h) {
+  const int TX = bt_interior(BRX, h), TY = bt_interior(bt_ry(tile), h);
+  int t = 0;
+  for (int k = 0; k < n; ++k)
+    t += (((d[k]->cyclic_x ? d[k]->ni : d[k]->NI) + TX - 1) / TX) * ((d[k]->NJ + TY - 1) / TY);
+  return t;
+}
+BtPlan bt_plan(const KDom *const *d, int n, bool rows, int h) {
+  if (!rows) {
+    if (h == 0)
+      for (h = 12; h > 5 && bt_tiles(d, n, BT_ANY, h) > 128; --h) {}
+    return {BT_ANY, h};
+  }
+  size_t bytes = 0;
+  for (int k = 0; k < n; ++k) bytes += (size_t)d[k]->P2 * 18 * sizeof(double);
+  const bool large = bytes > (size_t)256 << 20;
+  if (h == 0) {
+    h = 6;
+    if (!large)
+      for (h = 10; h > 5 && bt_tiles(d, n, BT_ROWS3, h) > 256; --h) {}
+  }
+  if (large || h > 10 || (h > 7 && bt_tiles(d, n, BT_ROWS3, h) > 256)) return {BT_ROWS4, h};
+  return {BT_ROWS3, h};
+}
+
+template <typename F>
+void bt_with_tile(int tile, F &&f) {
+  if (tile == BT_ANY) f(std::integral_constant<int, BT_ANY>{});
+  else if (tile == BT_ROWS3) f(std::integral_constant<int, BT_ROWS3>{});
+  else f(std::integral_constant<int, BT_ROWS4>{});
+}
+}  // namespace
 
 int launch_barotropic_blocked(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p,
                               const double *eta_t, const double *eta_bar_tau,
@@ -849,64 +1202,59 @@ int launch_barotropic_blocked(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p,
   const double c_pred = p->dtbt * p->pred_corr_gamma * rho0r;   // dtbt_gamma_rho0r, :1196
   const double c_corr = p->dtbt * rho0r;                        // dtbt_rho0r, :1197
   const dim3 grid((d.NI + 255) / 256, d.NJ), block(256);
-  hipLaunchKernelGGL(k_bt_acc_init, grid, block, 0, s, d, p->initsum_with_bar, eta_t,
-                     eta_bar_tau, eta_bar, ud);
-  MOM_LAUNCHED(ctx, "k_bt_acc_init");
-  // sf and the masks in planes 6 and 7 of the subcycle buffer (0-5 hold the
-  // ping-pong state)
-  double *sfp = ctx->bt + 6 * P2;
-  unsigned char *maskp = (unsigned char *)(ctx->bt + 7 * P2);
+  const BtBufs w(ctx);
   // the land path's conditions that do not depend on the data
   const bool land_ok = ctx->tune.bt_land_tiles && ctx->bt_grid_ok && p->dtbt > 0.0 &&
                        std::isfinite(c_pred) && std::isfinite(c_corr);
   const Inert inert = land_ok ? Inert{eta_bar_tau, ud_tau, forcing, rho_g, patm, thicku} : Inert{};
-  hipLaunchKernelGGL(k_bt_sfmask, grid, block, 0, s, d, pme, river, source, eta_smooth,
-                     ctx->kmt, ctx->kmu, sfp, maskp, inert);
-  BtIn in{rho_g, patm, thicku, forcing, ctx->f, ctx->dxu, ctx->dyu, ctx->datr, ctx->dxur,
-          ctx->dyur, sfp, maskp, ctx->bt_recip};
-  // tile flags in plane 8 (unused by the blocked path): at most one int a
-  // point, as a tile's interior holds at least one point
-  int *landp = land_ok ? (int *)(ctx->bt + 8 * P2) : nullptr;
+  const double *rowc = ctx->bt_rows_ok ? w.rowc : nullptr;
+  hipLaunchKernelGGL(k_bt_prep, grid, block, 0, s,
+                     BtPrep{d, pme, river, source, eta_smooth, ctx->kmt, ctx->kmu, w.sf, w.mask,
+                            inert, ctx->datr, ctx->dyu, ctx->dxu, ctx->dxur, ctx->dyur, ctx->f,
+                            p->dtbt, (double *)rowc});
+  MOM_LAUNCHED(ctx, "k_bt_prep");
+  const BtIn in{rho_g, patm, thicku, forcing, ctx->f, ctx->dxu, ctx->dyu, ctx->datr, ctx->dxur,
+                ctx->dyur, w.sf, w.mask, rowc, ctx->bt_recip};
+  int *landp = land_ok ? w.land : nullptr;
   int land_nsub = 0;
   const int xbase = d.cyclic_x ? 1 : 0, xcount = d.cyclic_x ? d.ni : d.NI;
-  double *eta_buf[2] = {ctx->bt, ctx->bt + P2};
-  double *ud_buf[2] = {ctx->bt + 2 * P2, ctx->bt + 4 * P2};
+  const KDom *const one = &d;
+  const BtPlan plan = bt_plan(&one, 1, rowc != nullptr, hsub);
+  const int ry = bt_ry(plan.tile);
+  hsub = plan.hsub;
+  const double *eb0 = p->initsum_with_bar ? eta_bar_tau : eta_t;
   const double *eta_src = eta_bar_tau, *ud_src = ud_tau;
   int which = 0;
   for (int s0 = 1; s0 <= p->nts; s0 += hsub) {
     const int nsub = std::min(hsub, p->nts - s0 + 1);
-    const int TX = bt_interior(BRX, nsub), TY = bt_interior(BRY, nsub);
+    const int TX = bt_interior(BRX, nsub), TY = bt_interior(ry, nsub);
     const int ntx = (xcount + TX - 1) / TX, nty = (d.NJ + TY - 1) / TY;
     if (landp && nsub != land_nsub) {
       // stream order: the launches that read the previous flags are done
-      hipLaunchKernelGGL(k_bt_land, dim3(ntx * nty), dim3(256), 0, s, d, maskp, nsub, xbase,
+      hipLaunchKernelGGL(k_bt_land, dim3(ntx * nty), dim3(256), 0, s, d, w.mask, ry, nsub, xbase,
                          ntx, ntx * nty, landp);
       MOM_LAUNCHED(ctx, "k_bt_land");
       land_nsub = nsub;
     }
-    const BtJob J{d, in, eta_src, ud_src, eta_buf[which], ud_buf[which], eta_bar, ud, s0, nsub,
-                  p->nts, p->stepping_a, p->dtbt, c_pred, c_corr, xbase, xcount, ntx, ntx * nty,
-                  landp};
+    const BtJob J{d, in, eta_src, ud_src, s0 == 1 ? eb0 : w.eb, s0 == 1 ? nullptr : w.ub,
+                  w.eta[which], w.ud[which], w.eb, w.ub, s0, nsub, p->nts, p->stepping_a,
+                  p->dtbt, c_pred, c_corr, xbase, xcount, ntx, ntx * nty, which, landp};
     const int per_xcd = (ntx * nty + 7) / 8;
-    hipLaunchKernelGGL(k_bt_block, dim3(8 * per_xcd), dim3(BNT), 0, s, J, per_xcd);
+    bt_with_tile(plan.tile, [&](auto t) {
+      hipLaunchKernelGGL(k_bt_block<t.value>, dim3(8 * per_xcd), dim3(64 * bt_nw(t.value)), 0, s, J,
+                         per_xcd);
+    });
     MOM_LAUNCHED(ctx, "k_bt_block");
-    eta_src = eta_buf[which];
-    ud_src = ud_buf[which];
+    eta_src = w.eta[which];
+    ud_src = w.ud[which];
     which ^= 1;
   }
   const double nts = (double)p->nts;
   const double rntsp1 = 1.0 / (nts + 1.0);
   const double rnts = p->stepping_a ? 1.0 / nts : 2.0 / (nts * (double)(p->nts + 1));
-  hipLaunchKernelGGL(k_bt_scale, grid, block, 0, s, d, rntsp1, rnts, eta_bar, ud);
-  const dim3 wg((d.NJ + 255) / 256), wb(256);
-  if (d.cyclic_x) {
-    hipLaunchKernelGGL(k_bt_wrap, wg, wb, 0, s, d, eta_bar, 1);
-    hipLaunchKernelGGL(k_bt_wrap, wg, wb, 0, s, d, ud, 2);
-  }
-  if (conv) {
-    hipLaunchKernelGGL(k_bt_conv, grid, block, 0, s, d, ud, ctx->dxu, ctx->dyu, ctx->datr, conv);
-    if (d.cyclic_x) hipLaunchKernelGGL(k_bt_wrap, wg, wb, 0, s, d, conv, 1);
-  }
+  hipLaunchKernelGGL(k_bt_tail, grid, block, 0, s,
+                     BtTail{d, eb0, w.eb, w.ub, eta_bar, ud, conv, rntsp1, rnts, ctx->dxu, ctx->dyu,
+                            ctx->datr});
   MOM_LAUNCHED(ctx, "k_bt_tail");
   return MOM_GPU_OK;
 }
@@ -919,7 +1267,7 @@ int launch_barotropic(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p, const doub
   if (ctx->tune.bt_subcycles_per_launch > 0)
     return launch_barotropic_blocked(ctx, p, eta_t, eta_bar_tau, ud_tau, forcing, thicku, patm,
                                      pme, river, source, eta_smooth, rho_g, eta_bar, ud, conv,
-                                     ctx->tune.bt_subcycles_per_launch);
+                                     ctx->tune.bt_subcycles_set ? ctx->tune.bt_subcycles_per_launch : 0);
   const KDom &d = ctx->kd;
   const size_t P2 = (size_t)d.P2;
   BtBuf b;
@@ -972,36 +1320,51 @@ int launch_barotropic_ensemble(mom_gpu_ensemble *e, const mom_gpu_bt_params_t *p
                                const mom_gpu_bt_fields_t *f) {
   const int nd = (int)e->ctx.size();
   if (nd > BT_MAXDOM) return mom_fail(e->lead, MOM_GPU_ERR_ARG, "ensemble: too many domains");
-  const int hsub = e->lead->tune.bt_subcycles_per_launch > 0 ? e->lead->tune.bt_subcycles_per_launch
-                                                             : 4;
+  const auto &tune = e->lead->tune;
+  int hsub = !tune.bt_subcycles_set ? 0
+             : tune.bt_subcycles_per_launch > 0 ? tune.bt_subcycles_per_launch : 4;
   std::vector<BtDom> doms(nd);
   std::vector<BtTail> tails(nd);
+  std::vector<BtPrep> preps(nd);
   std::memset((void *)doms.data(), 0, sizeof(BtDom) * nd);
   std::memset((void *)tails.data(), 0, sizeof(BtTail) * nd);
+  std::memset((void *)preps.data(), 0, sizeof(BtPrep) * nd);
   int maxNI = 1, maxNJ = 1, nlaunch = 0;
+  bool rows = true;                 // every domain's rows are uniform
+  std::vector<const KDom *> kds(nd);
+  for (int k = 0; k < nd; ++k) {
+    rows = rows && e->ctx[k]->bt_rows_ok;
+    kds[k] = &e->ctx[k]->kd;
+  }
+  const BtPlan plan = bt_plan(kds.data(), nd, rows, hsub);
+  hsub = plan.hsub;
   for (int k = 0; k < nd; ++k) {
     mom_gpu_ctx *ctx = e->ctx[k];
     const KDom &d = ctx->kd;
-    const size_t P2 = (size_t)d.P2;
     const mom_gpu_bt_fields_t &x = f[k];
     const double rho0r = 1.0 / p[k].rho0;
+    const BtBufs w(ctx);
+    const double *eb0 = p[k].initsum_with_bar ? x.eta_t_bar_tau : x.eta_t_tau;
+    BtPrep &P = preps[k];
+    P.d = d;
+    P.pme = x.pme; P.river = x.river; P.source = x.source; P.eta_smooth = x.eta_smooth;
+    P.kmt = ctx->kmt; P.kmu = ctx->kmu; P.sf = w.sf; P.mask = w.mask;
+    P.datr = ctx->datr; P.dyu = ctx->dyu; P.dxu = ctx->dxu; P.dxur = ctx->dxur;
+    P.dyur = ctx->dyur; P.f = ctx->f; P.dtbt = p[k].dtbt;
+    P.rowc = rows ? w.rowc : nullptr;
     BtDom &D = doms[k];
     D.d = d;
-    double *sfp = ctx->bt + 6 * P2;
-    unsigned char *maskp = (unsigned char *)(ctx->bt + 7 * P2);
-    hipLaunchKernelGGL(k_bt_sfmask, dim3((d.NI + 255) / 256, d.NJ), dim3(256), 0,
-                       e->lead->stream, d, x.pme, x.river, x.source, x.eta_smooth, ctx->kmt,
-                       ctx->kmu, sfp, maskp, Inert{});
     D.in = BtIn{x.rho_g, x.patm, x.thicku, x.forcing_bt, ctx->f, ctx->dxu, ctx->dyu, ctx->datr,
-                ctx->dxur, ctx->dyur, sfp, maskp, ctx->bt_recip};
+                ctx->dxur, ctx->dyur, w.sf, w.mask, P.rowc, ctx->bt_recip};
     D.eta_bar_tau = x.eta_t_bar_tau;
     D.ud_tau = x.udrho_tau;
-    D.eta_buf[0] = ctx->bt;
-    D.eta_buf[1] = ctx->bt + P2;
-    D.ud_buf[0] = ctx->bt + 2 * P2;
-    D.ud_buf[1] = ctx->bt + 4 * P2;
-    D.eb = x.eta_t_bar_taup1;
-    D.ub = x.udrho_taup1;
+    D.eb0 = eb0;
+    D.eta_buf[0] = w.eta[0];
+    D.eta_buf[1] = w.eta[1];
+    D.ud_buf[0] = w.ud[0];
+    D.ud_buf[1] = w.ud[1];
+    D.eb = w.eb;
+    D.ub = w.ub;
     D.nts = p[k].nts;
     D.step_a = p[k].stepping_a;
     D.dtbt = p[k].dtbt;
@@ -1011,9 +1374,9 @@ int launch_barotropic_ensemble(mom_gpu_ensemble *e, const mom_gpu_bt_params_t *p
     D.xcount = d.cyclic_x ? d.ni : d.NI;
     BtTail &T = tails[k];
     T.d = d;
-    T.initsum = p[k].initsum_with_bar;
-    T.eta_t = x.eta_t_tau;
-    T.eta_bar_tau = x.eta_t_bar_tau;
+    T.eb0 = eb0;
+    T.eb = w.eb;
+    T.ub = w.ub;
     T.eta_bar = x.eta_t_bar_taup1;
     T.ud = x.udrho_taup1;
     T.conv = x.conv_rho_ud_t;
@@ -1027,36 +1390,45 @@ int launch_barotropic_ensemble(mom_gpu_ensemble *e, const mom_gpu_bt_params_t *p
     maxNJ = std::max(maxNJ, d.NJ);
     nlaunch = std::max(nlaunch, (p[k].nts + hsub - 1) / hsub);
   }
-  const BtDom *ddev = (const BtDom *)ens_table(e, doms.data(), sizeof(BtDom) * nd);
-  if (!ddev) return MOM_GPU_ERR_HIP;
-  const BtTail *tdev = (const BtTail *)ens_table(e, tails.data(), sizeof(BtTail) * nd);
-  if (!tdev) return MOM_GPU_ERR_HIP;
+  // one table: the domains, their preparations, their tails (each 16 B aligned)
+  const size_t a16 = 16, sd = (sizeof(BtDom) * nd + a16 - 1) / a16 * a16,
+               sp = (sizeof(BtPrep) * nd + a16 - 1) / a16 * a16;
+  std::vector<unsigned char> buf(sd + sp + sizeof(BtTail) * nd, 0);
+  std::memcpy(buf.data(), doms.data(), sizeof(BtDom) * nd);
+  std::memcpy(buf.data() + sd, preps.data(), sizeof(BtPrep) * nd);
+  std::memcpy(buf.data() + sd + sp, tails.data(), sizeof(BtTail) * nd);
+  const unsigned char *dev = (const unsigned char *)ens_table(e, buf.data(), buf.size());
+  if (!dev) return MOM_GPU_ERR_HIP;
+  const BtDom *ddev = (const BtDom *)dev;
+  const BtPrep *pdev = (const BtPrep *)(dev + sd);
+  const BtTail *tdev = (const BtTail *)(dev + sd + sp);
   hipStream_t s = e->lead->stream;
   const dim3 g2((maxNI + 255) / 256, maxNJ, nd), b2(256);
-  hipLaunchKernelGGL(k_bt_acc_init_ens, g2, b2, 0, s, tdev);
-  MOM_LAUNCHED(e->lead, "k_bt_acc_init_ens");
+  hipLaunchKernelGGL(k_bt_prep_ens, g2, b2, 0, s, pdev);
+  MOM_LAUNCHED(e->lead, "k_bt_prep_ens");
   for (int ell = 0; ell < nlaunch; ++ell) {
     BtLaunch L{};
     L.ndom = nd;
     L.ell = ell;
     L.hsub = hsub;
+    L.ry = bt_ry(plan.tile);
     int total = 0;
     for (int k = 0; k < nd; ++k) {
       int nsub, ntx, ntiles;
-      bt_shape(doms[k], ell, hsub, nsub, ntx, ntiles);
+      bt_shape(doms[k], L, nsub, ntx, ntiles);
       L.first[k] = total;
       total += ntiles;
     }
     L.first[nd] = total;
     if (total == 0) continue;
-    hipLaunchKernelGGL(k_bt_block_ens, dim3(total), dim3(BNT), 0, s, ddev, L);
+    const int per_xcd = (total + 7) / 8;
+    bt_with_tile(plan.tile, [&](auto t) {
+      hipLaunchKernelGGL(k_bt_block_ens<t.value>, dim3(8 * per_xcd), dim3(64 * bt_nw(t.value)), 0,
+                         s, ddev, L, per_xcd);
+    });
     MOM_LAUNCHED(e->lead, "k_bt_block_ens");
   }
-  hipLaunchKernelGGL(k_bt_scale_ens, g2, b2, 0, s, tdev);
-  const dim3 gw((maxNJ + 255) / 256, 1, nd);
-  hipLaunchKernelGGL(k_bt_wrap_ens, gw, b2, 0, s, tdev, 0);
-  hipLaunchKernelGGL(k_bt_conv_ens, g2, b2, 0, s, tdev);
-  hipLaunchKernelGGL(k_bt_wrap_ens, gw, b2, 0, s, tdev, 1);
+  hipLaunchKernelGGL(k_bt_tail_ens, g2, b2, 0, s, tdev);
   MOM_LAUNCHED(e->lead, "k_bt_tail_ens");
   return MOM_GPU_OK;
 }

@@ -284,6 +284,7 @@ struct BtvBlk {
   double *xd, *ud, *fd;                // state written
   const unsigned char *mask;           // bit 0 tmask(k=1), bit 1 umask(k=1)
   int s0, nsub, nts, step_a, ntx, ntiles;
+  int rev;                             // 1: the tiles in reverse order (see k_bt_block)
 };
 
 // sf and the masks, constant over the subcycles
@@ -301,7 +302,7 @@ __global__ void k_btv_sfmask(BtvArgs<CG, PR> a, unsigned char *__restrict__ mask
 template <bool CG, bool PR>
 __global__ __launch_bounds__(VX *VW) void k_btv_block(BtvArgs<CG, PR> a, BtvBlk J, int per_xcd) {
   const int b = blockIdx.x;
-  const int t0 = (b & 7) * per_xcd + (b >> 3);
+  const int t0 = (b & 7) * per_xcd + (J.rev ? per_xcd - 1 - (b >> 3) : b >> 3);
   if (t0 >= J.ntiles) return;                  // the whole block
   const int tile = strip_tile<8>(t0, J.ntx, J.ntiles / J.ntx);
   const KDom d = a.d;
@@ -600,6 +601,7 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
     J.xd = xb[which];
     J.ud = ub[which];
     J.fd = fb[which];
+    J.rev = which;
     const int per_xcd = (J.ntiles + 7) / 8;
     hipLaunchKernelGGL((k_btv_block<CG, PR>), dim3(8 * per_xcd), dim3(VX * VW), 0, s, a, J,
                        per_xcd);
@@ -609,6 +611,21 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
     J.fs = J.fd;
   }
   return MOM_GPU_OK;
+}
+
+// Subcycles a launch: as set, otherwise the most (at most 12) with at most 128
+// regions, when a launch's time is its latency (90 x 60, 80 subcycles: 296 us at
+// 5, 205 at 12), and 6 above (517 x 389: 331 at 5, 320 at 6, 292 at 7, 433 at 8;
+// 1440 x 1080: 2475, 2257, 2420, 2445).  Results do not depend on it.
+int blocked_depth(const mom_gpu_ctx *ctx) {
+  if (ctx->tune.bt_subcycles_set) return ctx->tune.bt_subcycles_per_launch;
+  const KDom &d = ctx->kd;
+  int h = 12;
+  for (; h > 6; --h) {
+    const int TX = btv_tx(h, d.cyclic_x != 0), TY = btv_ty(h);
+    if (((d.NI + TX - 1) / TX) * ((d.NJ + TY - 1) / TY) <= 128) break;
+  }
+  return h;
 }
 
 // Tail (:2846-2894): the time means, each halo-updated, and
@@ -705,7 +722,7 @@ int run_variant(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p, const mom_gpu_bt
   a.initsum = p->initsum_with_bar ? 1 : 0;
   hipStream_t s = ctx->stream;
   const dim3 grid((d.NI + 63) / 64, d.NJ), block(64);
-  const int nts = p->nts, hsub = ctx->tune.bt_subcycles_per_launch;
+  const int nts = p->nts, hsub = blocked_depth(ctx);
   if (hsub > 0 && !d.cyclic_y && (!d.cyclic_x || d.ni >= MIN_NI)) {
     const int rc = run_blocked(ctx, a, nts, p->stepping_a, hsub);
     if (rc) return rc;

@@ -167,6 +167,7 @@ int mom_gpu_set_tuning(mom_gpu_ctx_t *ctx, const char *knob, int value) {
                    value == 5 || value == 6 || value == 8 || value == 10,
           "mom_gpu_set_tuning: step_group_f32 must be 1, 2, 4, 5, 6, 8 or 10");
   *slot = value;
+  if (slot == &ctx->tune.bt_subcycles_per_launch) ctx->tune.bt_subcycles_set = 1;
   return MOM_GPU_OK;
 }
 
@@ -349,6 +350,7 @@ int mom_gpu_create(const mom_gpu_domain_t *dom, const mom_gpu_grid_t *grid, mom_
   k.cyclic_x = dom->cyclic_x ? 1 : 0;
   k.cyclic_y = dom->cyclic_y ? 1 : 0;
   c->tune.bt_subcycles_per_launch = 5;
+  c->tune.bt_subcycles_set = 0;
   c->tune.mdfl_rows_per_wave = 1;
   c->tune.step_group_f64 = 2;
   c->tune.step_group_f32 = 10;
@@ -400,7 +402,7 @@ int mom_gpu_create(const mom_gpu_domain_t *dom, const mom_gpu_grid_t *grid, mom_
   CK(hipMemcpyAsync(c->dzt, grid->dzt, nk * sizeof(double), hipMemcpyDefault, c->stream));
   CK(hipMalloc(&c->qw, 16 * P2 * sizeof(double)));
   CK(hipMalloc(&c->qzw, 8 * nk * sizeof(double)));
-  CK(hipMalloc(&c->bt, 9 * P2 * sizeof(double)));
+  CK(hipMalloc(&c->bt, 12 * P2 * sizeof(double)));
   CK(hipMalloc(&c->tri_e, P2 * nk * sizeof(double)));
   c->red_n = 1024;
   CK(hipMalloc(&c->red, (8 * (size_t)c->red_n + 8) * sizeof(double)));

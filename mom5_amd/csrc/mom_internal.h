@@ -173,7 +173,9 @@ struct mom_gpu_ctx {
   // the grid metrics the blocked barotropic multiplies are bounded by 1e100
   // and dxu, dyu, datr carry no sign bit: the condition its land path needs
   int bt_grid_ok;
-  double bt_cori_dtbt;
+  // dxu, dyu, datr, dxur, dyur and f are the same along every row, bit for bit
+  // (spherical grids): the blocked barotropic takes them from the row
+  int bt_rows_ok;
   // REMAP_BT_TO_BU metrics dte, dtw, dus, dun, daur (5 planes, optional)
   double *remap;
   // state of the barotropic variants (22 planes, allocated on first use)
@@ -191,6 +193,7 @@ struct mom_gpu_ctx {
   // launch-shape knobs (mom_gpu_set_tuning)
   struct {
     int bt_subcycles_per_launch;   // 0: one launch per phase per subcycle
+    int bt_subcycles_set;          // 1 once mom_gpu_set_tuning gave it; else chosen per call
     int mdfl_rows_per_wave;        // 2 or 4 region rows per wavefront
     int step_group_f64;            // FP64 tracers per pass of the batched step (1, 2)
     int step_group_f32;            // FP32 tracers per pass (1, 2, 4)

@@ -316,6 +316,60 @@ def test_blocked_barotropic_grid_reciprocals(oracle_lib, exact):
     gpu.close()
 
 
+@pytest.mark.parametrize("ni,nj,cyclic,depths", [
+    (17, 5, True, (None, 2, 11, 12)), (70, 23, False, (None, 5, 10)),
+    (131, 47, True, (None, 7, 10, 11)), (400, 300, False, (None, 7, 8, 12)),
+    (1400, 1340, True, (None, 5))])
+@pytest.mark.parametrize("special", [False, True])
+def test_blocked_barotropic_uniform_rows(ni, nj, cyclic, depths, special):
+    """On a grid whose metrics do not change along a row the blocked
+    barotropic takes them from the row (tiles of 64 x 24 or 64 x 32, chosen
+    from the size and the subcycles a launch, which are chosen too until set):
+    every tile, depth and edge gives the result of the launch-per-phase path
+    (depth 0), bit for bit, also with a NaN and an infinity at a few points of
+    the first and last rows and the interior; and a grid that differs
+    at one point, which takes the general tile, too."""
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    print(f"[uniform rows {ni}x{nj} cyclic={cyclic} special={special}]", flush=True)
+    case = make_case(ni, nj, 2, land_frac=0.3, nts=14, seed=5, pme_scale=1e-4, cyclic_x=cyclic)
+    mid = case.grid["dxu"].shape[1] // 2
+    for key in ("dxu", "dyu", "dxur", "dyur", "datr", "f"):
+        case.grid[key] = np.repeat(case.grid[key][:, mid:mid + 1], case.grid[key].shape[1], axis=1)
+    if special:
+        e = case.fields["eta_t_bar"]
+        e[0, 3] = e[-1, 5] = np.nan
+        case.fields["udrho"][0, nj // 2, ni // 2] = np.inf
+        case.fields["forcing_bt"][1, 1, 2] = -0.0
+    shp = case.grid["dxu"].shape
+    f = {k: DeviceArray.from_host(v) for k, v in case.fields.items() if isinstance(v, np.ndarray)}
+    for uniform in (True, False):
+        if not uniform:
+            case.grid["f"] = case.grid["f"].copy()
+            case.grid["f"][1, 2] *= 1.0 + 2.0 ** -30
+        ref = None
+        for h in (0,) + depths:
+            gpu = OceanGPU(case.dom, case.grid)
+            if h is not None:
+                gpu.set_tuning("barotropic_subcycles_per_launch", h)
+            out = DeviceArray(shp), DeviceArray((2,) + shp), DeviceArray(shp)
+            gpu.update_ocean_barotropic(
+                nts=case.nts, dtbt=case.dtbt, eta_t_tau=f["eta_t"], eta_t_bar_tau=f["eta_t_bar"],
+                udrho_tau=f["udrho"], forcing_bt=f["forcing_bt"], thicku=f["thicku"],
+                patm=f["patm"], pme=f["pme"], river=f["river"], source=f["source"],
+                eta_smooth=f["eta_smooth"], rho_g=f["rho_g"], eta_t_bar_taup1=out[0],
+                udrho_taup1=out[1], conv_rho_ud_t=out[2], stepping_a=special)
+            gpu.sync()
+            got = [a.to_host() for a in out]
+            gpu.close()
+            for a in got:
+                if cyclic:      # no blocked subcycle reaches the halo corners
+                    a[..., 0, ::shp[1] - 1] = a[..., -1, ::shp[1] - 1] = 0.0
+            ref = ref or got
+            for a, b in zip(got, ref):
+                np.testing.assert_array_equal(a, b)
+
+
 def _land_tiles(case, nsub, cyclic=True):
     """Tiles of the blocked barotropic (64x32 regions, nsub subcycles) whose
     every point is inert: both masks 0, forcing and velocity zeros."""
