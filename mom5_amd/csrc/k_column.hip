@@ -105,6 +105,7 @@ struct VdJob {
   // and dcbase2 unused)
   const double *dcbase2;
   int n2;
+  const double *k33[NT];   // k_vdiff_twin64 with KK: each tracer's K33
 };
 
 template <typename TT>
@@ -961,22 +962,35 @@ __global__ __launch_bounds__(64) void k_vdiff_inc_ens(const VdJobF *__restrict__
   if (J) vdiff_inc_col<NTF_ENS, false>(*J, gi, gj);
 }
 
-// Ensemble, register-resident FP32 solver: every group of every domain in one
-// launch (no scratch is shared); tiles in XCD-aware order over the whole
-// table, H the largest slot count the domains need.
-template <int H>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
-void k_vdiff_twin_ens(const VdJobF *__restrict__ jobs, VdLaunch L, int per_xcd) {
+// The job lo of a block of two tiles and this wavefront pair's tile of it; L counts
+// tile pairs, so that a block never holds two jobs (their barriers differ) and the
+// cache lines that two neighbouring tiles share are written together.  False:
+// past the end, the whole block.
+__device__ inline bool vd_pair(const VdLaunch &L, int per_xcd, int &lo, int &tile) {
   const int b = blockIdx.x;
   const int t = (b & 7) * per_xcd + (b >> 3);
-  if (t >= L.first[L.njobs]) return;         // the whole block
-  int lo = 0, hi = L.njobs - 1;
+  if (t >= L.first[L.njobs]) return false;
+  lo = 0;
+  int hi = L.njobs - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (L.first[mid] <= t) lo = mid; else hi = mid - 1;
   }
   lo = __builtin_amdgcn_readfirstlane(lo);
-  twin_tile<H>(jobs[lo], t - L.first[lo]);
+  tile = 2 * (t - L.first[lo]) + (threadIdx.x >> 7);
+  return true;
+}
+
+// Ensemble, register-resident FP32 solver: every group of every domain in one
+// launch (no scratch is shared); tiles in XCD-aware order over the whole
+// table, H the largest slot count the domains need.
+template <int H>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void k_vdiff_twin_ens(const VdJobF *__restrict__ jobs, VdLaunch L, int per_xcd) {
+  int lo, tile;
+  if (!vd_pair(L, per_xcd, lo, tile)) return;
+  const VdJobF &J = jobs[lo];
+  twin_tile<H, 2>(J, min(tile, J.nblocks - 1), tile < J.nblocks);
 }
 
 // ---- FP64 tracers, every level of a column in registers ---------------------
@@ -1000,9 +1014,13 @@ void k_vdiff_twin_ens(const VdJobF *__restrict__ jobs, VdLaunch L, int per_xcd) 
 // its level count), so both meet in slot H-1; slots below ph are inert.  A
 // group's tracers share the coefficients' addresses, not their factorisation:
 // each tracer repeats it (the coefficients come from L2 the second time).
+// KK: every tracer of the job has its own K33 (J.k33), loaded with its
+// coefficients; with rho_dzt and dzwt from L2 after the first tracer and K33 a chunk
+// ahead, three tracers with K33 at 1440x1080x50 take 1.83 ms (one job each, K33
+// read where it is used: 2.55; 13 planes, 8.1 GB: 4.4 TB/s).
 // Wavefront pair threadIdx.x / 128 of a block of NP pairs; a pair whose
 // tile is past the end (live false) runs a valid tile without storing.
-template <int H, int NP = 1>
+template <int H, int NP, bool KK>
 __device__ __forceinline__ void twin64_tile(const VdJob<double> &J, int tile, bool live = true) {
   __shared__ double xv_all[NP][2][2][64], xq_all[NP][2][2][64];   // [pair][parity][half][column]
   const int pr = NP > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 7) : 0;
@@ -1027,15 +1045,10 @@ __device__ __forceinline__ void twin64_tile(const VdJob<double> &J, int tile, bo
   const int kb = max(2, kmo);
   const double tda = J.tdt * J.aidif;
   const double rho0 = J.rho0;
-  const double *k33 = J.g.k33;
   for (int n = 0; n < J.g.n; ++n) {
     // the tracer's diffusivity plane: its mixing class's diff_cbt
     const double *dcbase = (J.dcbase2 && n >= J.n2) ? J.dcbase2 : J.dcbase;
-    // dcb = rho0*diff_cbt(nmix) + K33 of the plane at offset pl (vdiff_col's
-    // expression)
-    auto dcb_at = [&](long pl) {
-      return rho0 * ld_at(dcbase + pl, ob8) + (k33 ? ld_at(k33 + pl, ob8) : 0.0);
-    };
+    const double *k33 = J.k33[n];
     double *z = J.g.z[n];
     const double stf = ld_at(J.g.stf[n], ob8), btf = ld_at(J.g.btf[n], ob8);
     double vs[H], qs[H];
@@ -1062,7 +1075,7 @@ __device__ __forceinline__ void twin64_tile(const VdJob<double> &J, int tile, bo
     // interface and plane loaded before the loop.  Inert slots load slot ph's.
     constexpr int CH = 4, NCH = (H + CH - 1) / CH;
     const long dwo = top ? P2 : 0, dco = top ? 0 : -P2;
-    double Ldh[NCH * CH], Ldw[NCH * CH], Ldc[NCH * CH];
+    double Ldh[NCH * CH], Ldw[NCH * CH], Ldc[NCH * CH], Ldk[KK ? NCH * CH : 1];
     auto cload = [&](int c) {
 #pragma unroll
       for (int u = 0; u < CH; ++u) {
@@ -1075,12 +1088,18 @@ __device__ __forceinline__ void twin64_tile(const VdJob<double> &J, int tile, bo
         Ldh[j] = ld_at(J.dh + plj, ob8);
         Ldw[j] = ld_at(J.dhw + plj + dwo, ob8);
         Ldc[j] = ld_at(dcbase + plj + dco, ob8);
+        if constexpr (KK) Ldk[j] = ld_at(k33 + plj + dco, ob8);
       }
     };
     // the first slot's other interface and plane (top: dzwt(0) and none; the
     // bottom: dzwt(nk) and diff_cbt(nk))
     const double dhw_first = ld_at(J.dhw + p0 + (top ? 0 : P2), ob8);
-    const double dcb_first = top ? 0.0 : dcb_at(p0);
+    // dcb = rho0*diff_cbt(nmix) + K33 (vdiff_col's expression)
+    double dcb_first = 0.0;
+    if (!top) {
+      dcb_first = rho0 * ld_at(dcbase + p0, ob8) + 0.0;
+      if constexpr (KK) dcb_first = rho0 * ld_at(dcbase + p0, ob8) + ld_at(k33 + p0, ob8);
+    }
     double bet = 0.0, qprev = 0.0, vprev = 0.0;
     double dcb_c = 0.0, dhw_c = 0.0;   // the interface shared with the next slot
     pl = p0;
@@ -1102,9 +1121,8 @@ __device__ __forceinline__ void twin64_tile(const VdJob<double> &J, int tile, bo
         const int r = j - phj;
         const int k = top ? r + 1 : nk - r;     // pl = P2*(k - 1)
         const double dhk = Ldh[j];
-        // the slot's diff_cbt plane: rho0*diff_cbt (+ K33, read here when a
-        // tracer has its own)
-        const double dcb_new = J.rho0 * Ldc[j] + (k33 ? ld_at(k33 + pl + dco, ob8) : 0.0);
+        double dcb_new;
+        if constexpr (KK) dcb_new = rho0 * Ldc[j] + Ldk[j]; else dcb_new = rho0 * Ldc[j] + 0.0;
         // dzwt plane k-1 is the interface above level k, plane k the one below
         double dcb_km1, dcb_k, dhw_km1, dhw_k;
         if (top) {
@@ -1185,14 +1203,14 @@ __device__ __forceinline__ void twin64_tile(const VdJob<double> &J, int tile, bo
 
 // Two neighbouring tiles a block (per_xcd counts tile pairs), as for the
 // FP32 solver: the halves of the cache lines they share are written together.
-template <int H>
+template <int H, bool KK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_vdiff_twin64(VdJob<double> J, int per_xcd) {
   const int b = blockIdx.x;
   const int t0 = 2 * ((b & 7) * per_xcd + (b >> 3));
   if (t0 >= J.nblocks) return;               // the whole block
   const int tile = t0 + (threadIdx.x >> 7);
-  twin64_tile<H, 2>(J, min(tile, J.nblocks - 1), tile < J.nblocks);
+  twin64_tile<H, 2, KK>(J, min(tile, J.nblocks - 1), tile < J.nblocks);
 }
 
 // Several FP64 tracers of one mixing class: k_vdiff_twin64's elimination with the
@@ -1407,18 +1425,12 @@ void k_vdiff_share(ShareJob J, int per_xcd) {
 // Ensemble: every FP64 group of every domain whose nk the register solver
 // takes, in one launch; tiles in XCD-aware order over the whole table.
 template <int H>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_vdiff_twin64_ens(const VdJob<double> *__restrict__ jobs, VdLaunch L, int per_xcd) {
-  const int b = blockIdx.x;
-  const int t = (b & 7) * per_xcd + (b >> 3);
-  if (t >= L.first[L.njobs]) return;         // the whole block
-  int lo = 0, hi = L.njobs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (L.first[mid] <= t) lo = mid; else hi = mid - 1;
-  }
-  lo = __builtin_amdgcn_readfirstlane(lo);
-  twin64_tile<H>(jobs[lo], t - L.first[lo]);
+  int lo, tile;
+  if (!vd_pair(L, per_xcd, lo, tile)) return;
+  const VdJob<double> &J = jobs[lo];
+  twin64_tile<H, 2, false>(J, min(tile, J.nblocks - 1), tile < J.nblocks);
 }
 
 __global__ void k_set_ints(int *__restrict__ p, int v, int n) {
@@ -1696,7 +1708,7 @@ int launch_invtri(mom_gpu_ctx *ctx, double *z, const double *topbc, const double
 }
 
 static int twin_slots(int nk);
-static void launch_twin64(mom_gpu_ctx *ctx, VdJob<double> J);
+static void launch_twin64(mom_gpu_ctx *ctx, VdJob<double> J, bool kk);
 static void launch_share(mom_gpu_ctx *ctx, const ShareJob &J);
 
 // FP64 tracers take the register-resident solver (k_vdiff_twin64) whenever nk
@@ -1704,7 +1716,8 @@ static void launch_share(mom_gpu_ctx *ctx, const ShareJob &J);
 // depend on them; the Thomas kernels (k_vdiff1, k_vdiff) serve other nk.
 // Jobs of up to NT tracers hold both mixing classes (class 1 first, n2 the
 // first of class 2), so that T and S share one launch and the tile's rho_dzt
-// and dzwt come from L2 for the second; a tracer with its own K33 goes alone.
+// and dzwt come from L2 for the second; tracers with their own K33 make such jobs
+// of their own.
 static int twin64_groups(mom_gpu_ctx *ctx, int ntr, void *const *T, const int *dtype, int want,
                          const double *const *stf, const double *const *btf,
                          const double *diff_cbt, const double *const *K33, int index_salt,
@@ -1720,25 +1733,16 @@ static int twin64_groups(mom_gpu_ctx *ctx, int ntr, void *const *T, const int *d
     J.nbx = nbx; J.nblocks = nbx * d.nj;
     return J;
   };
-  std::vector<int> c1, c2;
+  // by mixing class: [0] without, [1] with K33
+  std::vector<int> by[2][2];
   for (int n = 0; n < ntr; ++n) {
     if ((dtype ? dtype[n] : 8) != want) continue;
-    const int nm = (n == index_salt) ? 2 : 1;
-    const double *k33 = (K33 && K33[n]) ? K33[n] : nullptr;
-    if (k33) {
-      VdJob<double> J = job();
-      J.g.z[0] = (double *)T[n]; J.g.stf[0] = stf[n]; J.g.btf[0] = btf[n]; J.g.n = 1;
-      J.g.k33 = k33;
-      J.n2 = (nm == 2) ? 0 : 1;
-      launch_twin64(ctx, J);
-      MOM_LAUNCHED(ctx, "k_vdiff_twin64");
-      continue;
-    }
-    (nm == 1 ? c1 : c2).push_back(n);
+    by[K33 && K33[n] ? 1 : 0][n == index_salt ? 1 : 0].push_back(n);
   }
+  const std::vector<int> &c1 = by[0][0];
   const int n1 = (int)c1.size();
   std::vector<int> all(c1);
-  all.insert(all.end(), c2.begin(), c2.end());
+  all.insert(all.end(), by[0][1].begin(), by[0][1].end());
   // Three tracers of class 1 or more share its factorisation (class 2 is salt
   // alone).  With two the one factorisation saved is what fewer wavefronts in
   // flight cost: T, S and one more tracer at 1440x1080, 41 levels 1.49 ms with
@@ -1759,21 +1763,28 @@ static int twin64_groups(mom_gpu_ctx *ctx, int ntr, void *const *T, const int *d
       launch_share(ctx, J);
       MOM_LAUNCHED(ctx, "k_vdiff_share");
     }
-    return MOM_GPU_OK;
+    all.clear();
   }
-  for (size_t at = 0; at < all.size(); at += NT) {
-    const int cnt = (int)std::min((size_t)NT, all.size() - at);
-    VdJob<double> J = job();
-    for (int q = 0; q < cnt; ++q) {
-      const int n = all[at + q];
-      J.g.z[q] = (double *)T[n]; J.g.stf[q] = stf[n]; J.g.btf[q] = btf[n];
+  auto twin = [&](const std::vector<int> &ns, int n1, bool kk) {
+    for (size_t at = 0; at < ns.size(); at += NT) {
+      const int cnt = (int)std::min((size_t)NT, ns.size() - at);
+      VdJob<double> J = job();
+      for (int q = 0; q < cnt; ++q) {
+        const int n = ns[at + q];
+        J.g.z[q] = (double *)T[n]; J.g.stf[q] = stf[n]; J.g.btf[q] = btf[n];
+        if (kk) J.k33[q] = K33[n];
+      }
+      J.g.n = cnt;
+      J.n2 = std::max(0, std::min(cnt, n1 - (int)at));
+      launch_twin64(ctx, J, kk);
+      MOM_LAUNCHED(ctx, "k_vdiff_twin64");
     }
-    J.g.n = cnt;
-    J.n2 = std::max(0, std::min(cnt, n1 - (int)at));
-    launch_twin64(ctx, J);
-    MOM_LAUNCHED(ctx, "k_vdiff_twin64");
-  }
-  return MOM_GPU_OK;
+    return MOM_GPU_OK;
+  };
+  std::vector<int> own(by[1][0]);
+  own.insert(own.end(), by[1][1].begin(), by[1][1].end());
+  const int rc = twin(all, n1, false);
+  return rc ? rc : twin(own, (int)by[1][0].size(), true);
 }
 
 template <typename TT>
@@ -1956,7 +1967,7 @@ static int twin_slots(int nk) {
 
 // f(integral constant) for a count of slots that twin_slots returns.  Fine
 // steps: an unused slot costs its registers, and FP32 columns its arithmetic (T, S
-// at 1440x1080x50 in 26 slots instead of 32: SLOTNUM)
+// at 1440x1080x50 in 26 slots instead of 32: 1342 us, now 1255)
 template <typename F>
 static void with_slots(int h, F &&f) {
   switch (h) {
@@ -1974,12 +1985,15 @@ static void with_slots(int h, F &&f) {
   }
 }
 
-static void launch_twin64(mom_gpu_ctx *ctx, VdJob<double> J) {
+static void launch_twin64(mom_gpu_ctx *ctx, VdJob<double> J, bool kk) {
   const KDom &d = J.d;
   const int per_xcd = ((J.nblocks + 1) / 2 + 7) / 8;   // tile pairs per XCD
   const dim3 grid(8 * per_xcd), block(256);
   with_slots(twin_slots(d.nk), [&](auto H) {
-    hipLaunchKernelGGL(k_vdiff_twin64<H.value>, grid, block, 0, ctx->stream, J, per_xcd);
+    if (kk)
+      hipLaunchKernelGGL((k_vdiff_twin64<H.value, true>), grid, block, 0, ctx->stream, J, per_xcd);
+    else
+      hipLaunchKernelGGL((k_vdiff_twin64<H.value, false>), grid, block, 0, ctx->stream, J, per_xcd);
   });
 }
 
@@ -2234,6 +2248,29 @@ int launch_vdiff_ensemble(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *step
                                    "ensemble");
       if (rc) return rc;
     }
+    // FP64 tracers of both mixing classes in one job where the register solver
+    // takes them (as in twin64_groups)
+    const bool both = twin_slots(d.nk) > 0;
+    std::vector<int> cls;
+    for (int n = 0; both && n < s.ntr; ++n)
+      if (s.dtype[n] == 8 && n != s.index_salt) cls.push_back(n);
+    const int n1 = (int)cls.size();
+    if (both && s.index_salt >= 0 && s.index_salt < s.ntr && s.dtype[s.index_salt] == 8)
+      cls.push_back(s.index_salt);
+    for (size_t at = 0; at < cls.size(); at += NT) {
+      VdJob<double> J;
+      std::memset((void *)&J, 0, sizeof J);
+      J.g.n = (int)std::min((size_t)NT, cls.size() - at);
+      for (int q = 0; q < J.g.n; ++q) {
+        const int n = cls[at + q];
+        J.g.z[q] = (double *)s.T_taup1[n]; J.g.stf[q] = s.stf[n]; J.g.btf[q] = s.btf[n];
+      }
+      J.n2 = std::max(0, std::min(J.g.n, n1 - (int)at));
+      J.d = d; J.dcbase = s.diff_cbt; J.dcbase2 = s.diff_cbt + p3; J.rho0 = s.rho0;
+      J.kmt = ctx->kmt; J.dh = dh; J.dhw = s.dzwt; J.tdt = s.dtime; J.aidif = s.aidif;
+      J.ework = ctx->tri_e; J.nbx = nbx; J.nblocks = nbx * d.nj;
+      g64[dd].push_back(J);
+    }
     for (int nmix = 1; nmix <= 2; ++nmix) {
       const double *dcb = s.diff_cbt + p3 * (nmix - 1);
       VdJob<double> j64;
@@ -2259,6 +2296,7 @@ int launch_vdiff_ensemble(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *step
       for (int n = 0; n < s.ntr; ++n) {
         if (((n == s.index_salt) ? 2 : 1) != nmix) continue;
         if (s.dtype[n] == 8) {
+          if (both) continue;
           TriGroup<double> &g = j64.g;
           g.z[g.n] = (double *)s.T_taup1[n]; g.stf[g.n] = s.stf[n]; g.btf[g.n] = s.btf[n];
           if (++g.n == NT) flush64();
@@ -2291,14 +2329,14 @@ int launch_vdiff_ensemble(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *step
       int total = 0;
       for (size_t j = 0; j < nj; ++j) {
         L.first[j] = total;
-        total += all64[at + j].nblocks;
+        total += (all64[at + j].nblocks + 1) / 2;
       }
       L.first[nj] = total;
       L.njobs = (int)nj;
       const void *dev = ens_table(e, all64.data() + at, sizeof(VdJob<double>) * nj);
       if (!dev) return MOM_GPU_ERR_HIP;
       const int per_xcd = (total + 7) / 8;
-      const dim3 grid(8 * per_xcd), block(128);
+      const dim3 grid(8 * per_xcd), block(256);
       hipStream_t st = e->lead->stream;
       const VdJob<double> *jt = (const VdJob<double> *)dev;
       with_slots(h64, [&](auto H) {
@@ -2319,14 +2357,14 @@ int launch_vdiff_ensemble(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *step
     int total = 0;
     for (size_t j = 0; j < nj; ++j) {
       L.first[j] = total;
-      total += all[at + j].nblocks;
+      total += (all[at + j].nblocks + 1) / 2;
     }
     L.first[nj] = total;
     L.njobs = (int)nj;
     const void *dev = ens_table(e, all.data() + at, sizeof(VdJobF) * nj);
     if (!dev) return MOM_GPU_ERR_HIP;
     const int per_xcd = (total + 7) / 8;
-    const dim3 grid(8 * per_xcd), block(128);
+    const dim3 grid(8 * per_xcd), block(256);
     hipStream_t st = e->lead->stream;
     with_slots(hmax, [&](auto H) {
       hipLaunchKernelGGL(k_vdiff_twin_ens<H.value>, grid, block, 0, st, (const VdJobF *)dev, L, per_xcd);

@@ -246,6 +246,43 @@ def test_vert_diffuse_implicit(setup):
                            what=f"tracer {n}")
 
 
+@pytest.mark.parametrize("nk", [2, 41, 80])
+def test_vert_diffuse_implicit_own_k33(nk):
+    """Tracers with a K33 of their own share jobs (eight a job, both mixing
+    classes): each equals, bit for bit, the tracer solved alone, and with its
+    mixing coefficient passed as K33 the tracer solved without one."""
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    case = make_case(67, 9, nk, land_frac=0.3, seed=nk, stf_scale=1e-3)
+    gpu, f = OceanGPU(case.dom, case.grid), case.fields
+    H, rng = DeviceArray.from_host, np.random.default_rng(nk)
+    base = case.tracers[0][1]
+    shp, ntr, rho0 = base.shape, 11, 1035.0
+    Ts = [base * (1.0 + 0.01 * n) for n in range(ntr)]
+    K = [None if n in (2, 5) else 1e-2 * rng.random(shp) for n in range(ntr)]
+    stf = [f["stf"][n % 2] for n in range(ntr)]
+    rho, dzwt, mix = H(f["rho_dzt"]), H(f["dzwt"]), H(f["diff_cbt"])
+
+    def run(ns, salt, kk, mixing):
+        d = [H(Ts[n]) for n in ns]
+        gpu.vert_diffuse_implicit(d, [H(stf[n]) for n in ns], [H(stf[n]) for n in ns], mixing,
+                                  rho, dzwt, case.dt, index_salt=salt, rho0=rho0,
+                                  K33s=[None if kk[n] is None else H(kk[n]) for n in ns])
+        gpu.sync()
+        return [x.to_host() for x in d]
+
+    print(f"[own K33, nk {nk}]", flush=True)
+    got = run(range(ntr), 1, K, mix)
+    for n in range(ntr):
+        same(got[n], run([n], 0 if n == 1 else -1, K, mix)[0])
+    as_k33 = [rho0 * f["diff_cbt"][1 if n == 1 else 0] for n in range(ntr)]
+    a = run(range(ntr), 1, as_k33, H(np.zeros_like(f["diff_cbt"])))
+    b = run(range(ntr), 1, [None] * ntr, mix)
+    for x, y in zip(a, b):
+        same(x, y)
+    gpu.close()
+
+
 @pytest.mark.parametrize("per_launch", [0, 1, 4, 7, 12])
 @pytest.mark.parametrize("stepping_a,initsum", [(False, True), (True, False)])
 def test_update_ocean_barotropic(setup, stepping_a, initsum, per_launch):
