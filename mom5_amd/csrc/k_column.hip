@@ -1447,41 +1447,54 @@ struct LimTable {
   int n;
 };
 
-__global__ void k_tmask_limit(KDom d, LimTable t, int it, int is, int ts_same,
-                              const int *__restrict__ kmt) {
-  // 64 x 4 points of one level a work-group
-  const int ii = blockIdx.x * 64 + threadIdx.x;   // gi = ii - 1
-  const int gj = blockIdx.y * 4 + threadIdx.y - 1;
-  const int k = blockIdx.z + 1;
-  const int gi = ii - 1;
+// A thread takes LIM_NK levels of one point, tracer after tracer, with the level
+// below carried from one level to the next and a level's loads issued before
+// the level above is written: HBM reads each tracer once (a thread per point
+// and level read it again for the level above).  Three tracers at 1440x1080x50:
+// 1.09 to 0.95 ms (six planes, 3.9 TB/s; two levels ahead 1.00).
+constexpr int LIM_NK = 10;
+__global__ __launch_bounds__(256) void k_tmask_limit(KDom d, LimTable t, int it, int is,
+                                                     int ts_same, const int *__restrict__ kmt,
+                                                     int ntx, int ntiles, int per_xcd) {
+  // 64 x 4 points a work-group, neighbouring tiles on one XCD
+  const int b = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (b >= ntiles) return;
+  const int tile = strip_tile<8>(b, ntx, ntiles / ntx);
+  const int gi = (tile % ntx) * 64 + threadIdx.x - 1;
+  const int gj = (tile / ntx) * 4 + threadIdx.y - 1;
   if (gi > d.ni - 1 || gj > d.nj - 1) return;
-  const int o = d2(d, gi, gj), P2 = d.P2, ok = o + P2 * (k - 1);
-  const double m0 = (k <= kmt[o]) ? 1.0 : 0.0;
-  const double me = (k <= kmt[o + 1]) ? 1.0 : 0.0;
-  const double mn_ = (k <= kmt[o + d.NI]) ? 1.0 : 0.0;
-  const double mb = (k < d.nk && k + 1 <= kmt[o]) ? 1.0 : 0.0;
-  double flagT = 0.0, flagS = 0.0;
+  const int k1 = blockIdx.y * LIM_NK + 1, k2 = min(k1 + LIM_NK - 1, d.nk);
+  const int o = d2(d, gi, gj);
+  const size_t P2 = (size_t)d.P2;
+  const int km = kmt[o], ke = kmt[o + 1], kn = kmt[o + d.NI];
+  unsigned flagT = 0, flagS = 0;                  // bit k - k1
   for (int n = 0; n < t.n; ++n) {
-    const double *T = t.T[n];
+    const double *T = t.T[n] + o;
+    double *lim = t.lim[n] + o;
     const double lo = t.mn[n], hi = t.mx[n];
-    double L = 0.0;
-    double x = T[ok];
-    if (m0 == 1.0 && (x < lo || x > hi)) L = m0;
-    x = T[ok + 1];
-    if (me == 1.0 && (x < lo || x > hi)) L = m0;
-    x = T[ok + d.NI];
-    if (mn_ == 1.0 && (x < lo || x > hi)) L = m0;
-    if (k < d.nk) {
-      x = T[ok + P2];
-      if (mb == 1.0 && (x < lo || x > hi)) L = m0;
+    auto out = [&](double x) { return x < lo || x > hi; };
+    size_t pk = P2 * (k1 - 1);
+    double xc = T[pk], xe = T[pk + 1], xn = T[pk + d.NI];
+    unsigned flags = 0;
+    for (int k = k1; k <= k2; ++k) {
+      const size_t pn = P2 * min(k, d.nk - 1);    // the level below (the last: itself)
+      const double yc = T[pn], ye = T[pn + 1], yn = T[pn + d.NI];
+      const bool far = k <= km && (out(xc) || (k <= ke && out(xe)) || (k <= kn && out(xn)) ||
+                                   (k < d.nk && k + 1 <= km && out(yc)));
+      flags |= (far ? 1u : 0u) << (k - k1);
+      lim[pk] = far ? 1.0 : 0.0;
+      pk = pn;
+      xc = yc; xe = ye; xn = yn;
     }
-    if (n == it) flagT = L;
-    if (n == is) flagS = L;
-    t.lim[n][ok] = L;
+    if (n == it) flagT = flags;
+    if (n == is) flagS = flags;
   }
-  if (ts_same && it >= 0 && is >= 0 && (flagT == 1.0 || flagS == 1.0)) {
-    t.lim[it][ok] = 1.0;
-    t.lim[is][ok] = 1.0;
+  if (ts_same && it >= 0 && is >= 0) {
+    for (unsigned both = flagT | flagS; both; both &= both - 1) {
+      const size_t ok = o + P2 * (k1 - 1 + __builtin_ctz(both));
+      t.lim[it][ok] = 1.0;
+      t.lim[is][ok] = 1.0;
+    }
   }
 }
 
@@ -2090,8 +2103,10 @@ int launch_tmask_limit(mom_gpu_ctx *ctx, int ntr, const double *const *T, const 
     t.T[n] = T[n]; t.lim[n] = lim[n]; t.mn[n] = mn[n]; t.mx[n] = mx[n];
   }
   // i in isc-1..iec, j in jsc-1..jec
-  hipLaunchKernelGGL(k_tmask_limit, dim3((d.ni + 1 + 63) / 64, (d.nj + 1 + 3) / 4, d.nk),
-                     dim3(64, 4), 0, ctx->stream, d, t, it, is, ts_same, ctx->kmt);
+  const int ntx = (d.ni + 1 + 63) / 64, ntiles = ntx * ((d.nj + 1 + 3) / 4);
+  const int per_xcd = (ntiles + 7) / 8;
+  hipLaunchKernelGGL(k_tmask_limit, dim3(8 * per_xcd, (d.nk + LIM_NK - 1) / LIM_NK), dim3(64, 4),
+                     0, ctx->stream, d, t, it, is, ts_same, ctx->kmt, ntx, ntiles, per_xcd);
   MOM_LAUNCHED(ctx, "k_tmask_limit");
   return MOM_GPU_OK;
 }

@@ -121,13 +121,15 @@ struct StepJob {
 
 // One 64-wide tile of one job, marched through all levels.  Every thread of
 // the block calls it with the same job and tile.
-// TH: some FP64 tracer of the group has other th_tendency terms.  A pass without
+// TH: 1 where some FP64 tracer of the group has other th_tendency terms, 2 for the
+// tendency alone (th_tendency += ..., tab.out; one FP64 tracer, ONEB).  A pass without
 // them must not hold their load: at the join of the branch around it the wait is
 // for every load in flight, the next level's too.  (Only the shapes with loads
 // in flight there, one row a wavefront and up to two tracers, have both forms.)
+constexpr int TENDENCY = 2;
 template <typename TT, int G, int RPW>
 constexpr bool both_th() { return sizeof(TT) == 8 && RPW == 1 && G <= 2; }
-template <typename TT, int G, int RPW, int NW, bool TH>
+template <typename TT, int G, int RPW, int NW, int TH>
 __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
   const KDom d = J.d;
   const StepTab<TT> &tab = J.tab;
@@ -367,16 +369,19 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
         const size_t pk = (size_t)P2 * (kf - 1);
         const double mi = mk<double>(kf, km[q]);
         const double rm1 = nm[q];
-        const double rr = Rr ? nx[q] : 1.0 / (nx[q] + EPSLN);
+        double rr = 0.0;
+        if constexpr (TH != TENDENCY) rr = Rr ? nx[q] : 1.0 / (nx[q] + EPSLN);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
           double thin = 0.0;
-          if constexpr (TH) thin = tab.th[g] ? ld_lv(tab.th[g] + pk, bz[q]) : 0.0;
+          if constexpr (TH == 1) thin = tab.th[g] ? ld_lv(tab.th[g] + pk, bz[q]) : 0.0;
           const double Tc = t0[g][q];
           double tr = pf_tx[g][q] + pf_xf[q] * (s_fy[bp][g][ry - 1][lane] - s_fy[bp][g][ry][lane]);
           tr = tr + pf_dtr[q] * Tc * pf_brk[q];
+          if constexpr (TH == TENDENCY) thin = rm1;   // the terms so far
           const double th = thin + mdfl64::tendency(pf_r[q], tr, Tc, rdt, mi);
-          st_lv(tab.out[g] + pk, bt[q], (rm1 * Tc + dtime * th) * rr);
+          if constexpr (TH == TENDENCY) st_lv(tab.out[g] + pk, bt[q], th);
+          else st_lv(tab.out[g] + pk, bt[q], (rm1 * Tc + dtime * th) * rr);
         }
       }
     }
@@ -578,8 +583,12 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
       if (k > 1) update_deferred(k - 1);
 #pragma unroll
       for (int q = 0; q < RPW; ++q) {
-        nm[q] = ld_lv(Rm1 + (size_t)P2 * k0, bz[q]);
-        nx[q] = ld_lv(Rx + (size_t)P2 * k0, bz[q]);
+        if constexpr (TH == TENDENCY) {
+          nm[q] = ld_lv(tab.out[0] + (size_t)P2 * k0, bz[q]);
+        } else {
+          nm[q] = ld_lv(Rm1 + (size_t)P2 * k0, bz[q]);
+          nx[q] = ld_lv(Rx + (size_t)P2 * k0, bz[q]);
+        }
       }
     }
     if constexpr (PRE) {
@@ -745,7 +754,7 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
 }
 
 
-template <typename TT, int G, int RPW, int NW, bool TH>
+template <typename TT, int G, int RPW, int NW, int TH>
 __global__ __launch_bounds__(RX * NW) void k_step(StepJob<TT> J, int per_xcd) {
   const int b = blockIdx.x;
   // XCD-aware: each XCD takes per_xcd consecutive positions of the order of
@@ -759,7 +768,7 @@ __global__ __launch_bounds__(RX * NW) void k_step(StepJob<TT> J, int per_xcd) {
 // counter in order (jobs sorted largest first) until none is left.  first[j]
 // is the index of job j's first item; total = sum of the jobs' tiles.  Every
 // block leaves the loop once the counter passes total.
-template <typename TT, int G, int RPW, int NW, bool TH>
+template <typename TT, int G, int RPW, int NW, int TH>
 __global__ __launch_bounds__(RX * NW) void k_step_queue(const StepJob<TT> *__restrict__ jobs,
                                                         const int *__restrict__ first, int njobs,
                                                         int total, int *__restrict__ counter) {
@@ -1087,6 +1096,23 @@ static int ensemble_type(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *steps
 
 // Advection + explicit update for ntr MDFL-Sweby tracers.  dtype[n]: 8 = FP64
 // (reference rounding), 4 = FP32 (single precision, division-free limiter).
+int launch_mdfl_tendency(mom_gpu_ctx *ctx, const double *T, const double *u, const double *v,
+                         const double *w, const double *rho, double dtime, double *th) {
+  constexpr int NW = 16, TY = NW - 4;
+  const KDom &d = ctx->kd;
+  const int ntx = (d.ni + TX - 1) / TX, ntiles = ntx * ((d.nj + TY - 1) / TY);
+  const int per = (ntiles + 7) / 8;
+  StepTab<double> tab{};
+  tab.T[0] = T;
+  tab.out[0] = th;
+  const StepJob<double> J{d, tab, u, v, w, rho, nullptr, nullptr, ctx->kmt, ctx->dat, ctx->datr,
+                          ctx->dxte, ctx->dyte, ctx->dxtn, ctx->dytn, dtime, ntx, ntiles};
+  hipLaunchKernelGGL((k_step<double, 1, 1, NW, TENDENCY>), dim3(8 * per), dim3(RX * NW), 0,
+                     ctx->stream, J, per);
+  MOM_LAUNCHED(ctx, "k_step (tendency)");
+  return MOM_GPU_OK;
+}
+
 int launch_tracer_step(mom_gpu_ctx *ctx, int ntr, const void *const *T_in, void *const *T_out,
                        const int *dtype, const double *const *th_in, const double *u,
                        const double *v, const double *w, const double *rho,

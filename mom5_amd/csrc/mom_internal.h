@@ -237,6 +237,8 @@ int mom_fail(mom_gpu_ctx *ctx, int code, const char *fmt, ...);
   } while (0)
 
 // Kernel launchers implemented in the k_*.hip translation units.
+int launch_mdfl_tendency(mom_gpu_ctx *ctx, const double *T, const double *u, const double *v,
+                         const double *w, const double *rho, double dtime, double *th);
 int launch_mdfl(mom_gpu_ctx *ctx, int flavor, const double *T,
                 const double *u, const double *v, const double *w,
                 const double *rho, double dtime, double lim, double *th,

@@ -110,6 +110,50 @@ def test_advect_sweby_all(setup):
         assert_close_scaled(dw[n].to_host(), wrk_ref[n], th_scale, what=f"wrk1 {n}")
 
 
+@pytest.mark.parametrize("ni,nj,nk,cyclic", [(7, 5, 2, True), (61, 13, 2, False), (60, 12, 3, True),
+                                             (131, 25, 12, False), (121, 37, 21, True)])
+def test_plain_routines_sizes(oracle_lib, ni, nj, nk, cyclic):
+    """The per-tracer routines at the edges of their tiles and level chunks: the
+    MDFL-Sweby tendency alone (the batched step's pass) equals, bit for bit,
+    the routine that writes its other outputs too; Quicker and the limiter
+    masks equal the CPU restatement."""
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    print(f"[plain routines {ni}x{nj}x{nk} cyclic={cyclic}]", flush=True)
+    case = make_case(ni, nj, nk, land_frac=0.2, seed=ni, cyclic_x=cyclic, barotropic=False)
+    orc, gpu = oracle_lib.Oracle(case), OceanGPU(case.dom, case.grid)
+    H, rng = DeviceArray.from_host, np.random.default_rng(nk)
+    f = {k: H(case.fields[k]) for k in ("uhrho_et", "vhrho_nt", "wrho_bt", "rho_dzt")}
+    Ts = [t for _, t in case.tracers]
+    th0 = rng.standard_normal(orc.shape3)
+    got = []
+    for wrk in (None, gpu.field3()):
+        th = H(th0)
+        gpu.horz_advect_tracer("mdfl_sweby", H(Ts[0]), th, uhrho_et=f["uhrho_et"],
+                               vhrho_nt=f["vhrho_nt"], wrho_bt=f["wrho_bt"],
+                               rho_dzt_tau=f["rho_dzt"], dtime=case.dt, wrk1=wrk)
+        gpu.sync()
+        got.append(th.to_host())
+    same(got[0], got[1])
+    mins, maxs = [float(np.quantile(t, 0.2)) for t in Ts], [float(np.quantile(t, 0.8)) for t in Ts]
+    lim = orc.tmask_limit(Ts, mins, maxs, 0, 1, True)
+    outs = [gpu.field3() for _ in Ts]
+    gpu.compute_tmask_limit([H(t) for t in Ts], mins, maxs, outs, 0, 1, True)
+    gpu.sync()
+    for a, b in zip(outs, lim):
+        same(a.to_host(), b)
+    th, th_ref = H(th0), th0.copy()
+    th_ref[:, 1:-1, 1:-1] += -orc.horz_quicker(Ts[0], Ts[0], lim[0], False, want_flux=True)[0]
+    dT, dlim = H(Ts[0]), H(lim[0])
+    gpu.horz_advect_tracer("quicker", dT, th, T_tau=dT, uhrho_et=f["uhrho_et"],
+                           vhrho_nt=f["vhrho_nt"], tmask_limit=dlim)
+    th_ref[:, 1:-1, 1:-1] += -orc.vert_quicker(Ts[0], Ts[0], lim[0], want_flux=True)[0]
+    gpu.vert_advect_tracer("quicker", dT, th, T_tau=dT, wrho_bt=f["wrho_bt"], tmask_limit=dlim)
+    gpu.sync()
+    same(th.to_host(), th_ref)
+    gpu.close()
+
+
 def _limits(case):
     mins = [2.0, 34.8] + [-0.1] * (len(case.tracers) - 2)
     maxs = [20.0, 35.2] + [0.01] * (len(case.tracers) - 2)
