@@ -117,10 +117,12 @@ struct StepJob {
   const double *dat, *datr, *dxte, *dyte, *dxtn, *dytn;
   double dtime;
   int ntx, ntiles;
+  int nchunk;   // level chunks a tile is split into (k_step)
 };
 
-// One 64-wide tile of one job, marched through all levels.  Every thread of
-// the block calls it with the same job and tile.
+// One 64-wide tile of one job, marched through levels ka..kb.  Every thread of
+// the block calls it with the same arguments.  A chunk that does not start at
+// the surface forms the flux through its top face again, from the level above.
 // TH: 1 where some FP64 tracer of the group has other th_tendency terms, 2 for the
 // tendency alone (th_tendency += ..., tab.out; one FP64 tracer, ONEB).  A pass without
 // them must not hold their load: at the join of the branch around it the wait is
@@ -130,7 +132,7 @@ constexpr int TENDENCY = 2;
 template <typename TT, int G, int RPW>
 constexpr bool both_th() { return sizeof(TT) == 8 && RPW == 1 && G <= 2; }
 template <typename TT, int G, int RPW, int NW, int TH>
-__device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
+__device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka, int kb) {
   const KDom d = J.d;
   const StepTab<TT> &tab = J.tab;
   const double *__restrict__ U = J.U;
@@ -193,6 +195,7 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
   if (si < 0 || si >= d.ni) {
     if (d.cyclic_x) si = wrapi(si, d.ni); else colok = false;
   }
+  const int kz = max(ka - 1, 1);   // the first level whose z face is formed
   int km[RPW], offz[RPW], gjr[RPW], sjr[RPW];
   bool ok[RPW], rowok[RPW];
   // per-row state: FP64 for FP64 groups (reference rounding), FP32 for FP32
@@ -223,10 +226,11 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
       if (ok[q]) {
         const TT *T = tab.T[g];
         const int o = offz[q];
-        t0[g][q] = T[o];
-        t1[g][q] = t0[g][q];
-        t2[g][q] = T[o + P2 * (min(2, nk) - 1)];
-        t3[g][q] = T[o + P2 * (min(3, nk) - 1)];
+        const size_t pl = P2;
+        t0[g][q] = T[o + pl * (max(kz - 1, 1) - 1)];
+        t1[g][q] = T[o + pl * (kz - 1)];
+        t2[g][q] = T[o + pl * (min(kz + 1, nk) - 1)];
+        t3[g][q] = T[o + pl * (min(kz + 2, nk) - 1)];
       } else {
         t0[g][q] = t1[g][q] = t2[g][q] = t3[g][q] = TT(0);
       }
@@ -326,11 +330,12 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
     for (int q = 0; q < RPW; ++q) {
       bh[q] = gi >= -1 && gi <= d.ni && gjr[q] >= -1 && gjr[q] <= d.nj
                   ? (unsigned)d2(d, gi, gjr[q]) * 8u : 0u;
-      nw[q] = ld_lv(W + P2, bz[q]);
-      nr[q] = ld_lv(R, bz[q]);
-      nu[q] = ld_lv(U, bx[q]);
-      nh[q] = ld_lv(R, bh[q]);
-      nv[q] = ld_lv(V, by[q]);
+      const size_t pa = (size_t)P2 * (ka - 1);
+      nw[q] = ld_lv(W + P2 + pa, bz[q]);
+      nr[q] = ld_lv(R + pa, bz[q]);
+      nu[q] = ld_lv(U + pa, bx[q]);
+      nh[q] = ld_lv(R + pa, bh[q]);
+      nv[q] = ld_lv(V + pa, by[q]);
     }
   }
   auto lv_load = [&](int k, LvIn *L) {
@@ -580,7 +585,7 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
     }
     __syncthreads();
     if constexpr (ONEB) {
-      if (k > 1) update_deferred(k - 1);
+      if (k > ka) update_deferred(k - 1);
 #pragma unroll
       for (int q = 0; q < RPW; ++q) {
         if constexpr (TH == TENDENCY) {
@@ -746,10 +751,40 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile) {
       }
     }
   };
-  for (int k = 1; k <= nk; ++k) level(k);
+  // the z face above the chunk (level()'s Z, the flux alone)
+  if (ka > 1) {
+#pragma unroll
+    for (int q = 0; q < RPW; ++q) {
+      const size_t pz = (size_t)P2 * (kz - 1);
+      const double w0 = ld_lv(W + pz + P2, bz[q]), r0 = ld_lv(R + pz, bz[q]);
+      const double w = ok[q] ? w0 : 0.0, r = ok[q] ? r0 : 1.0;
+      const TT mB = mk<TT>(kz + 1, km[q]), mC = mk<TT>(min(kz + 2, nk), km[q]);
+      FaceC<float> cf{0.0f, 0.0f, 0.0f, 0.0f};
+      FaceW wz{0.0f, 0.0f};
+      mdfl64::Face cz{};
+      if constexpr (!EXACT) {
+        const float wf = (float)w;
+        cf = face_coef_f((float)datv[q] * wf, fabsf(wf * (float)dtime * rcpf((float)r)));
+        wz = face_w(cf, mB);
+      } else {
+        cz = mdfl64::face(datv[q] * w, mdfl64::cfl_z(w, dtime * mdfl64::rcp64(r)), mB);
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const TT Rjp = t0[g][q] - t1[g][q], Rj = t1[g][q] - t2[g][q];
+        const TT Rjm = (t2[g][q] - t3[g][q]) * mC;
+        if constexpr (!EXACT) ftp[g][q] = flux_fast(cf, wz, Rjm, Rj, Rjp, t2[g][q], t1[g][q]);
+        else ftp[g][q] = mdfl64::flux(cz, Rjm, Rj, Rjp, t2[g][q], t1[g][q]);
+        t0[g][q] = t1[g][q]; t1[g][q] = t2[g][q]; t2[g][q] = t3[g][q];
+        if (ok[q]) t3[g][q] = ld_lv(tab.T[g] + (size_t)P2 * (min(kz + 3, nk) - 1), bt[q]);
+      }
+      wkm1[q] = (RT)w;
+    }
+  }
+  for (int k = ka; k <= kb; ++k) level(k);
   if constexpr (ONEB) {
     __syncthreads();
-    update_deferred(nk);
+    update_deferred(kb);
   }
 }
 
@@ -760,8 +795,10 @@ __global__ __launch_bounds__(RX * NW) void k_step(StepJob<TT> J, int per_xcd) {
   // XCD-aware: each XCD takes per_xcd consecutive positions of the order of
   // 8-wide strips, so x- and y-neighbours share their halo in one L2
   const int t = (b & 7) * per_xcd + (b >> 3);
-  if (t >= J.ntiles) return;
-  step_tile<TT, G, RPW, NW, TH>(J, strip_tile<8>(t, J.ntx, J.ntiles / J.ntx));
+  if (t >= J.ntiles * J.nchunk) return;
+  const int c = t % J.nchunk, nk = J.d.nk;
+  step_tile<TT, G, RPW, NW, TH>(J, strip_tile<8>(t / J.nchunk, J.ntx, J.ntiles / J.ntx),
+                                nk * c / J.nchunk + 1, nk * (c + 1) / J.nchunk);
 }
 
 // Ensemble pass: a persistent grid takes (job, tile) items from a device-side
@@ -784,7 +821,7 @@ __global__ __launch_bounds__(RX * NW) void k_step_queue(const StepJob<TT> *__res
       const int mid = (lo + hi + 1) >> 1;
       if (first[mid] <= item) lo = mid; else hi = mid - 1;
     }
-    step_tile<TT, G, RPW, NW, TH>(jobs[lo], item - first[lo]);
+    step_tile<TT, G, RPW, NW, TH>(jobs[lo], item - first[lo], 1, jobs[lo].d.nk);
   }
 }
 
@@ -914,6 +951,18 @@ static void add_th_f32(hipStream_t s, const KDom &d, float *out, const double *t
                      th, R, Rr, dtime);
 }
 
+// Level chunks a tile is split into: as many as still take one round of the 256
+// CUs (a tile fills one), at least four levels each (a chunk costs about 1.2
+// levels more).  us of a step or pass alone / among three states in turn:
+//   90x60x25, 10 tiles: one chunk 208 / 83, 6 chunks 154 / 67
+//   240x180x40, T, S and four FP32, 60 tiles: 273 / 135, 4 chunks 136 / 126
+//   360x240x40, T, S and six FP32, 120 tiles: 381 / 264, 2 chunks 269 / 274
+//   517x389x41, 297 tiles: 850 / 664; 2 chunks 758 / 688, but what the rounds gain
+//   alone costs work that other streams would have filled the chip with.
+static int level_chunks(int ntiles, int nk) {
+  return std::max(1, std::min(256 / ntiles, nk / 4));
+}
+
 template <typename TT>
 static bool any_th(const StepTab<TT> &t, int n) {
   for (int g = 0; g < n; ++g)
@@ -934,9 +983,9 @@ struct GroupLaunch {
     const int ntx = (d.ni + TX - 1) / TX;
     const int nty = (d.nj + TY - 1) / TY;
     const int ntiles = ntx * nty;
-    const int per = (ntiles + 7) / 8;
+    const int chunks = level_chunks(ntiles, d.nk), per = (ntiles * chunks + 7) / 8;
     const StepJob<TT> J{d, tab, u, v, w, rho, rm1, rr, ctx->kmt, ctx->dat, ctx->datr,
-                        ctx->dxte, ctx->dyte, ctx->dxtn, ctx->dytn, dtime, ntx, ntiles};
+                        ctx->dxte, ctx->dyte, ctx->dxtn, ctx->dytn, dtime, ntx, ntiles, chunks};
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(8 * per), dim3(RX * NW), 0, ctx->stream, J, per);
     };
@@ -1101,12 +1150,13 @@ int launch_mdfl_tendency(mom_gpu_ctx *ctx, const double *T, const double *u, con
   constexpr int NW = 16, TY = NW - 4;
   const KDom &d = ctx->kd;
   const int ntx = (d.ni + TX - 1) / TX, ntiles = ntx * ((d.nj + TY - 1) / TY);
-  const int per = (ntiles + 7) / 8;
+  const int chunks = level_chunks(ntiles, d.nk), per = (ntiles * chunks + 7) / 8;
   StepTab<double> tab{};
   tab.T[0] = T;
   tab.out[0] = th;
   const StepJob<double> J{d, tab, u, v, w, rho, nullptr, nullptr, ctx->kmt, ctx->dat, ctx->datr,
-                          ctx->dxte, ctx->dyte, ctx->dxtn, ctx->dytn, dtime, ntx, ntiles};
+                          ctx->dxte, ctx->dyte, ctx->dxtn, ctx->dytn, dtime, ntx, ntiles,
+                          chunks};
   hipLaunchKernelGGL((k_step<double, 1, 1, NW, TENDENCY>), dim3(8 * per), dim3(RX * NW), 0,
                      ctx->stream, J, per);
   MOM_LAUNCHED(ctx, "k_step (tendency)");

@@ -133,3 +133,22 @@ def test_ensemble_members_match_oracle():
         assert np.array_equal(m.eta_bar[m.cur].to_host(), eb), k
         assert np.array_equal(m.udrho[m.cur].to_host(), ud), k
     ens.close()
+
+
+@pytest.mark.parametrize("ni,nj,nk", [(20, 9, 33), (20, 9, 4), (61, 40, 8), (200, 100, 29),
+                                      (400, 210, 9)])
+def test_level_chunks_of_small_domains(ni, nj, nk):
+    """A small domain stepped alone splits its tiles by levels (here one to
+    eight chunks, one to 126 tiles) and forms the flux between two chunks twice;
+    the ensemble pass never splits: the same bits, FP64 and FP32."""
+    from mom5_amd.ensemble import EnsembleStep, make_regional_ensemble
+    print(f"[level chunks {ni}x{nj}x{nk}]", flush=True)
+    cases = make_regional_ensemble([dict(ni=ni, nj=nj, nk=nk, nts=4, lat_s=10.0, lat_n=20.0,
+                                         lon_span=10.0, seed=21)], n_passive=3)
+    alone, ens_m = _members(cases, fresh=True), _members(cases, fresh=True)
+    alone[0].run(3)
+    _sync(alone)
+    ens = EnsembleStep(ens_m)
+    ens.run(3)
+    ens.gpu.sync()
+    _assert_same(alone, ens_m, "chunks")
