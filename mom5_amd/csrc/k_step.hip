@@ -90,13 +90,16 @@ __device__ inline FaceW face_w(const FaceC<float> &c, float mab) {
   const bool pos = c.M >= 0.0f;
   return FaceW{c.M * mab, pos ? 1.0f : -1.0f, pos};
 }
-__device__ inline float flux_fast(const FaceC<float> &c, const FaceW &w, float Rjm, float Rj,
-                                  float Rjp, float Tpos, float Tneg) {
+// with the upwind side's neighbouring difference and tracer
+__device__ inline float flux_up(const FaceC<float> &c, const FaceW &w, float Rn, float Rj,
+                                float Tu) {
   const float d0a = c.d0 * Rj;
   const float sel = minmax_sel(Rj);
-  const float Rn = w.pos ? Rjm : Rjp;
-  const float Tu = w.pos ? Tpos : Tneg;
   return w.wm * fmaf(w.sg, psi_r(c, d0a, Rj, sel, Rn), Tu);
+}
+__device__ inline float flux_fast(const FaceC<float> &c, const FaceW &w, float Rjm, float Rj,
+                                  float Rjp, float Tpos, float Tneg) {
+  return flux_up(c, w, w.pos ? Rjm : Rjp, Rj, w.pos ? Tpos : Tneg);
 }
 
 template <typename TT>
@@ -170,7 +173,12 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
   // With the loads at the level's start two FP64 tracers took 1.75 ms at
   // 1440x1080x50; so, and without branches, 1.50 ms, now bound by vector
   // instructions: 347 a level and wavefront, issued 82% of the time (ten FP32
-  // tracers: 752, 91%).
+  // tracers: 712, 91%).  The tracers' loads take no branch: a point outside the
+  // domain reads past the level's end, a 0 (with the branch, and a window kept as
+  // four tracers instead of three and a difference, FP32 took 752 instructions
+  // and waited for the loads where the loop closes: pass of T, S and six FP32
+  // at 517x389x41 827 us alone, now 800; eight FP64 at 1440x1080x50 9.24 to 9.04
+  // ms).
   constexpr bool EARLYT = RPW == 1 && EXACT && G <= 2;
   constexpr bool ONEB = EARLYT &&
                         2 * 2 * G * RY * RX * sizeof(TT) + RY * RX * sizeof(int) <= 160 * 1024;
@@ -231,6 +239,8 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
         t1[g][q] = T[o + pl * (kz - 1)];
         t2[g][q] = T[o + pl * (min(kz + 1, nk) - 1)];
         t3[g][q] = T[o + pl * (min(kz + 2, nk) - 1)];
+        // shapes that update within the level keep the difference, not the tracer above
+        if constexpr (!ONEB) t0[g][q] = t0[g][q] - t1[g][q];
       } else {
         t0[g][q] = t1[g][q] = t2[g][q] = t3[g][q] = TT(0);
       }
@@ -312,11 +322,13 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
   }
   // byte offsets within a level: of the point (FP64 fields and tracers), of
   // its east face and of its north face (FP64 fields)
+  const unsigned tlev = (unsigned)P2 * (unsigned)sizeof(TT);   // bytes of a tracer's level
   unsigned bz[RPW], bt[RPW], bx[RPW], by[RPW];
 #pragma unroll
   for (int q = 0; q < RPW; ++q) {
     bz[q] = (unsigned)offz[q] * 8u;
-    bt[q] = (unsigned)offz[q] * (unsigned)sizeof(TT);
+    // a point outside the domain: past the level, where its tracer reads 0
+    bt[q] = ok[q] ? (unsigned)offz[q] * (unsigned)sizeof(TT) : tlev;
     bx[q] = (unsigned)oxq[q] * 8u;
     by[q] = (unsigned)oyq[q] * 8u;
   }
@@ -438,10 +450,12 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
         const float wdiff = (float)wkm1[q] - wf;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-          const float Rjp = t0[g][q] - t1[g][q];
+          // the old difference is done with before the new one takes its register
+          float Rn = wz.pos ? (t2[g][q] - t3[g][q]) * mC : t0[g][q];
+          asm volatile("" : "+v"(Rn), "+v"(t1[g][q]));
           const float Rj = t1[g][q] - t2[g][q];
-          const float Rjm = (t2[g][q] - t3[g][q]) * mC;
-          const float fbt = flux_fast(c, wz, Rjm, Rj, Rjp, t2[g][q], t1[g][q]);
+          t0[g][q] = Rj;
+          const float fbt = flux_up(c, wz, Rn, Rj, wz.pos ? t2[g][q] : t1[g][q]);
           tz[g][q] = fmaf(dtrf, fmaf(datrf, fbt - ftp[g][q], t1[g][q] * wdiff), t1[g][q]);
           fbtv[g][q] = fbt;
         }
@@ -456,8 +470,9 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
         const double wdiff = wkm1[q] - w;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-          const double Rjp = t0[g][q] - t1[g][q];
+          const double Rjp = ONEB ? t0[g][q] - t1[g][q] : t0[g][q];
           const double Rj = t1[g][q] - t2[g][q];
+          if constexpr (!ONEB) t0[g][q] = Rj;
           const double Rjm = (t2[g][q] - t3[g][q]) * mC;
           const double fbt = mdfl64::flux(cz, Rjm, Rj, Rjp, t2[g][q], t1[g][q]);
           tz[g][q] = t1[g][q] + dtr * (datrv[q] * (fbt - ftp[g][q]) + t1[g][q] * wdiff);
@@ -473,10 +488,8 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
       const size_t p3 = (size_t)P2 * (min(k + 3, nk) - 1);
 #pragma unroll
       for (int q = 0; q < RPW; ++q) {
-        if (ok[q]) {
 #pragma unroll
-          for (int g = 0; g < G; ++g) t4[g][q] = ld_lv(tab.T[g] + p3, bt[q]);
-        }
+        for (int g = 0; g < G; ++g) t4[g][q] = ld_lv0(tab.T[g] + p3, bt[q], tlev);
       }
     }
     // the next level's (the last level loads its own again)
@@ -739,15 +752,22 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         if constexpr (EXACT) ftp[g][q] = fbtv[g][q];
-        t0[g][q] = t1[g][q]; t1[g][q] = t2[g][q]; t2[g][q] = t3[g][q];
+        if constexpr (ONEB) t0[g][q] = t1[g][q];
+        if constexpr (EXACT) {
+          t1[g][q] = t2[g][q]; t2[g][q] = t3[g][q];
+        } else {
+          // moved here, not where the loop closes: the loads below then go to t3
+          // itself and are waited for where the next level uses it
+          asm volatile("v_mov_b32 %0, %1" : "=v"(t1[g][q]) : "v"(t2[g][q]));
+          asm volatile("v_mov_b32 %0, %1" : "=v"(t2[g][q]) : "v"(t3[g][q]));
+        }
         if constexpr (EARLYT) t3[g][q] = t4[g][q];
       }
       if constexpr (!EARLYT) {
         const size_t p3 = (size_t)P2 * (min(k + 3, nk) - 1);
-        if (ok[q]) {
+        if constexpr (!EXACT) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int g = 0; g < G; ++g) t3[g][q] = ld_lv(tab.T[g] + p3, bt[q]);
-        }
+        for (int g = 0; g < G; ++g) t3[g][q] = ld_lv0(tab.T[g] + p3, bt[q], tlev);
       }
     }
   };
@@ -771,12 +791,13 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
       }
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const TT Rjp = t0[g][q] - t1[g][q], Rj = t1[g][q] - t2[g][q];
+        const TT Rjp = ONEB ? t0[g][q] - t1[g][q] : t0[g][q], Rj = t1[g][q] - t2[g][q];
         const TT Rjm = (t2[g][q] - t3[g][q]) * mC;
         if constexpr (!EXACT) ftp[g][q] = flux_fast(cf, wz, Rjm, Rj, Rjp, t2[g][q], t1[g][q]);
         else ftp[g][q] = mdfl64::flux(cz, Rjm, Rj, Rjp, t2[g][q], t1[g][q]);
-        t0[g][q] = t1[g][q]; t1[g][q] = t2[g][q]; t2[g][q] = t3[g][q];
-        if (ok[q]) t3[g][q] = ld_lv(tab.T[g] + (size_t)P2 * (min(kz + 3, nk) - 1), bt[q]);
+        t0[g][q] = ONEB ? t1[g][q] : Rj;
+        t1[g][q] = t2[g][q]; t2[g][q] = t3[g][q];
+        t3[g][q] = ld_lv0(tab.T[g] + (size_t)P2 * (min(kz + 3, nk) - 1), bt[q], tlev);
       }
       wkm1[q] = (RT)w;
     }

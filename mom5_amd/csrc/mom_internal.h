@@ -129,6 +129,17 @@ __device__ inline float ld_lv(const float *base, unsigned boff) {
 __device__ inline double ld_lv(const double *base, unsigned boff) {
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(lvl_rsrc(base), (int)boff, 0, 0));
 }
+// the same with the range check at the level's end: a point at or past bytes
+// reads 0 (buffer loads out of the descriptor's range return 0)
+__device__ inline __amdgpu_buffer_rsrc_t lvl_rsrc(const void *p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
+}
+__device__ inline float ld_lv0(const float *base, unsigned boff, unsigned bytes) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(lvl_rsrc(base, bytes), (int)boff, 0, 0));
+}
+__device__ inline double ld_lv0(const double *base, unsigned boff, unsigned bytes) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(lvl_rsrc(base, bytes), (int)boff, 0, 0));
+}
 __device__ inline void st_lv(float *base, unsigned boff, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), lvl_rsrc(base), (int)boff, 0, 0);
 }
