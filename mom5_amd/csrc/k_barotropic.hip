@@ -223,13 +223,16 @@ constexpr double EPSLN_GRID = 1.0e-40;   // shared/constants/constants.F90:123
 // reciprocal ocean_grids.F90:949-951 forms; bit 1 where a metric the blocked
 // barotropic multiplies is outside LAND_BOUND in magnitude (or not a number)
 // or dxu, dyu, datr carries a sign bit; bit 2 where a metric bt_rows_tile takes from
-// its row differs from the row's first point.  The host ORs them up.
+// its row differs from the row's first point; bit 3 where one of those or of the
+// C-grid variants' does.  The host ORs them up.
 constexpr double LAND_BOUND = 1.0e100;
 __device__ inline bool bounded(double x) { return fabs(x) <= LAND_BOUND; }
 __global__ void k_check_recip(KDom d, const double *__restrict__ dxu,
                               const double *__restrict__ dxur, const double *__restrict__ dyu,
                               const double *__restrict__ dyur, const double *__restrict__ datr,
-                              const double *__restrict__ f, int *__restrict__ bad) {
+                              const double *__restrict__ f, const double *__restrict__ dat,
+                              const double *__restrict__ dxte, const double *__restrict__ dytn,
+                              int *__restrict__ bad) {
   auto differ = [](double a, double b) {
     return __builtin_bit_cast(unsigned long long, a) != __builtin_bit_cast(unsigned long long, b);
   };
@@ -248,7 +251,9 @@ __global__ void k_check_recip(KDom d, const double *__restrict__ dxu,
   const bool row_bad = differ(dxu[o], dxu[r]) || differ(dyu[o], dyu[r]) ||
                        differ(dxur[o], dxur[r]) || differ(dyur[o], dyur[r]) ||
                        differ(datr[o], datr[r]) || differ(f[o], f[r]);
-  bad[o] = (recip_bad ? 1 : 0) | (grid_bad ? 2 : 0) | (row_bad ? 4 : 0);
+  const bool crow_bad = row_bad || differ(dat[o], dat[r]) || differ(dxte[o], dxte[r]) ||
+                        differ(dytn[o], dytn[r]);
+  bad[o] = (recip_bad ? 1 : 0) | (grid_bad ? 2 : 0) | (row_bad ? 4 : 0) | (crow_bad ? 8 : 0);
 }
 
 // The per-call inputs that decide whether a point is inert under the
@@ -1092,7 +1097,8 @@ int launch_check_recip(mom_gpu_ctx *ctx) {
   int *dev = nullptr;
   MOM_HIP(ctx, hipMalloc(&dev, n * sizeof(int)));
   hipLaunchKernelGGL(k_check_recip, dim3((d.NI + 127) / 128, d.NJ), dim3(128), 0, ctx->stream, d,
-                     ctx->dxu, ctx->dxur, ctx->dyu, ctx->dyur, ctx->datr, ctx->f, dev);
+                     ctx->dxu, ctx->dxur, ctx->dyu, ctx->dyur, ctx->datr, ctx->f, ctx->dat, ctx->dxte,
+                     ctx->dytn, dev);
   hipError_t le = hipGetLastError();
   int *host = (int *)malloc(n * sizeof(int));
   hipError_t e1 = host ? hipMemcpyAsync(host, dev, n * sizeof(int), hipMemcpyDeviceToHost,
@@ -1112,6 +1118,7 @@ int launch_check_recip(mom_gpu_ctx *ctx) {
   ctx->bt_grid_ok = (bad & 2) == 0;
   // (the rows' constants lie behind the masks in one plane: 64 B a row)
   ctx->bt_rows_ok = (bad & 4) == 0 && d.NI >= 16;
+  ctx->btv_rows_ok = (bad & 8) == 0 && d.NI >= 16;
   return MOM_GPU_OK;
 }
 

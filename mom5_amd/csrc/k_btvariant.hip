@@ -249,16 +249,24 @@ __global__ void k_btv_corrector(BtvArgs<CG, PR> a, int fstau, int fstaup1, doubl
 
 // ---- temporally blocked subcycles -----------------------------------------
 // The two-launch form above moves every plane through memory twice a subcycle.
-// Here one work-group owns a 64 x 32 region of the data domain and advances it
-// nsub subcycles with its state in registers, reading and writing the planes
-// once a launch.  80 C-grid pressure subcycles at 1440x1080: 11.4 ms with two
-// launches each (112 + 43 us), 2.2 ms in sixteen launches of five.
+// Here one work-group owns a region of the data domain and advances it nsub
+// subcycles with its state in registers, reading and writing the planes once a
+// launch.
 //
-// A wavefront holds two neighbouring rows, so x neighbours are DPP lane shifts
-// and half of the y neighbours the thread's own registers; the other half goes
-// through LDS, one row a wavefront and quantity.  The forcing and the thickness
-// are read once a subcycle and lie in LDS too, which keeps a thread within the
-// 128 registers that 16 wavefronts a CU allow.
+// A wavefront holds neighbouring rows, so x neighbours are DPP lane shifts and
+// most y neighbours the thread's own registers; the others go through LDS, one
+// row a wavefront and quantity.  The forcing and the thickness are read once a
+// subcycle and lie in LDS too.
+//
+// Grids that do not change along a row (checked at creation) keep a row's
+// constants in scalar registers, so 8 wavefronts of three rows (64 x 24) take at
+// most 128 registers and two blocks share a CU: one loads while the other steps.
+// Other grids, and the C-grid depth scheme (whose LDS holds two more planes), take
+// 16 wavefronts of two rows (64 x 32), one block a CU.  A subcycle is bound by
+// its FP64 instructions (C-grid pressure: 87 a point), a launch by loading the
+// planes as much.  80 subcycles at 1440x1080, C-grid pressure: 11.4 ms with two
+// launches a subcycle, 2.26 ms in 64 x 32 regions with per-point constants and
+// edge tests everywhere (130 instructions a point), 1.56 ms so; B-grid pressure 1.03 ms.
 //
 // Dependencies: a transport needs the transports one point away in each
 // direction, x also those of one point west and south.  After nsub subcycles a
@@ -270,26 +278,55 @@ __global__ void k_btv_corrector(BtvArgs<CG, PR> a, int fstau, int fstaup1, doubl
 // from column NI-2 (1), two lanes to the left (right): two more halo lanes a
 // side.  A chain of dependencies crosses that seam once if ni > nsub, so
 // domains narrower than MIN_NI, and cyclic-y ones, keep the two launches.
-constexpr int VX = 64, VW = 16, VY = 2 * VW;
+constexpr int VX = 64;                 // region columns; rows: R a wavefront, NW wavefronts
 constexpr int MIN_NI = 16;             // > the most subcycles a launch takes (12)
 
 __host__ __device__ constexpr int btv_lo(int nsub, bool cyc) { return nsub + 1 + (cyc ? 2 : 0); }
 __host__ __device__ constexpr int btv_tx(int nsub, bool cyc) {
   return VX - 2 * nsub - 1 - (cyc ? 4 : 0);
 }
-__host__ __device__ constexpr int btv_ty(int nsub) { return VY - 2 * nsub - 1; }
+__host__ __device__ constexpr int btv_ty(int nsub, int ry) { return ry - 2 * nsub - 1; }
 
 struct BtvBlk {
   const double *xs, *us, *fs;          // state read: x, transports (2), force at two levels (4)
   double *xd, *ud, *fd;                // state written
   const unsigned char *mask;           // bit 0 tmask(k=1), bit 1 umask(k=1)
+  const double *rowc;                  // the rows' constants (UNI)
   int s0, nsub, nts, step_a, ntx, ntiles;
   int rev;                             // 1: the tiles in reverse order (see k_bt_block)
 };
 
+// A point's constants of the grid.  B-grid: datr, dyu/2, dxu/2, dxur/2, dyur/2,
+// cori1, cori2 (:1285-1286), f/2; C-grid: datr, dat, -, 1/(dxte + eps),
+// 1/(dytn + eps), -, -, f/4 (the halves and quarters of the averages they
+// multiply: powers of two, exact short of the subnormals).
+struct RowC {
+  double datr, m1, m2, g1, g2, k1, k2, f;
+};
+template <bool CG, bool PR>
+__device__ inline RowC row_const(const BtvArgs<CG, PR> &a, int o) {
+  RowC c{};
+  c.datr = a.datr[o];
+  const double f = a.f[o];
+  if (CG) {
+    c.m1 = a.dat[o];
+    c.g1 = 1.0 / (a.dxte[o] + kEpsln);
+    c.g2 = 1.0 / (a.dytn[o] + kEpsln);
+    c.f = 0.25 * f;
+  } else {
+    c.m1 = 0.5 * a.dyu[o]; c.m2 = 0.5 * a.dxu[o];
+    c.g1 = 0.5 * a.dxur[o]; c.g2 = 0.5 * a.dyur[o];
+    c.k1 = 0.5 * a.dtbt * f;
+    c.k2 = 1.0 / (1.0 + c.k1 * c.k1);
+    c.f = 0.5 * f;
+  }
+  return c;
+}
+
 // sf and the masks, constant over the subcycles
 template <bool CG, bool PR>
-__global__ void k_btv_sfmask(BtvArgs<CG, PR> a, unsigned char *__restrict__ mask) {
+__global__ void k_btv_sfmask(BtvArgs<CG, PR> a, unsigned char *__restrict__ mask,
+                             double *__restrict__ rowc) {
   const int ii = blockIdx.x * blockDim.x + threadIdx.x, jj = blockIdx.y;
   if (ii >= a.d.NI) return;
   const int o = ii + a.d.NI * jj;
@@ -297,86 +334,117 @@ __global__ void k_btv_sfmask(BtvArgs<CG, PR> a, unsigned char *__restrict__ mask
   const double s = a.pme[o] + a.river[o] + a.source[o] - a.smooth[o];
   a.sf[o] = PR ? tm * (a.grav * s + a.dpatm_dt[o]) : tm * s;
   mask[o] = (unsigned char)((1 <= a.kmt[o] ? 1 : 0) | (1 <= a.kmu[o] ? 2 : 0));
+  if (rowc && ii == 0) {
+    const RowC c = row_const(a, o);
+    double *r = rowc + (size_t)8 * jj;
+    r[0] = c.datr; r[1] = c.m1; r[2] = c.m2; r[3] = c.g1; r[4] = c.g2; r[5] = c.k1; r[6] = c.k2;
+    r[7] = c.f;
+  }
 }
 
-template <bool CG, bool PR>
-__global__ __launch_bounds__(VX *VW) void k_btv_block(BtvArgs<CG, PR> a, BtvBlk J, int per_xcd) {
-  const int b = blockIdx.x;
-  const int t0 = (b & 7) * per_xcd + (J.rev ? per_xcd - 1 - (b >> 3) : b >> 3);
-  if (t0 >= J.ntiles) return;                  // the whole block
-  const int tile = strip_tile<8>(t0, J.ntx, J.ntiles / J.ntx);
+template <bool CG, bool PR, int R, int NW>
+struct BtvLds {
+  static constexpr bool PL = CG && !PR;
+  // p and u1 (C) of the wavefronts' first rows, vh and u2 (C) or uh (B) of their last
+  double p[NW][VX], v[NW][VX], u1[NW][VX], u2[CG ? NW : 1][VX];
+  // forcing (2), thickness (C: 2), C: tmasken (1, a wavefront of three rows); C-grid
+  // depth: rho_g, patm
+  static constexpr int NC = PL ? 6 : (CG ? (R > 2 ? 5 : 4) : 3);
+  double c[NC][R][NW][VX];
+};
+
+// EDGE: the region meets the domain's first or last row or column, or the seam; the
+// others carry no such tests (two instances: in one, the branches cost registers).
+// UNI: the grid does not change along a row; its constants are scalars.
+template <bool CG, bool PR, int R, int NW, bool EDGE, bool UNI>
+__device__ __forceinline__ void btv_tile(const BtvArgs<CG, PR> &a, const BtvBlk &J, int tx, int ty,
+                                         BtvLds<CG, PR, R, NW> &S) {
   const KDom d = a.d;
   const int P2 = d.P2, nsub = J.nsub;
   const bool cyc = d.cyclic_x != 0;
-  __shared__ double s_p[VW][VX], s_v[VW][VX];             // p of the low rows, vh of the high
-  __shared__ double s_u1[VW][VX], s_u2[VW][VX];           // C: u1 of the low rows, u2 of the high
-  // forcing (2), thickness (C: 2); C-grid depth: rho_g, patm
   constexpr bool PL = CG && !PR;
-  __shared__ double s_c[PL ? 6 : (CG ? 4 : 3)][2][VW][VX];
+  constexpr bool KL = CG && !PL && R > 2;     // tmasken of the east face in LDS
+  auto &s_c = S.c;
   const int lane = threadIdx.x & (VX - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / VX);
-  const int wm = max(wave - 1, 0), wp = min(wave + 1, VW - 1);
+  const int wm = max(wave - 1, 0), wp = min(wave + 1, NW - 1);
   const int LX = btv_lo(nsub, cyc), LY = btv_lo(nsub, false);
-  const int TX = btv_tx(nsub, cyc), TY = btv_ty(nsub);
-  const int seq = (tile % J.ntx) * TX - LX + lane;        // position in the column sequence
+  const int TX = btv_tx(nsub, cyc), TY = btv_ty(nsub, R * NW);
+  const int seq = tx * TX - LX + lane;                    // position in the column sequence
   const int col = cyc ? wrapi(seq, d.NI) : seq;
-  const int row0 = (tile / J.ntx) * TY - LY + 2 * wave;
+  const int row0 = ty * TY - LY + R * wave;
   const bool colok = cyc || (seq >= 0 && seq < d.NI);
   // a region that holds the seam of a cyclic-x domain (uniform)
-  const int seq0 = (tile % J.ntx) * TX - LX;
-  const bool seam = cyc && (seq0 <= 0 || seq0 + VX > d.NI - 2);
+  const int seq0 = tx * TX - LX;
+  const bool seam = EDGE && cyc && (seq0 <= 0 || seq0 + VX > d.NI - 2);
   const bool first = J.s0 == 1;
+  const double rho0r = a.rho0r, dtbt = a.dtbt, ngrav = -a.grav;
+  typedef const __attribute__((address_space(4))) double ConstD;
 
-  int off[2];
-  bool in[2], tmb[2], umb[2], div0[2], grad0[2], comp[2], fromw[2], frome[2];
-  double x[2], u1[2], u2[2], fa1[2], fa2[2], fb1[2], fb2[2], sx[2], su1[2], su2[2];
-  double datr[2], m1[2], m2[2], g1c[2], g2c[2], k1[2], k2[2], f[2], sf[2], rg[2], pa[2];
+  auto inside = [&](int q) {
+    const int r = R * wave + q, j = row0 + q;
+    return colok && j >= 0 && j < d.NJ && lane >= LX && lane < LX + TX && seq < d.NI && r >= LY &&
+           r < LY + TY;
+  };
+  auto div0 = [&](int q) { return EDGE && (col == 0 || row0 + q == 0); };
+  auto grad0 = [&](int q) { return EDGE && (col == d.NI - 1 || row0 + q == d.NJ - 1); };
+  auto crow = [&](int q) { return row0 + q >= 1 && row0 + q <= d.nj; };
+  auto nocomp = [&](int q) { return EDGE && !(crow(q) && col >= 1 && col <= d.ni); };
+  // the halo update of a cyclic-x domain's halo columns: from two lanes away
+  auto update = [&](int q, double e) {
+    const double w = lane_prev(lane_prev(e)), n = lane_next(lane_next(e));
+    return !crow(q) ? e : (col == 0 ? w : (col == d.NI - 1 ? n : e));
+  };
+  bool tmb[R];
+  double x[R], u1[R], u2[R], fa1[R], fa2[R], fb1[R], fb2[R], sx[R], su1[R], su2[R];
+  double datr[R], m1[R], m2[R], g1c[R], g2c[R], k1[R], k2[R], f[R], sf[R], rg[R], pa[R], um[R];
   double fS = 0.0;
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
+  for (int q = 0; q < R; ++q) {
     const int j = row0 + q;
-    const bool present = colok && j >= 0 && j < d.NJ;
-    const bool crow = j >= 1 && j <= d.nj;
+    const bool present = !EDGE || (colok && j >= 0 && j < d.NJ);
     const int o = present ? col + d.NI * j : 0;
-    off[q] = o;
-    in[q] = present && lane >= LX && lane < LX + TX && seq < d.NI && 2 * wave + q >= LY &&
-            2 * wave + q < LY + TY;
-    div0[q] = col == 0 || j == 0;
-    grad0[q] = col == d.NI - 1 || j == d.NJ - 1;
-    comp[q] = crow && col >= 1 && col <= d.ni;
-    fromw[q] = cyc && crow && col == 0;
-    frome[q] = cyc && crow && col == d.NI - 1;
     double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
-    tmb[q] = umb[q] = false;
+    tmb[q] = false;
     x[q] = u1[q] = u2[q] = fa1[q] = fa2[q] = fb1[q] = fb2[q] = sx[q] = su1[q] = su2[q] = 0.0;
-    datr[q] = m1[q] = m2[q] = g1c[q] = g2c[q] = k1[q] = k2[q] = f[q] = sf[q] = rg[q] = pa[q] = 0.0;
+    datr[q] = m1[q] = m2[q] = g1c[q] = g2c[q] = k1[q] = k2[q] = f[q] = 0.0;
+    sf[q] = rg[q] = pa[q] = um[q] = 0.0;
+    if constexpr (UNI) {
+      const int jc = EDGE ? min(max(j, 0), d.NJ - 1) : j;       // uniform
+      ConstD *rc = (ConstD *)(unsigned long long)(J.rowc + (size_t)8 * jc);
+      datr[q] = rc[0]; m1[q] = rc[1]; g1c[q] = rc[3]; g2c[q] = rc[4]; f[q] = rc[7];
+      if (!CG) { m2[q] = rc[2]; k1[q] = rc[5]; k2[q] = rc[6]; }
+      if (CG && q == 0) {
+        ConstD *rs = (ConstD *)(unsigned long long)(J.rowc + (size_t)8 * max(jc - 1, 0));
+        fS = EDGE && j < 1 ? 0.0 : rs[7];
+      }
+    }
     if (present) {
       const unsigned char mb = J.mask[o];
       tmb[q] = (mb & 1) != 0;
-      umb[q] = (mb & 2) != 0;
+      um[q] = (mb & 2) ? 1.0 : 0.0;
       x[q] = J.xs[o]; u1[q] = J.us[o]; u2[q] = J.us[o + P2];
-      sf[q] = a.sf[o]; datr[q] = a.datr[o]; f[q] = a.f[o];
-      c0 = a.forcing[o]; c1 = a.forcing[o + P2];
-      c2 = a.thick[o];
+      sf[q] = a.sf[o];
+      // + 0.0 (depth): the forcing is the last term of the sum it is added to
+      c0 = PR ? a.forcing[o] : a.forcing[o] + 0.0;
+      c1 = PR ? a.forcing[o + P2] : a.forcing[o + P2] + 0.0;
+      c2 = PR ? rho0r * a.thick[o] : a.thick[o];
       if (!PR) { rg[q] = a.rho_g[o]; pa[q] = a.patm[o]; }
+      if constexpr (!UNI) {
+        const RowC c = row_const(a, o);
+        datr[q] = c.datr; m1[q] = c.m1; g1c[q] = c.g1; g2c[q] = c.g2; f[q] = c.f;
+        if (!CG) { m2[q] = c.m2; k1[q] = c.k1; k2[q] = c.k2; }
+        if (CG && q == 0) fS = j >= 1 ? 0.25 * a.f[o - d.NI] : 0.0;
+      }
       if (CG) {
-        c3 = a.thick[o + P2];
-        m1[q] = a.dat[o];
-        g1c[q] = 1.0 / (a.dxte[o] + kEpsln);
-        g2c[q] = 1.0 / (a.dytn[o] + kEpsln);
+        c3 = PR ? rho0r * a.thick[o + P2] : a.thick[o + P2];
         k1[q] = a.tmasken[o]; k2[q] = a.tmasken[o + P2];
         if (!first) {
           fa1[q] = J.fs[o]; fa2[q] = J.fs[o + P2];
           fb1[q] = J.fs[o + 2 * (size_t)P2]; fb2[q] = J.fs[o + 3 * (size_t)P2];
         }
-        if (q == 0) fS = j >= 1 ? a.f[o - d.NI] : 0.0;
-      } else {
-        m1[q] = a.dyu[o]; m2[q] = a.dxu[o];
-        g1c[q] = a.dxur[o]; g2c[q] = a.dyur[o];
-        k1[q] = 0.5 * a.dtbt * f[q];             // cori1, cori2 (:1285-1286)
-        k2[q] = 1.0 / (1.0 + k1[q] * k1[q]);
       }
-      if (in[q]) {
+      if (inside(q)) {
         if (first) {
           sx[q] = a.initsum ? a.xbar_tau[o] : a.x_tau[o];
         } else {
@@ -392,14 +460,17 @@ __global__ __launch_bounds__(VX *VW) void k_btv_block(BtvArgs<CG, PR> a, BtvBlk 
       s_c[4][q][wave][lane] = rg[q];
       s_c[5][q][wave][lane] = pa[q];
     }
+    if constexpr (KL) s_c[4][q][wave][lane] = k1[q];
   }
-  const double fW0 = lane_prev(f[0]), fW1 = lane_prev(f[1]);
+  double fW[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) fW[q] = UNI ? f[q] : lane_prev(f[q]);
 
-  // the transports through a cell's edges of both rows, those other rows read to LDS
-  double uh[2], vh[2], dv[2];
+  // the transports through a cell's edges of the rows, those other rows read to LDS
+  double uh[R], vh[R], g[R];
   auto share = [&]() {
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
+    for (int q = 0; q < R; ++q) {
       if (CG) {      // DIV_UD, C-grid (ocean_operators.F90:526-536)
         uh[q] = u1[q] * m1[q] * g1c[q];
         vh[q] = u2[q] * m1[q] * g2c[q];
@@ -408,31 +479,37 @@ __global__ __launch_bounds__(VX *VW) void k_btv_block(BtvArgs<CG, PR> a, BtvBlk 
         vh[q] = u2[q] * m2[q];
       }
     }
-    s_v[wave][lane] = vh[1];
-    if (CG) {
-      s_u1[wave][lane] = u1[0];
-      s_u2[wave][lane] = u2[1];
+    S.v[wave][lane] = vh[R - 1];
+    if constexpr (CG) {
+      S.u1[wave][lane] = u1[0];
+      S.u2[wave][lane] = u2[R - 1];
     } else {
-      s_u1[wave][lane] = uh[1];
+      S.u1[wave][lane] = uh[R - 1];
     }
   };
+  // g = the divergence term + sf: what the predictor and the corrector scale
   auto diverge = [&]() {
-    const double vs = s_v[wm][lane];
-    if (CG) {
-      dv[0] = ((uh[0] - lane_prev(uh[0])) + (vh[0] - vs)) * datr[0];
-      dv[1] = ((uh[1] - lane_prev(uh[1])) + (vh[1] - vh[0])) * datr[1];
-    } else {         // B-grid (:570-605)
-      const double us = s_u1[wm][lane];
-      const double bay0 = 0.5 * (uh[0] + us), bay1 = 0.5 * (uh[1] + uh[0]);
-      const double baxs = 0.5 * (vs + lane_prev(vs));
-      const double bax0 = 0.5 * (vh[0] + lane_prev(vh[0]));
-      const double bax1 = 0.5 * (vh[1] + lane_prev(vh[1]));
-      dv[0] = ((bay0 - lane_prev(bay0)) + (bax0 - baxs)) * datr[0];
-      dv[1] = ((bay1 - lane_prev(bay1)) + (bax1 - bax0)) * datr[1];
+    double vs = S.v[wm][lane], us = 0.0;
+    if constexpr (!CG) {
+      us = S.u1[wm][lane];
+      vs = vs + lane_prev(vs);                // twice the average, as m2 is half dxu
     }
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
-      if (div0[q]) dv[q] = 0.0;
+    for (int q = 0; q < R; ++q) {
+      double dv;
+      if constexpr (CG) {
+        dv = ((uh[q] - lane_prev(uh[q])) + (vh[q] - vs)) * datr[q];
+        vs = vh[q];
+      } else {         // B-grid (:570-605)
+        const double bay = uh[q] + us, bax = vh[q] + lane_prev(vh[q]);
+        dv = ((bay - lane_prev(bay)) + (bax - vs)) * datr[q];
+        us = uh[q];
+        vs = bax;
+      }
+      if (div0(q)) dv = 0.0;
+      const double tmp = PR ? ngrav * dv : (tmb[q] ? -dv : -dv * 0.0);
+      g[q] = tmp + sf[q];
+    }
   };
   share();
   __syncthreads();
@@ -442,19 +519,20 @@ __global__ __launch_bounds__(VX *VW) void k_btv_block(BtvArgs<CG, PR> a, BtvBlk 
     const int itime = J.s0 + t;
     // A: the prediction and the pressure; C-grid: the Coriolis force, from
     // the transports that the phases B before wrote
-    double F1[2], F2[2], p[2];
+    double F1[R], F2[R], p[R + 1];
     if constexpr (CG) {
-      const double u2s = s_u2[wm][lane], u1n = s_u1[wp][lane];
-      const double e0 = u2[0] + lane_next(u2[0]), e1 = u2[1] + lane_next(u2[1]);
-      const double es = u2s + lane_next(u2s);
-      F1[0] = 0.25 * (f[0] * e0 + fS * es);
-      F1[1] = 0.25 * (f[1] * e1 + f[0] * e0);
-      const double n0 = u1[0] + u1[1], n1 = u1[1] + u1n;
-      F2[0] = -(0.25 * (f[0] * n0 + fW0 * lane_prev(n0)));
-      F2[1] = -(0.25 * (f[1] * n1 + fW1 * lane_prev(n1)));
+      const double u1n = S.u1[wp][lane];
+      double es = S.u2[wm][lane], fs = fS;
+      es = es + lane_next(es);
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        if (!comp[q]) F1[q] = F2[q] = 0.0;
+      for (int q = 0; q < R; ++q) {
+        const double e = u2[q] + lane_next(u2[q]);
+        F1[q] = f[q] * e + fs * es;
+        const double n = u1[q] + (q + 1 < R ? u1[min(q + 1, R - 1)] : u1n);
+        F2[q] = -(f[q] * n + fW[q] * lane_prev(n));
+        es = e;
+        fs = f[q];
+        if (nocomp(q)) F1[q] = F2[q] = 0.0;
         if (itime == 1) {                     // all three levels (:3711-3730)
           fa1[q] = fb1[q] = F1[q];
           fa2[q] = fb2[q] = F2[q];
@@ -462,16 +540,11 @@ __global__ __launch_bounds__(VX *VW) void k_btv_block(BtvArgs<CG, PR> a, BtvBlk 
       }
     }
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
+    for (int q = 0; q < R; ++q) {
       double e = x[q];
-      if (a.predict) {
-        const double tmp = PR ? -a.grav * dv[q] : (tmb[q] ? -dv[q] : -dv[q] * 0.0);
-        e = x[q] + a.c_pred * (tmp + sf[q]);
-      }
-      if (!CG && seam) {                      // the legacy halo update (:3383, :4140)
-        const double w = lane_prev(lane_prev(e)), n = lane_next(lane_next(e));
-        e = fromw[q] ? w : (frome[q] ? n : e);
-      }
+      if (a.predict) e = x[q] + a.c_pred * g[q];
+      if constexpr (!CG)
+        if (seam) e = update(q, e);           // the legacy halo update (:3383, :4140)
       if constexpr (PR)
         p[q] = tmb[q] ? e : e * 0.0;
       else if constexpr (PL)
@@ -479,89 +552,68 @@ __global__ __launch_bounds__(VX *VW) void k_btv_block(BtvArgs<CG, PR> a, BtvBlk 
       else
         p[q] = rg[q] * e + pa[q];
     }
-    s_p[wave][lane] = p[0];
+    S.p[wave][lane] = p[0];
     __syncthreads();
     // B: pressure gradient and transports
-    {
-      const double pn1 = s_p[wp][lane];
-      double n1[2], n2[2];
+    p[R] = S.p[wp][lane];
+    double pe = lane_next(p[0]), fax = p[0] + pe;
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const double pn = q == 0 ? p[1] : pn1;
-        const double pe = lane_next(p[q]), pne = CG ? 0.0 : lane_next(pn);
-        double h1 = 0.0, h2 = 0.0;
-        if (!grad0[q]) {
-          if (CG) {    // GRAD_BAROTROPIC_P, C-grid (ocean_operators.F90:664-669)
-            h1 = (pe - p[q]) * g1c[q] * k1[q];
-            h2 = (pn - p[q]) * g2c[q] * k2[q];
-          } else {     // B-grid (:651-660)
-            const double p_fay = 0.5 * (p[q] + pn);
-            const double p_fax = 0.5 * (p[q] + pe);
-            const double pip_fay = 0.5 * (pe + pne);
-            const double pjp_fax = 0.5 * (pn + pne);
-            const double y1 = (pip_fay - p_fay) * g1c[q], y2 = (pjp_fax - p_fax) * g2c[q];
-            h1 = umb[q] ? y1 : y1 * 0.0;
-            h2 = umb[q] ? y2 : y2 * 0.0;
-          }
-        }
-        const double th1 = s_c[2][q][wave][lane], th2 = CG ? s_c[CG ? 3 : 2][q][wave][lane] : th1;
-        const double pf1 = PR ? -(a.rho0r * th1 * h1) : -(th1 * h1);
-        const double pf2 = PR ? -(a.rho0r * th2 * h2) : -(th2 * h2);
-        const double fo1 = s_c[0][q][wave][lane], fo2 = s_c[1][q][wave][lane];
-        if (CG) {
-          constexpr double ab0 = 23.0 / 12.0, ab1 = -16.0 / 12.0, ab2 = 5.0 / 12.0;  // :617-619
-          double acc1 = 0.0, acc2 = 0.0;
-          if (comp[q]) {
-            acc1 = ab0 * F1[q] + ab1 * fa1[q] + ab2 * fb1[q];
-            acc2 = ab0 * F2[q] + ab1 * fa2[q] + ab2 * fb2[q];
-          }
-          const double s1 = acc1 + pf1 + fo1, s2 = acc2 + pf2 + fo2;
-          n1[q] = u1[q] + a.dtbt * k1[q] * (PR ? s1 : s1 + 0.0);
-          n2[q] = u2[q] + a.dtbt * k2[q] * (PR ? s2 : s2 + 0.0);
-          if (seam) {                         // the halo update of udrho_bt (:3895-3897)
-            const double w1 = lane_prev(lane_prev(n1[q])), w2 = lane_prev(lane_prev(n2[q]));
-            const double e1 = lane_next(lane_next(n1[q])), e2 = lane_next(lane_next(n2[q]));
-            n1[q] = fromw[q] ? w1 : (frome[q] ? e1 : n1[q]);
-            n2[q] = fromw[q] ? w2 : (frome[q] ? e2 : n2[q]);
-          }
-          fb1[q] = fa1[q]; fb2[q] = fa2[q];
-          fa1[q] = F1[q]; fa2[q] = F2[q];
-        } else {
-          const double fo = f[q], v1 = u1[q], v2 = u2[q];
-          double r1, r2;
-          if (PR) {
-            r1 = v1 + a.dtbt * (0.5 * fo * v2 + pf1 + fo1);
-            r2 = v2 + a.dtbt * (-(0.5 * fo * v1) + pf2 + fo2);
-          } else {
-            r1 = v1 + a.dtbt * (0.5 * fo * v2 + pf1 + fo1 + 0.0);
-            r2 = v2 + a.dtbt * (-(0.5 * fo * v1) + pf2 + fo2 + 0.0);
-          }
-          n1[q] = k2[q] * (r1 + k1[q] * r2);
-          n2[q] = k2[q] * (r2 - k1[q] * r1);
-        }
+    for (int q = 0; q < R; ++q) {
+      const double pn = p[q + 1], pne = lane_next(pn);
+      double h1, h2;
+      const double k1q = KL ? s_c[KL ? 4 : 0][q][wave][lane] : k1[q];
+      if constexpr (CG) {    // GRAD_BAROTROPIC_P, C-grid (ocean_operators.F90:664-669)
+        h1 = (pe - p[q]) * g1c[q] * k1q;
+        h2 = (pn - p[q]) * g2c[q] * k2[q];
+      } else {     // B-grid (:651-660), the halves in g1c, g2c
+        const double fay = p[q] + pn, pip = pe + pne, pjp = pn + pne;
+        h1 = (pip - fay) * g1c[q] * um[q];
+        h2 = (pjp - fax) * g2c[q] * um[q];
+        fax = pjp;
       }
-#pragma unroll
-      for (int q = 0; q < 2; ++q) { u1[q] = n1[q]; u2[q] = n2[q]; }
-      // the reads of s_v, s_u1, s_u2 of phases C and A are behind the barrier above
-      share();
+      pe = pne;
+      if (grad0(q)) h1 = h2 = 0.0;
+      const double th1 = s_c[2][q][wave][lane], th2 = CG ? s_c[CG ? 3 : 2][q][wave][lane] : th1;
+      const double fo1 = s_c[0][q][wave][lane], fo2 = s_c[1][q][wave][lane];
+      const double v1 = u1[q], v2 = u2[q];
+      if constexpr (CG) {
+        constexpr double ab0 = 23.0 / 12.0, ab1 = -16.0 / 12.0, ab2 = 5.0 / 12.0;  // :617-619
+        double acc1 = ab0 * F1[q] + ab1 * fa1[q] + ab2 * fb1[q];
+        double acc2 = ab0 * F2[q] + ab1 * fa2[q] + ab2 * fb2[q];
+        if (nocomp(q)) acc1 = acc2 = 0.0;
+        u1[q] = v1 + dtbt * k1q * (acc1 - th1 * h1 + fo1);
+        u2[q] = v2 + dtbt * k2[q] * (acc2 - th2 * h2 + fo2);
+        if (seam) {                         // the halo update of udrho_bt (:3895-3897)
+          u1[q] = update(q, u1[q]);
+          u2[q] = update(q, u2[q]);
+        }
+        fb1[q] = fa1[q]; fb2[q] = fa2[q];
+        fa1[q] = F1[q]; fa2[q] = F2[q];
+      } else {
+        const double r1 = v1 + dtbt * (f[q] * v2 - th1 * h1 + fo1);
+        const double r2 = v2 + dtbt * (-(f[q] * v1) - th2 * h2 + fo2);
+        u1[q] = k2[q] * (r1 + k1[q] * r2);
+        u2[q] = k2[q] * (r2 - k1[q] * r1);
+      }
     }
+    // the reads of S.v, S.u1, S.u2 of phases C and A are behind the barrier above
+    share();
     __syncthreads();
     // C: corrector and time sums
     diverge();
-    const double wgt = (double)(J.nts - itime + 1);
+    const double wgt = J.step_a ? 1.0 : (double)(J.nts - itime + 1);
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const double tmp = PR ? -a.grav * dv[q] : (tmb[q] ? -dv[q] : -dv[q] * 0.0);
-      x[q] = x[q] + a.c_corr * (tmp + sf[q]);
+    for (int q = 0; q < R; ++q) {
+      x[q] = x[q] + a.c_corr * g[q];
       sx[q] = sx[q] + x[q];
-      su1[q] = su1[q] + (J.step_a ? u1[q] : wgt * u1[q]);
-      su2[q] = su2[q] + (J.step_a ? u2[q] : wgt * u2[q]);
+      su1[q] = su1[q] + wgt * u1[q];
+      su2[q] = su2[q] + wgt * u2[q];
     }
   }
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    if (!in[q]) continue;
-    const int o = off[q];
+  for (int q = 0; q < R; ++q) {
+    if (!inside(q)) continue;
+    const int o = col + d.NI * (row0 + q);
     J.xd[o] = x[q];
     J.ud[o] = u1[q];
     J.ud[o + P2] = u2[q];
@@ -577,6 +629,52 @@ __global__ __launch_bounds__(VX *VW) void k_btv_block(BtvArgs<CG, PR> a, BtvBlk 
   }
 }
 
+// rows and wavefronts of a region
+template <bool CG, bool PR>
+__host__ __device__ constexpr int btv_r(bool uni) { return uni && (PR || !CG) ? 3 : 2; }
+template <bool CG, bool PR>
+__host__ __device__ constexpr int btv_nw(bool uni) { return btv_r<CG, PR>(uni) == 3 ? 8 : 16; }
+template <bool CG, bool PR>
+__host__ __device__ constexpr int btv_ry(bool uni) {
+  return btv_r<CG, PR>(uni) * btv_nw<CG, PR>(uni);
+}
+
+template <bool CG, bool PR, bool UNI>
+__global__ __launch_bounds__((VX * btv_nw<CG, PR>(UNI)), 4) void k_btv_block(BtvArgs<CG, PR> a,
+                                                                          BtvBlk J, int per_xcd) {
+  constexpr int R = btv_r<CG, PR>(UNI), NW = btv_nw<CG, PR>(UNI), RY = R * NW;
+  __shared__ BtvLds<CG, PR, R, NW> lds;
+  const int b = blockIdx.x;
+  const int t0 = (b & 7) * per_xcd + (J.rev ? per_xcd - 1 - (b >> 3) : b >> 3);
+  if (t0 >= J.ntiles) return;                  // the whole block
+  const int tile = strip_tile<8>(t0, J.ntx, J.ntiles / J.ntx);
+  const int tx = tile % J.ntx, ty = tile / J.ntx;
+  const KDom &d = a.d;
+  const bool cyc = d.cyclic_x != 0;
+  const int x0 = tx * btv_tx(J.nsub, cyc) - btv_lo(J.nsub, cyc);
+  const int y0 = ty * btv_ty(J.nsub, RY) - btv_lo(J.nsub, false);
+  if (x0 <= 0 || x0 + VX > d.NI - 2 || y0 <= 0 || y0 + RY > d.NJ - 2)
+    btv_tile<CG, PR, R, NW, true, UNI>(a, J, tx, ty, lds);
+  else
+    btv_tile<CG, PR, R, NW, false, UNI>(a, J, tx, ty, lds);
+}
+
+template <bool CG, bool PR>
+int btv_tiles(const KDom &d, bool uni, int h) {
+  const int TX = btv_tx(h, d.cyclic_x != 0), TY = btv_ty(h, btv_ry<CG, PR>(uni));
+  return TY < 1 ? 1 << 30 : ((d.NI + TX - 1) / TX) * ((d.NJ + TY - 1) / TY);
+}
+
+// Rows of scalar constants, where the grid allows it and the lower region of three
+// rows a wavefront keeps enough of an interior (1440x1080 C-grid pressure, 8
+// subcycles a launch: 2.32 ms, 64 x 32 regions 2.45; 10: 5.1 and 3.1; a domain
+// in one round does not mind: 90x60, 10: 186 and 214 us).
+template <bool CG, bool PR>
+bool rows_uniform(const mom_gpu_ctx *ctx, int hsub) {
+  if (!(CG ? ctx->btv_rows_ok : ctx->bt_rows_ok)) return false;
+  return btv_r<CG, PR>(true) == 2 || hsub <= 8 || btv_tiles<CG, PR>(ctx->kd, true, hsub) <= 256;
+}
+
 // nsub = hsub subcycles a launch; the state alternates between two sets of
 // planes of ctx->btv (a region reads its neighbours' points).
 template <bool CG, bool PR>
@@ -588,14 +686,17 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
   unsigned char *mask = (unsigned char *)(w + 7 * P2);    // the place of cori1
   double *xb[2] = {w, w + P2}, *ub[2] = {w + 2 * P2, w + 4 * P2};
   double *fb[2] = {w + 8 * P2, w + 18 * P2};              // 4 planes each: 8-11, 18-21
+  const bool uni = rows_uniform<CG, PR>(ctx, hsub);
+  double *rowc = uni ? w + 7 * P2 + (P2 + 7) / 8 : nullptr;   // behind the masks
   hipLaunchKernelGGL((k_btv_sfmask<CG, PR>), dim3((d.NI + 255) / 256, d.NJ), dim3(256), 0, s, a,
-                     mask);
+                     mask, rowc);
   MOM_LAUNCHED(ctx, "k_btv_sfmask");
-  BtvBlk J{a.xbar_tau, a.ud_tau, nullptr, nullptr, nullptr, nullptr, mask, 1, 0, nts, step_a, 0, 0};
+  BtvBlk J{a.xbar_tau, a.ud_tau, nullptr, nullptr, nullptr, nullptr, mask, rowc, 1, 0, nts, step_a,
+           0, 0, 0};
   const bool cyc = d.cyclic_x != 0;
   for (int which = 0; J.s0 <= nts; J.s0 += hsub, which ^= 1) {
     J.nsub = min(hsub, nts - J.s0 + 1);
-    const int TX = btv_tx(J.nsub, cyc), TY = btv_ty(J.nsub);
+    const int TX = btv_tx(J.nsub, cyc), TY = btv_ty(J.nsub, btv_ry<CG, PR>(uni));
     J.ntx = (d.NI + TX - 1) / TX;
     J.ntiles = J.ntx * ((d.NJ + TY - 1) / TY);
     J.xd = xb[which];
@@ -603,8 +704,12 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
     J.fd = fb[which];
     J.rev = which;
     const int per_xcd = (J.ntiles + 7) / 8;
-    hipLaunchKernelGGL((k_btv_block<CG, PR>), dim3(8 * per_xcd), dim3(VX * VW), 0, s, a, J,
-                       per_xcd);
+    if (uni)
+      hipLaunchKernelGGL((k_btv_block<CG, PR, true>), dim3(8 * per_xcd), 
+                         dim3(VX * btv_nw<CG, PR>(true)), 0, s, a, J, per_xcd);
+    else
+      hipLaunchKernelGGL((k_btv_block<CG, PR, false>), dim3(8 * per_xcd), 
+                         dim3(VX * btv_nw<CG, PR>(false)), 0, s, a, J, per_xcd);
     MOM_LAUNCHED(ctx, "k_btv_block");
     J.xs = J.xd;
     J.us = J.ud;
@@ -613,18 +718,21 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
   return MOM_GPU_OK;
 }
 
-// Subcycles a launch: as set, otherwise the most (at most 12) with at most 128
-// regions, when a launch's time is its latency (90 x 60, 80 subcycles: 296 us at
-// 5, 205 at 12), and 6 above (517 x 389: 331 at 5, 320 at 6, 292 at 7, 433 at 8;
-// 1440 x 1080: 2475, 2257, 2420, 2445).  Results do not depend on it.
+// Subcycles a launch: as set, otherwise the most with one round of regions, when a
+// launch's time is its latency, and 5 or 6 above.  80 subcycles, us alone: scalar
+// rows (two blocks a CU, at most 256 regions, at most 10) 90x60 C-grid pressure 254
+// at 5, 186 at 10; 360x240 256 at 5, 221 at 7, 285 at 8; 517x389 388 at 5, 326
+// at 7, but among three states in turn 184 and 211; 1440x1080 1709 at 5, 1748 at
+// 6.  Other regions (one block a CU, at most 128, at most 12) 90x60 C-grid depth
+// 291 at 5, 203 at 12; 1440x1080 2167 at 5, 1993 at 6, 2119 at 7.  Results do
+// not depend on it.
+template <bool CG, bool PR>
 int blocked_depth(const mom_gpu_ctx *ctx) {
   if (ctx->tune.bt_subcycles_set) return ctx->tune.bt_subcycles_per_launch;
-  const KDom &d = ctx->kd;
-  int h = 12;
-  for (; h > 6; --h) {
-    const int TX = btv_tx(h, d.cyclic_x != 0), TY = btv_ty(h);
-    if (((d.NI + TX - 1) / TX) * ((d.NJ + TY - 1) / TY) <= 128) break;
-  }
+  const bool uni = (CG ? ctx->btv_rows_ok : ctx->bt_rows_ok) && btv_r<CG, PR>(true) == 3;
+  const int most = uni ? 256 : 128, least = uni ? 5 : 6;
+  int h = uni ? 10 : 12;
+  while (h > least && btv_tiles<CG, PR>(ctx->kd, uni, h) > most) --h;
   return h;
 }
 
@@ -722,7 +830,7 @@ int run_variant(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p, const mom_gpu_bt
   a.initsum = p->initsum_with_bar ? 1 : 0;
   hipStream_t s = ctx->stream;
   const dim3 grid((d.NI + 63) / 64, d.NJ), block(64);
-  const int nts = p->nts, hsub = blocked_depth(ctx);
+  const int nts = p->nts, hsub = blocked_depth<CG, PR>(ctx);
   if (hsub > 0 && !d.cyclic_y && (!d.cyclic_x || d.ni >= MIN_NI)) {
     const int rc = run_blocked(ctx, a, nts, p->stepping_a, hsub);
     if (rc) return rc;

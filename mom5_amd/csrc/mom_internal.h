@@ -185,8 +185,9 @@ struct mom_gpu_ctx {
   // and dxu, dyu, datr carry no sign bit: the condition its land path needs
   int bt_grid_ok;
   // dxu, dyu, datr, dxur, dyur and f are the same along every row, bit for bit
-  // (spherical grids): the blocked barotropic takes them from the row
-  int bt_rows_ok;
+  // (spherical grids): the blocked barotropic takes them from the row; its C-grid
+  // variants need dat, dxte and dytn to be so too
+  int bt_rows_ok, btv_rows_ok;
   // REMAP_BT_TO_BU metrics dte, dtw, dus, dun, daur (5 planes, optional)
   double *remap;
   // state of the barotropic variants (22 planes, allocated on first use)

@@ -137,3 +137,44 @@ def test_variant_blocked_bitwise(cyclic, cgrid, press):
                 for name, a, b in zip(("x_bar", "udrho", "conv_rho_ud_t"), got, want):
                     assert np.array_equal(_bits(a), _bits(b)), (name, hsub)
         g.close()
+
+
+# The rows' constants as scalars where the grid does not change along a row (tiles
+# of 64 x 24) and as point values where it does at one point (64 x 32): both the
+# two-launch path's bits, at every depth's tile and the depth chosen from the size.
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("ni,nj,cyclic", [(17, 9, True), (70, 25, False), (190, 131, True)])
+@pytest.mark.parametrize("cgrid,press", [(False, False), (True, False), (False, True),
+                                         (True, True)])
+def test_variant_blocked_uniform_rows(ni, nj, cyclic, cgrid, press, uniform):
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    print(f"[barotropic variant rows {ni}x{nj} cyclic={cyclic} cgrid={cgrid} press={press} "
+          f"uniform={uniform}]", flush=True)
+    kw = {} if cyclic else dict(cyclic_x=False, lat_s=20.0, lat_n=50.0, lon_span=30.0)
+    c = make_case(ni, nj, 3, seed=63, land_frac=0.3, barotropic=True, **kw)
+    for k in ("dxu", "dyu", "dxur", "dyur", "dat", "datr", "dxte", "dytn", "f"):
+        a = c.grid[k]
+        c.grid[k] = np.repeat(a[:, ni // 2:ni // 2 + 1], a.shape[1], axis=1)
+    if not uniform:
+        for k in ("dxur", "dytn"):
+            c.grid[k][nj // 2, ni // 3] *= 1.0 + 2.0 ** -20
+    fl = _inputs(c, cgrid, press, seed=12)
+    H, sh = DeviceArray.from_host, fl["patm"].shape
+    kw = {k: H(v) for k, v in fl.items() if v is not None and k not in ("udrho", "xbar_tau")}
+    xbar, ud, want = H(fl["xbar_tau"]), H(fl["udrho"]), None
+    for hsub in (0, None, 3, 7, 8, 11):
+        g = OceanGPU(c.dom, c.grid)
+        if hsub is not None:
+            g.set_tuning("barotropic_subcycles_per_launch", hsub)
+        out = DeviceArray(sh), DeviceArray((2,) + sh), DeviceArray(sh)
+        g.update_ocean_barotropic_variant(
+            cgrid=cgrid, pressure_based=press, nts=13, dtbt=c.dtbt, x_bar_tau=xbar, udrho_tau=ud,
+            x_bar_taup1=out[0], udrho_taup1=out[1], conv_rho_ud_t=out[2],
+            stepping_a=bool(ni % 2), initsum_with_bar=True, **kw)
+        g.sync()
+        got = [a.to_host() for a in out]
+        g.close()
+        want = want or got
+        for name, a, b in zip(("x_bar", "udrho", "conv_rho_ud_t"), got, want):
+            assert np.array_equal(_bits(a), _bits(b)), (name, hsub)
