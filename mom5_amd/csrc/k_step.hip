@@ -172,8 +172,8 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
   // take other shapes (their halo rows' x and y faces read different rows).
   // With the loads at the level's start two FP64 tracers took 1.75 ms at
   // 1440x1080x50; so, and without branches, 1.50 ms, now bound by vector
-  // instructions: 347 a level and wavefront, issued 82% of the time (ten FP32
-  // tracers: 712, 91%).  The tracers' loads take no branch: a point outside the
+  // instructions: 340 a level and wavefront, issued 82% of the time (ten FP32
+  // tracers: 687).  The tracers' loads take no branch: a point outside the
   // domain reads past the level's end, a 0 (with the branch, and a window kept as
   // four tracers instead of three and a difference, FP32 took 752 instructions
   // and waited for the loads where the loop closes: pass of T, S and six FP32
@@ -634,6 +634,12 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
       const int ry = wave + NW * q;
       const int gj = gjr[q];
       const TT mY2 = mk<TT>(k, ky2[q]), mY1 = mk<TT>(k, ky1[q]), mY0 = mk<TT>(k, ky0[q]);
+      // The neighbouring difference of the upwind side only: from the upwind tracer
+      // to the one beyond it (row ry - 1 or ry + 2, by lane), (T(j) - T(j-1))*mY0 or
+      // (T(j+2) - T(j+1))*mY2; the face's weight carries mY1.  (Both differences
+      // formed and one taken: 347 and 712 instructions; eight FP64 tracers at
+      // 1440x1080x50 9.12 ms, so 8.99.  The same by ds_bpermute in the x sweep: no
+      // gain.)
       if constexpr (!EXACT) {
         // FP32 groups: a row (one wavefront) with no face skips the sweep;
         // within a row no branch, as in the x sweep.  The update reads the
@@ -645,14 +651,13 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
                                   rcpf(((float)cur[q].rs + (float)cur[q].rn) * mdytn[q]));
           const FaceC<float> cyf = face_coef_f(mdxtn[q] * vf, face ? cfl : 0.0f);
           const FaceW wy = face_w(cyf, mY1);
+          const int ou = (wy.pos ? ry - 1 : ry + 2) * RX + lane;
+          const TT mu = wy.pos ? mY0 : -mY2;
 #pragma unroll
           for (int g = 0; g < G; ++g) {
-            const TT tjm1 = s_tx[bb][g][ry - 1][lane], tj = s_tx[bb][g][ry][lane];
-            const TT tjp1 = s_tx[bb][g][ry + 1][lane], tjp2 = s_tx[bb][g][ry + 2][lane];
-            const TT Rjp = (tjp2 - tjp1) * mY2;
-            const TT Rj = tjp1 - tj;   // the face weights carry mY1
-            const TT Rjm = (tj - tjm1) * mY0;
-            s_fy[bb][g][ry][lane] = flux_fast(cyf, wy, Rjm, Rj, Rjp, tj, tjp1);
+            const TT tj = s_tx[bb][g][ry][lane], tjp1 = s_tx[bb][g][ry + 1][lane];
+            const TT Tu = wy.pos ? tj : tjp1;
+            s_fy[bb][g][ry][lane] = flux_up(cyf, wy, (Tu - (&s_tx[bb][g][0][0])[ou]) * mu, tjp1 - tj, Tu);
           }
         }
       } else {
@@ -664,16 +669,15 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
           cy = mdfl64::face(hdxtn[q] * v, mdfl64::cfl_h(v, dtime, rs + rn, hdytn[q]),
                             (double)mY1);
         }
+        const int ou = (cy.pos ? ry - 1 : ry + 2) * RX + lane;
+        const TT mu = cy.pos ? mY0 : -mY2;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
           TT fy = TT(0);
           if (face) {
-            const TT tjm1 = s_tx[bb][g][ry - 1][lane], tj = s_tx[bb][g][ry][lane];
-            const TT tjp1 = s_tx[bb][g][ry + 1][lane], tjp2 = s_tx[bb][g][ry + 2][lane];
-            const TT Rjp = (tjp2 - tjp1) * mY2;
-            const TT Rj = tjp1 - tj;   // the face's weight carries mY1
-            const TT Rjm = (tj - tjm1) * mY0;
-            fy = mdfl64::flux(cy, Rjm, Rj, Rjp, tj, tjp1);
+            const TT tj = s_tx[bb][g][ry][lane], tjp1 = s_tx[bb][g][ry + 1][lane];
+            const TT Tu = cy.pos ? tj : tjp1;
+            fy = mdfl64::flux_up(cy, (Tu - (&s_tx[bb][g][0][0])[ou]) * mu, tjp1 - tj, Tu);
           }
           s_fy[bb][g][ry][lane] = fy;
           fyv[g][q] = fy;

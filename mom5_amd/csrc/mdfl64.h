@@ -87,12 +87,14 @@ __device__ __forceinline__ double psi_s(const Face &f, double Rj, unsigned long 
 // the masked differences, as the reference forms them (a dry face has Rj = 0
 // and a zero weight).  Rjm enters the limiter of the M > 0 term, Rjp that of
 // the M < 0 term.
+// flux_up takes the upwind side's neighbouring difference Rn and tracer Tu.
+__device__ __forceinline__ double flux_up(const Face &f, double Rn, double Rj, double Tu) {
+  const unsigned long long sgn = __builtin_bit_cast(unsigned long long, Rj) & (1ull << 63);
+  return f.wm * (Tu + flip(psi_s(f, Rj, sgn, Rn), sgn ^ f.nsg));
+}
 __device__ __forceinline__ double flux(const Face &f, double Rjm, double Rj, double Rjp,
                                        double Tpos, double Tneg) {
-  const unsigned long long sgn = __builtin_bit_cast(unsigned long long, Rj) & (1ull << 63);
-  const double Rn = f.pos ? Rjm : Rjp;
-  const double Tu = f.pos ? Tpos : Tneg;
-  return f.wm * (Tu + flip(psi_s(f, Rj, sgn, Rn), sgn ^ f.nsg));
+  return flux_up(f, f.pos ? Rjm : Rjp, Rj, f.pos ? Tpos : Tneg);
 }
 
 // Courant numbers: |w*dtime/rho_dzt| of a bottom face (dtr = dtime/rho_dzt)
