@@ -1210,8 +1210,14 @@ int launch_barotropic_blocked(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p,
   const double c_corr = p->dtbt * rho0r;                        // dtbt_rho0r, :1197
   const dim3 grid((d.NI + 255) / 256, d.NJ), block(256);
   const BtBufs w(ctx);
-  // the land path's conditions that do not depend on the data
-  const bool land_ok = ctx->tune.bt_land_tiles && ctx->bt_grid_ok && p->dtbt > 0.0 &&
+  const KDom *const one = &d;
+  const BtPlan plan = bt_plan(&one, 1, ctx->bt_rows_ok, hsub);
+  hsub = plan.hsub;
+  // the land path's conditions that do not depend on the data; with at most one
+  // tile a CU its tiles would only wait for the others, and forming the flags costs
+  // a launch (90x60: 5 us of a step's 154)
+  const bool land_ok = bt_tiles(&one, 1, plan.tile, hsub) > 256 && ctx->tune.bt_land_tiles &&
+                       ctx->bt_grid_ok && p->dtbt > 0.0 &&
                        std::isfinite(c_pred) && std::isfinite(c_corr);
   const Inert inert = land_ok ? Inert{eta_bar_tau, ud_tau, forcing, rho_g, patm, thicku} : Inert{};
   const double *rowc = ctx->bt_rows_ok ? w.rowc : nullptr;
@@ -1225,10 +1231,7 @@ int launch_barotropic_blocked(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p,
   int *landp = land_ok ? w.land : nullptr;
   int land_nsub = 0;
   const int xbase = d.cyclic_x ? 1 : 0, xcount = d.cyclic_x ? d.ni : d.NI;
-  const KDom *const one = &d;
-  const BtPlan plan = bt_plan(&one, 1, rowc != nullptr, hsub);
   const int ry = bt_ry(plan.tile);
-  hsub = plan.hsub;
   const double *eb0 = p->initsum_with_bar ? eta_bar_tau : eta_t;
   const double *eta_src = eta_bar_tau, *ud_src = ud_tau;
   int which = 0;
