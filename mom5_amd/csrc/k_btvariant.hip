@@ -702,7 +702,7 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
     J.xd = xb[which];
     J.ud = ub[which];
     J.fd = fb[which];
-    J.rev = which;
+    J.rev = uni ? which : 0;
     const int per_xcd = (J.ntiles + 7) / 8;
     if (uni)
       hipLaunchKernelGGL((k_btv_block<CG, PR, true>), dim3(8 * per_xcd), 
