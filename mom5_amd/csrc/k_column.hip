@@ -1014,6 +1014,7 @@ void k_vdiff_twin_ens(const VdJobF *__restrict__ jobs, VdLaunch L, int per_xcd) 
 // its level count), so both meet in slot H-1; slots below ph are inert.  A
 // group's tracers share the coefficients' addresses, not their factorisation:
 // each tracer repeats it (the coefficients come from L2 the second time).
+// Tracers n0 .. n1-1 of the job.
 // KK: every tracer of the job has its own K33 (J.k33), loaded with its
 // coefficients; with rho_dzt and dzwt from L2 after the first tracer and K33 a chunk
 // ahead, three tracers with K33 at 1440x1080x50 take 1.83 ms (one job each, K33
@@ -1021,7 +1022,8 @@ void k_vdiff_twin_ens(const VdJobF *__restrict__ jobs, VdLaunch L, int per_xcd) 
 // Wavefront pair threadIdx.x / 128 of a block of NP pairs; a pair whose
 // tile is past the end (live false) runs a valid tile without storing.
 template <int H, int NP, bool KK>
-__device__ __forceinline__ void twin64_tile(const VdJob<double> &J, int tile, bool live = true) {
+__device__ __forceinline__ void twin64_tile(const VdJob<double> &J, int tile, bool live, int n0,
+                                            int n1) {
   __shared__ double xv_all[NP][2][2][64], xq_all[NP][2][2][64];   // [pair][parity][half][column]
   const int pr = NP > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 7) : 0;
   double (*xv)[2][64] = xv_all[pr];
@@ -1045,7 +1047,7 @@ __device__ __forceinline__ void twin64_tile(const VdJob<double> &J, int tile, bo
   const int kb = max(2, kmo);
   const double tda = J.tdt * J.aidif;
   const double rho0 = J.rho0;
-  for (int n = 0; n < J.g.n; ++n) {
+  for (int n = n0; n < n1; ++n) {
     // the tracer's diffusivity plane: its mixing class's diff_cbt
     const double *dcbase = (J.dcbase2 && n >= J.n2) ? J.dcbase2 : J.dcbase;
     const double *k33 = J.k33[n];
@@ -1210,7 +1212,9 @@ void k_vdiff_twin64(VdJob<double> J, int per_xcd) {
   const int t0 = 2 * ((b & 7) * per_xcd + (b >> 3));
   if (t0 >= J.nblocks) return;               // the whole block
   const int tile = t0 + (threadIdx.x >> 7);
-  twin64_tile<H, 2, KK>(J, min(tile, J.nblocks - 1), tile < J.nblocks);
+  const bool one = gridDim.y > 1;            // a tracer a block
+  twin64_tile<H, 2, KK>(J, min(tile, J.nblocks - 1), tile < J.nblocks, one ? blockIdx.y : 0,
+                        one ? blockIdx.y + 1 : J.g.n);
 }
 
 // Several FP64 tracers of one mixing class: k_vdiff_twin64's elimination with the
@@ -1430,7 +1434,7 @@ void k_vdiff_twin64_ens(const VdJob<double> *__restrict__ jobs, VdLaunch L, int 
   int lo, tile;
   if (!vd_pair(L, per_xcd, lo, tile)) return;
   const VdJob<double> &J = jobs[lo];
-  twin64_tile<H, 2, false>(J, min(tile, J.nblocks - 1), tile < J.nblocks);
+  twin64_tile<H, 2, false>(J, min(tile, J.nblocks - 1), tile < J.nblocks, 0, J.g.n);
 }
 
 __global__ void k_set_ints(int *__restrict__ p, int v, int n) {
@@ -2001,7 +2005,11 @@ static void with_slots(int h, F &&f) {
 static void launch_twin64(mom_gpu_ctx *ctx, VdJob<double> J, bool kk) {
   const KDom &d = J.d;
   const int per_xcd = ((J.nblocks + 1) / 2 + 7) / 8;   // tile pairs per XCD
-  const dim3 grid(8 * per_xcd), block(256);
+  // A small domain's tracers go to blocks of their own while all take one round (two
+  // blocks a CU): step of T and S at 90x60x25 alone 151 us, so 144; among three
+  // states 56.1 and 53.2
+  const int ny = 8 * per_xcd * J.g.n <= 512 ? J.g.n : 1;
+  const dim3 grid(8 * per_xcd, ny), block(256);
   with_slots(twin_slots(d.nk), [&](auto H) {
     if (kk)
       hipLaunchKernelGGL((k_vdiff_twin64<H.value, true>), grid, block, 0, ctx->stream, J, per_xcd);

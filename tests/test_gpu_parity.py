@@ -327,6 +327,35 @@ def test_vert_diffuse_implicit_own_k33(nk):
     gpu.close()
 
 
+@pytest.mark.parametrize("ni,nj", [(70, 9), (130, 170), (130, 171), (300, 240)])
+@pytest.mark.parametrize("k33", [False, True])
+def test_vert_diffuse_implicit_tracers_by_block(ni, nj, k33):
+    """T and S of a small domain are solved by blocks of their own, of a larger
+    one by the same block: either way each tracer is, bit for bit, what it is
+    alone (sizes either side of the rule's line)."""
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    print(f"[tracers by block {ni}x{nj} k33={k33}]", flush=True)
+    case = make_case(ni, nj, 6, land_frac=0.3, seed=ni, barotropic=False, stf_scale=1e-3)
+    gpu, f, H = OceanGPU(case.dom, case.grid), case.fields, DeviceArray.from_host
+    Ts = [t for _, t in case.tracers][:2]
+    K = H(1e-2 * np.random.default_rng(nj).random(Ts[0].shape))
+    rho, dzwt, mix = H(f["rho_dzt"]), H(f["dzwt"]), H(f["diff_cbt"])
+
+    def run(ns, salt):
+        d = [H(Ts[n]) for n in ns]
+        gpu.vert_diffuse_implicit(d, [H(f["stf"][n]) for n in ns], [H(f["btf"][n]) for n in ns],
+                                  mix, rho, dzwt, case.dt, index_salt=salt,
+                                  K33s=[K] * len(d) if k33 else None)
+        gpu.sync()
+        return [x.to_host() for x in d]
+
+    both = run([0, 1], 1)
+    same(both[0], run([0], -1)[0])
+    same(both[1], run([1], 0)[0])
+    gpu.close()
+
+
 @pytest.mark.parametrize("per_launch", [0, 1, 4, 7, 12])
 @pytest.mark.parametrize("stepping_a,initsum", [(False, True), (True, False)])
 def test_update_ocean_barotropic(setup, stepping_a, initsum, per_launch):
