@@ -134,7 +134,11 @@ struct StepJob {
 constexpr int TENDENCY = 2;
 template <typename TT, int G, int RPW>
 constexpr bool both_th() { return sizeof(TT) == 8 && RPW == 1 && G <= 2; }
-template <typename TT, int G, int RPW, int NW, int TH>
+// CY (one-row shapes): the domain is cyclic in y, whose halo rows' x faces read the
+// rows they mirror and whose y faces the halo rows themselves: one load a level
+// more (step of T and S at 1440x1080x50 2.69 ms, others 2.59; by two rows a
+// wavefront 3.53; T, S and ten FP32 at 720x540x50 2.06, 2.05 and 3.25).
+template <typename TT, int G, int RPW, int NW, int TH, bool CY>
 __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka, int kb) {
   const KDom d = J.d;
   const StepTab<TT> &tab = J.tab;
@@ -168,8 +172,8 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
   // it.  What makes room for them: the rho_dzt of the faces is one value a point
   // (at its own place in the data domain, halo included), the other sides of
   // the east and north faces come from the next lane and, through LDS, the next
-  // row; five loads of rho_dzt a level become two.  Domains that are cyclic in y
-  // take other shapes (their halo rows' x and y faces read different rows).
+  // row; five loads of rho_dzt a level become two, three where the halo rows' x
+  // and y faces read different rows (CY).
   // With the loads at the level's start two FP64 tracers took 1.75 ms at
   // 1440x1080x50; so, and without branches, 1.50 ms, now bound by vector
   // instructions: 340 a level and wavefront, issued 82% of the time (ten FP32
@@ -335,18 +339,21 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
   const double *Rx = Rr ? Rr : R;
   // PRE shapes: the next level's inputs (nh: rho_dzt at the point's own place;
   // nm, nx: the update's)
-  double nw[RPW], nr[RPW], nu[RPW], nh[RPW], nv[RPW], nm[RPW], nx[RPW];
-  unsigned bh[RPW];
+  // (CY: nhx is the one of the row the x faces read)
+  double nw[RPW], nr[RPW], nu[RPW], nh[RPW], nhx[RPW], nv[RPW], nm[RPW], nx[RPW];
+  unsigned bh[RPW], bhx[RPW];
   if constexpr (PRE) {
 #pragma unroll
     for (int q = 0; q < RPW; ++q) {
       bh[q] = gi >= -1 && gi <= d.ni && gjr[q] >= -1 && gjr[q] <= d.nj
                   ? (unsigned)d2(d, gi, gjr[q]) * 8u : 0u;
+      if constexpr (CY) bhx[q] = gi >= -1 && gi <= d.ni ? (unsigned)d2(d, gi, sjr[q]) * 8u : 0u;
       const size_t pa = (size_t)P2 * (ka - 1);
       nw[q] = ld_lv(W + P2 + pa, bz[q]);
       nr[q] = ld_lv(R + pa, bz[q]);
       nu[q] = ld_lv(U + pa, bx[q]);
       nh[q] = ld_lv(R + pa, bh[q]);
+      if constexpr (CY) nhx[q] = ld_lv(R + pa, bhx[q]);
       nv[q] = ld_lv(V + pa, by[q]);
     }
   }
@@ -501,9 +508,9 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
         nr[q] = ld_lv(R + pr, bz[q]);
         // the x and y faces of this level
         cur[q].u = nu[q];
-        cur[q].rw = nh[q];
+        cur[q].rw = CY ? nhx[q] : nh[q];
         cur[q].v = nv[q];
-        if constexpr (EXACT) cur[q].re = lane_next(nh[q]);
+        if constexpr (EXACT) cur[q].re = lane_next(cur[q].rw);
         s_r[bb][wave + NW * q][lane] = (TT)nh[q];
       }
     }
@@ -594,6 +601,7 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
       for (int q = 0; q < RPW; ++q) {
         nu[q] = ld_lv(U + pr, bx[q]);
         nh[q] = ld_lv(R + pr, bh[q]);
+        if constexpr (CY) nhx[q] = ld_lv(R + pr, bhx[q]);
       }
     }
     __syncthreads();
@@ -814,7 +822,7 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
 }
 
 
-template <typename TT, int G, int RPW, int NW, int TH>
+template <typename TT, int G, int RPW, int NW, int TH, bool CY>
 __global__ __launch_bounds__(RX * NW) void k_step(StepJob<TT> J, int per_xcd) {
   const int b = blockIdx.x;
   // XCD-aware: each XCD takes per_xcd consecutive positions of the order of
@@ -822,15 +830,15 @@ __global__ __launch_bounds__(RX * NW) void k_step(StepJob<TT> J, int per_xcd) {
   const int t = (b & 7) * per_xcd + (b >> 3);
   if (t >= J.ntiles * J.nchunk) return;
   const int c = t % J.nchunk, nk = J.d.nk;
-  step_tile<TT, G, RPW, NW, TH>(J, strip_tile<8>(t / J.nchunk, J.ntx, J.ntiles / J.ntx),
-                                nk * c / J.nchunk + 1, nk * (c + 1) / J.nchunk);
+  step_tile<TT, G, RPW, NW, TH, CY>(J, strip_tile<8>(t / J.nchunk, J.ntx, J.ntiles / J.ntx),
+                                    nk * c / J.nchunk + 1, nk * (c + 1) / J.nchunk);
 }
 
 // Ensemble pass: a persistent grid takes (job, tile) items from a device-side
 // counter in order (jobs sorted largest first) until none is left.  first[j]
 // is the index of job j's first item; total = sum of the jobs' tiles.  Every
 // block leaves the loop once the counter passes total.
-template <typename TT, int G, int RPW, int NW, int TH>
+template <typename TT, int G, int RPW, int NW, int TH, bool CY>
 __global__ __launch_bounds__(RX * NW) void k_step_queue(const StepJob<TT> *__restrict__ jobs,
                                                         const int *__restrict__ first, int njobs,
                                                         int total, int *__restrict__ counter) {
@@ -846,7 +854,7 @@ __global__ __launch_bounds__(RX * NW) void k_step_queue(const StepJob<TT> *__res
       const int mid = (lo + hi + 1) >> 1;
       if (first[mid] <= item) lo = mid; else hi = mid - 1;
     }
-    step_tile<TT, G, RPW, NW, TH>(jobs[lo], item - first[lo], 1, jobs[lo].d.nk);
+    step_tile<TT, G, RPW, NW, TH, CY>(jobs[lo], item - first[lo], 1, jobs[lo].d.nk);
   }
 }
 
@@ -862,10 +870,8 @@ struct Shape {
   int rpw, nw;
 };
 
-// cyc_y: a domain cyclic in y, which one-row shapes do not take
 template <typename TT>
-static Shape shape_of(int rpw, int waves, bool cyc_y) {
-  if (cyc_y && rpw == 1) return {2, 8};
+static Shape shape_of(int rpw, int waves) {
   if (sizeof(TT) == 4) {
     if (rpw == 1 && waves == 16) return {1, 16};
     if (rpw == 2 && waves == 16) return {2, 16};
@@ -995,6 +1001,24 @@ static bool any_th(const StepTab<TT> &t, int n) {
   return false;
 }
 
+// f(TH, CY) as constants, for the instances that a shape has.
+template <typename TT, int G, int RPW, typename F>
+static void with_instance(bool th, bool cyc_y, F &&f) {
+  using Yes = std::true_type;
+  using No = std::false_type;
+  auto pick = [&](auto cy) {
+    if constexpr (both_th<TT, G, RPW>()) {
+      if (!th) return f(No{}, cy);
+    }
+    f(Yes{}, cy);
+  };
+  // (four FP64 tracers load both rows' rho_dzt in either case)
+  if constexpr (RPW == 1 && (sizeof(TT) == 4 || G <= 2)) {
+    if (cyc_y) return pick(Yes{});
+  }
+  pick(No{});
+}
+
 template <typename TT>
 struct GroupLaunch {
   mom_gpu_ctx *ctx;
@@ -1014,12 +1038,10 @@ struct GroupLaunch {
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(8 * per), dim3(RX * NW), 0, ctx->stream, J, per);
     };
-    if constexpr (both_th<TT, G, RPW>()) {
-      if (any_th(tab, G)) go(k_step<TT, G, RPW, NW, true>);
-      else go(k_step<TT, G, RPW, NW, false>);
-    } else {
-      go(k_step<TT, G, RPW, NW, true>);
-    }
+    const bool th = !both_th<TT, G, RPW>() || any_th(tab, G);
+    with_instance<TT, G, RPW>(th, d.cyclic_y != 0, [&](auto th_, auto cy) {
+      go(k_step<TT, G, RPW, NW, th_.value, cy.value>);
+    });
     return MOM_GPU_OK;
   }
 };
@@ -1030,7 +1052,7 @@ static void launch_all(mom_gpu_ctx *ctx, int gmax, int rpw, int waves, int ntr,
                        const double *const *th_in, int want, const double *u, const double *v,
                        const double *w, const double *rho, const double *rm1, const double *rr,
                        double dtime) {
-  const Shape sh = shape_of<TT>(rpw, waves, ctx->kd.cyclic_y != 0);
+  const Shape sh = shape_of<TT>(rpw, waves);
   std::vector<int> idx;
   for (int n = 0; n < ntr; ++n)
     if (dtype[n] == want) idx.push_back(n);
@@ -1086,12 +1108,9 @@ static int queue_launch(mom_gpu_ensemble *e, std::vector<StepJob<TT>> &jobs, int
   };
   bool th = !both_th<TT, G, RPW>();
   for (const StepJob<TT> &J : jobs) th = th || any_th(J.tab, G);
-  if constexpr (both_th<TT, G, RPW>()) {
-    if (th) go(k_step_queue<TT, G, RPW, NW, true>);
-    else go(k_step_queue<TT, G, RPW, NW, false>);
-  } else {
-    go(k_step_queue<TT, G, RPW, NW, true>);
-  }
+  with_instance<TT, G, RPW>(th, jobs[0].d.cyclic_y != 0, [&](auto th_, auto cy) {
+    go(k_step_queue<TT, G, RPW, NW, th_.value, cy.value>);
+  });
   MOM_LAUNCHED(e->lead, "k_step_queue");
   return MOM_GPU_OK;
 }
@@ -1108,12 +1127,11 @@ struct QueueLaunch {
 template <typename TT>
 static int ensemble_type(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *steps, int want,
                          int gmax, int rpw, int waves, int &slot) {
-  // jobs bucketed by group size (the shape's sizes no larger than gmax), per domain
-  bool cyc_y = false;
-  for (const mom_gpu_ctx *c : e->ctx) cyc_y = cyc_y || c->kd.cyclic_y;
-  const Shape sh = shape_of<TT>(rpw, waves, cyc_y);
+  // jobs bucketed by group size (the shape's sizes no larger than gmax), per domain,
+  // and, where the kernels differ (one-row shapes), by whether it is cyclic in y
+  const Shape sh = shape_of<TT>(rpw, waves);
   constexpr int GMAX = 12;
-  std::vector<StepJob<TT>> by[GMAX + 1];
+  std::vector<StepJob<TT>> by[2][GMAX + 1];
   const int TY = sh.nw * sh.rpw - 4;
   for (size_t dd = 0; dd < e->ctx.size(); ++dd) {
     mom_gpu_ctx *ctx = e->ctx[dd];
@@ -1135,8 +1153,9 @@ static int ensemble_type(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *steps
       }
       const int ntx = (d.ni + TX - 1) / TX;
       const int ntiles = ntx * ((d.nj + TY - 1) / TY);
-      by[c].emplace_back();
-      StepJob<TT> &J = by[c].back();
+      std::vector<StepJob<TT>> &jobs = by[sh.rpw == 1 && d.cyclic_y ? 1 : 0][c];
+      jobs.emplace_back();
+      StepJob<TT> &J = jobs.back();
       std::memset((void *)&J, 0, sizeof J);
       J.d = d;
       J.tab = t;
@@ -1149,8 +1168,9 @@ static int ensemble_type(mom_gpu_ensemble *e, const mom_gpu_tracer_step_t *steps
     }
   }
   int rc = MOM_GPU_OK;
-  for (const int *g = group_sizes<TT>(sh); *g && rc == MOM_GPU_OK; ++g)
-    if (!by[*g].empty()) rc = with_shape<TT>(*g, sh, QueueLaunch<TT>{e, by[*g], slot++});
+  for (auto &cyc : by)
+    for (const int *g = group_sizes<TT>(sh); *g && rc == MOM_GPU_OK; ++g)
+      if (!cyc[*g].empty()) rc = with_shape<TT>(*g, sh, QueueLaunch<TT>{e, cyc[*g], slot++});
   if (rc || sizeof(TT) == 8) return rc;
   bool added = false;
   for (size_t dd = 0; dd < e->ctx.size(); ++dd) {
@@ -1182,7 +1202,7 @@ int launch_mdfl_tendency(mom_gpu_ctx *ctx, const double *T, const double *u, con
   const StepJob<double> J{d, tab, u, v, w, rho, nullptr, nullptr, ctx->kmt, ctx->dat, ctx->datr,
                           ctx->dxte, ctx->dyte, ctx->dxtn, ctx->dytn, dtime, ntx, ntiles,
                           chunks};
-  hipLaunchKernelGGL((k_step<double, 1, 1, NW, TENDENCY>), dim3(8 * per), dim3(RX * NW), 0,
+  hipLaunchKernelGGL((k_step<double, 1, 1, NW, TENDENCY, false>), dim3(8 * per), dim3(RX * NW), 0,
                      ctx->stream, J, per);
   MOM_LAUNCHED(ctx, "k_step (tendency)");
   return MOM_GPU_OK;

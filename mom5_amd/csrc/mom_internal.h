@@ -341,7 +341,7 @@ struct mom_gpu_ensemble {
   std::vector<mom_gpu_ctx *> ctx;   // not owned; ctx[0] is the lead (stream, errors)
   mom_gpu_ctx *lead = nullptr;
   int *counters = nullptr;          // device work-queue counters
-  static constexpr int NCOUNT = 16;
+  static constexpr int NCOUNT = 32;   // one a queue launch: at most 18 a step
   TableCache<void *> tables;        // launch tables, shared by content
 };
 

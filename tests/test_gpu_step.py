@@ -470,3 +470,56 @@ def test_shared_factorisation_equals_single_tracers(nk):
             g.sync()
             assert np.array_equal(group[n].to_host(), one.to_host()), (ntr, n)
     g.close()
+
+
+def _case_on(cyc_y, ni, nj, nk, n_passive, seed):
+    from mom5_amd import OceanGPU
+    from mom5_amd.synth import make_case
+    case = make_case(ni, nj, nk, land_frac=0.2, seed=seed, n_passive=n_passive, barotropic=False)
+    return case, OceanGPU(dict(case.dom, cyclic_y=int(cyc_y)), case.grid)
+
+
+def test_cyclic_y_domains_take_the_same_passes():
+    """A domain cyclic in y is advanced by as many passes as another one: T and S
+    in one, ten FP32 tracers in one (counted as the nodes of a captured step)."""
+    nodes = []
+    for cyc_y in (0, 1):
+        case, g = _case_on(cyc_y, 70, 30, 5, 10, 91)
+        print(f"[passes of 2 FP64 + 10 FP32, cyclic_y={cyc_y}]", flush=True)
+        from mom5_amd.step import BatchedStep
+        dt = [np.float64] * 2 + [np.float32] * 10
+        st = BatchedStep(case, gpu=g, diffuse=False, barotropic=False, tracers=[
+            (nm, np.asarray(t, d)) for (nm, t), d in zip(case.tracers, dt)])
+        graph = st.capture(2)
+        nodes.append(graph.nodes)
+        graph.close()
+        g.close()
+    assert nodes == [4, 4]          # two steps of two passes each
+
+
+def test_ensemble_with_a_cyclic_y_member():
+    """Members cyclic in y beside others: each equals itself stepped alone, bit
+    for bit, FP64 and FP32, with a remainder of FP32 groups."""
+    from mom5_amd.ensemble import EnsembleStep
+    from mom5_amd.step import BatchedStep
+    shapes = [(0, 70, 30, 5), (1, 61, 25, 6), (0, 125, 13, 4), (1, 33, 40, 7)]
+    print(f"[ensemble with cyclic_y members {shapes}]", flush=True)
+    dt = [np.float64] * 3 + [np.float32] * 7
+    alone, together = [], []
+    for n, (cyc_y, ni, nj, nk) in enumerate(shapes):
+        case, g = _case_on(cyc_y, ni, nj, nk, 8, 92 + n)
+        for members in (alone, together):
+            members.append(BatchedStep(case, gpu=g, diffuse=False, barotropic=False, tracers=[
+                (nm, np.asarray(t, d)) for (nm, t), d in zip(case.tracers, dt)]))
+    for m in alone:
+        m.run(3)
+        m.gpu.sync()
+    ens = EnsembleStep(together)
+    ens.run(3)
+    ens.gpu.sync()
+    for k, (a, b) in enumerate(zip(alone, together)):
+        for n in range(a.ntr):
+            x, y = a.tracer(n).to_host(), b.tracer(n).to_host()
+            assert np.isfinite(x).all(), (k, n)
+            assert np.array_equal(x, y), (k, n)
+    ens.close()
