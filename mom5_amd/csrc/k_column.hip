@@ -1231,6 +1231,7 @@ void k_vdiff_twin64(VdJob<double> J, int per_xcd) {
 // One tile (64 columns, two wavefronts) a block: the factors of two tiles fill a
 // CU's LDS at 76 levels.  (Two tiles a block: the same within 4%.)
 constexpr int SHARE_NT = 32;
+constexpr int SHARE_NK = 76;   // levels at which two blocks still share a CU
 struct ShareJob {
   KDom d;
   double *z[SHARE_NT];
@@ -1764,8 +1765,11 @@ static int twin64_groups(mom_gpu_ctx *ctx, int ntr, void *const *T, const int *d
   // alone).  With two the one factorisation saved is what fewer wavefronts in
   // flight cost: T, S and one more tracer at 1440x1080, 41 levels 1.49 ms with
   // k_vdiff_twin64 against 1.57, 50 levels 1.84 against 1.75; with two more 2.46
-  // against 2.04 at 50 levels.
-  if (c1.size() >= 3) {
+  // against 2.04 at 50 levels.  Above SHARE_NK levels the factors leave room for one
+  // block of two wavefronts a CU: three tracers and salt at 1000x750, 76 levels
+  // 1.64 ms with k_vdiff_twin64 and 1.45 so, 77 levels 1.67 and 2.57; eight and
+  // salt, 77 levels 3.68 and 4.30.
+  if (c1.size() >= 3 && d.nk <= SHARE_NK) {
     for (size_t at = 0; at < all.size(); at += SHARE_NT) {
       ShareJob J{};
       J.d = d; J.dcb[0] = diff_cbt; J.dcb[1] = diff_cbt + p3; J.rho0 = rho0; J.kmt = ctx->kmt;
@@ -2030,8 +2034,7 @@ static void launch_share(mom_gpu_ctx *ctx, const ShareJob &J) {
   else if (h <= 25) go(k_vdiff_share<25>);
   else if (h <= 30) go(k_vdiff_share<30>);
   else if (h <= 34) go(k_vdiff_share<34>);
-  else if (h <= 38) go(k_vdiff_share<38>);
-  else go(k_vdiff_share<40>);
+  else go(k_vdiff_share<(SHARE_NK + 1) / 2>);
 }
 
 static void launch_twin(mom_gpu_ctx *ctx, VdJobF J) {

@@ -523,3 +523,24 @@ def test_ensemble_with_a_cyclic_y_member():
             assert np.isfinite(x).all(), (k, n)
             assert np.array_equal(x, y), (k, n)
     ens.close()
+
+
+@pytest.mark.parametrize("nk,launches", [(76, 1), (77, 2), (80, 2)])
+def test_shared_factorisation_ends_where_one_block_fills_a_cu(nk, launches):
+    """Nine FP64 tracers share one factorisation (one launch) up to 76 levels; with
+    more its LDS would hold one block a CU and the solver of eight a launch, two a
+    CU, is the faster one."""
+    from mom5_amd import DeviceArray
+    case, g = _case_on(0, 40, 9, nk, 7, 97)
+    print(f"[nine FP64 tracers, {nk} levels]", flush=True)
+    H, f = DeviceArray.from_host, case.fields
+    T = [H(np.asarray(t, np.float64)) for _, t in case.tracers]
+    st = H(np.zeros(T[0].shape[1:]))
+    dcb, rho, dzwt = H(f["diff_cbt"]), H(f["rho_dzt"]), H(f["dzwt"])
+    g.sync()
+    g.graph_begin()
+    g.vert_diffuse_implicit(T, [st] * 9, [st] * 9, dcb, rho, dzwt, 1800.0, index_salt=1)
+    graph = g.graph_end()
+    assert graph.nodes == launches
+    graph.close()
+    g.close()
