@@ -1452,15 +1452,18 @@ struct LimTable {
   int n;
 };
 
-// A thread takes LIM_NK levels of one point, tracer after tracer, with the level
+// A thread takes lev levels of one point, tracer after tracer, with the level
 // below carried from one level to the next and a level's loads issued before
 // the level above is written: HBM reads each tracer once (a thread per point
 // and level read it again for the level above).  Three tracers at 1440x1080x50:
-// 1.09 to 0.95 ms (six planes, 3.9 TB/s; two levels ahead 1.00).
-constexpr int LIM_NK = 10;
+// 1.09 to 0.95 ms (six planes, 3.9 TB/s; two levels ahead 1.00, ten levels a thread
+// 0.97).  Small domains take fewer levels a thread, down to one, so that the chip
+// holds every point at once (about 2048 blocks): a chain of ten levels costs 90x60x25
+// 11.5 us instead of 6.3, 180x120x30 15.3 instead of 8.9 (two levels).
+constexpr int LIM_NK = 5;
 __global__ __launch_bounds__(256) void k_tmask_limit(KDom d, LimTable t, int it, int is,
                                                      int ts_same, const int *__restrict__ kmt,
-                                                     int ntx, int ntiles, int per_xcd) {
+                                                     int lev, int ntx, int ntiles, int per_xcd) {
   // 64 x 4 points a work-group, neighbouring tiles on one XCD
   const int b = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (b >= ntiles) return;
@@ -1468,7 +1471,7 @@ __global__ __launch_bounds__(256) void k_tmask_limit(KDom d, LimTable t, int it,
   const int gi = (tile % ntx) * 64 + threadIdx.x - 1;
   const int gj = (tile / ntx) * 4 + threadIdx.y - 1;
   if (gi > d.ni - 1 || gj > d.nj - 1) return;
-  const int k1 = blockIdx.y * LIM_NK + 1, k2 = min(k1 + LIM_NK - 1, d.nk);
+  const int k1 = blockIdx.y * lev + 1, k2 = min(k1 + lev - 1, d.nk);
   const int o = d2(d, gi, gj);
   const size_t P2 = (size_t)d.P2;
   const int km = kmt[o], ke = kmt[o + 1], kn = kmt[o + d.NI];
@@ -2116,8 +2119,10 @@ int launch_tmask_limit(mom_gpu_ctx *ctx, int ntr, const double *const *T, const 
   // i in isc-1..iec, j in jsc-1..jec
   const int ntx = (d.ni + 1 + 63) / 64, ntiles = ntx * ((d.nj + 1 + 3) / 4);
   const int per_xcd = (ntiles + 7) / 8;
-  hipLaunchKernelGGL(k_tmask_limit, dim3(8 * per_xcd, (d.nk + LIM_NK - 1) / LIM_NK), dim3(64, 4),
-                     0, ctx->stream, d, t, it, is, ts_same, ctx->kmt, ntx, ntiles, per_xcd);
+  const long long one = (long long)ntiles * d.nk;       // blocks at a level a thread
+  const int lev = (int)std::min((long long)LIM_NK, (one + 2047) / 2048);
+  hipLaunchKernelGGL(k_tmask_limit, dim3(8 * per_xcd, (d.nk + lev - 1) / lev), dim3(64, 4), 0,
+                     ctx->stream, d, t, it, is, ts_same, ctx->kmt, lev, ntx, ntiles, per_xcd);
   MOM_LAUNCHED(ctx, "k_tmask_limit");
   return MOM_GPU_OK;
 }

@@ -552,3 +552,24 @@ def test_tracer_content(setup):
         ref = orc.tracer_content(T)
         got = gpu.tracer_content(DeviceArray.from_host(T), dev["rho_dzt"])
         assert abs(got - ref) <= 1e-15 * abs(ref), (got, ref)
+
+
+@pytest.mark.parametrize("ni,nj,nk", [(90, 60, 25), (180, 120, 30), (240, 160, 27), (240, 160, 37),
+                                      (300, 200, 41)])
+def test_tmask_limit_levels_a_thread(oracle_lib, ni, nj, nk):
+    """The limiter masks at each count of levels a thread takes (1 to 5, by size; the
+    last ones do not divide nk) equal the CPU restatement, flags of T and S
+    OR'ed."""
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    print(f"[limiter masks {ni}x{nj}x{nk}]", flush=True)
+    case = make_case(ni, nj, nk, land_frac=0.2, seed=ni + nk, barotropic=False)
+    orc, gpu = oracle_lib.Oracle(case), OceanGPU(case.dom, case.grid)
+    Ts = [t for _, t in case.tracers]
+    lo, hi = [float(np.quantile(t, 0.1)) for t in Ts], [float(np.quantile(t, 0.9)) for t in Ts]
+    outs = [gpu.field3() for _ in Ts]
+    gpu.compute_tmask_limit([DeviceArray.from_host(t) for t in Ts], lo, hi, outs, 0, 1, True)
+    gpu.sync()
+    for a, b in zip(outs, orc.tmask_limit(Ts, lo, hi, 0, 1, True)):
+        same(a.to_host(), b)
+    gpu.close()
