@@ -113,10 +113,15 @@ int mom_gpu_copy(mom_gpu_ctx_t *ctx, double *dst, const double *src, size_t n);
 /* Launch-shape knobs, set per context (the autotuner, mom5_amd/tune.py,
  * drives these; results do not depend on them, bit for bit, except FP32
  * results on vdiff_solver).  Knobs:
- *   "barotropic_subcycles_per_launch"  0: three launches per subcycle (two for
- *                                      the variants); n>0: n subcycles per
- *                                      launch (1..12).  Until it is set (5 is
- *                                      read back) it is chosen from the size
+ *   "barotropic_subcycles_per_launch"  -1: chosen from the size, call by call;
+ *                                      0: three launches per subcycle (two for
+ *                                      the variants, four subcycles a launch for
+ *                                      ensembles); n>0: n subcycles per
+ *                                      launch (1..12; the variants: at most n,
+ *                                      and no more than they would choose)
+ *   "barotropic_subcycles_used"        read only: subcycles a launch of the
+ *                                      context's last barotropic call (0: one
+ *                                      launch per phase; -1: no call yet)
  *   "mdfl_rows_per_wave"               1, 2 or 4: rows a wavefront of the MDFL kernel
  *                                      (16 wavefronts with 1 row, 8 otherwise)
  *   "step_group_f64"                   1, 2 or 4 FP64 tracers per batched pass
@@ -177,7 +182,8 @@ int mom_gpu_copy(mom_gpu_ctx_t *ctx, double *dst, const double *src, size_t n);
  *                                      included, while the ocean's state
  *                                      stays finite)
  * Defaults (the fastest measured at 3600x2700x75 with T, S and ten FP32
- * tracers): 5, 1, 2, 10, 1, 1, 16, 16, 1, 256, 0, 1, 1, 1 in the order above.  Unknown knobs and
+ * tracers): -1, 1, 2, 10, 1, 1, 16, 16, 1, 256, 0, 1, 1, 1 in the order above
+ * (those that can be set).  Unknown knobs and
  * out-of-range values return MOM_GPU_ERR_ARG. */
 int mom_gpu_set_tuning(mom_gpu_ctx_t *ctx, const char *knob, int value);
 int mom_gpu_get_tuning(const mom_gpu_ctx_t *ctx, const char *knob, int *value);

@@ -1214,6 +1214,7 @@ int launch_barotropic_blocked(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p,
   const KDom *const one = &d;
   const BtPlan plan = bt_plan(&one, 1, ctx->bt_rows_ok, hsub);
   hsub = plan.hsub;
+  ctx->bt_subcycles_used = hsub;
   // the land path's conditions that do not depend on the data; with at most one
   // tile a CU its tiles would only wait for the others, and forming the flags costs
   // a launch (90x60: 5 us of a step's 154)
@@ -1276,10 +1277,12 @@ int launch_barotropic(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p, const doub
                       const double *thicku, const double *patm, const double *pme,
                       const double *river, const double *source, const double *eta_smooth,
                       const double *rho_g, double *eta_bar, double *ud, double *conv) {
-  if (ctx->tune.bt_subcycles_per_launch > 0)
+  const int knob = ctx->tune.bt_subcycles_per_launch;
+  if (knob != 0)
     return launch_barotropic_blocked(ctx, p, eta_t, eta_bar_tau, ud_tau, forcing, thicku, patm,
                                      pme, river, source, eta_smooth, rho_g, eta_bar, ud, conv,
-                                     ctx->tune.bt_subcycles_set ? ctx->tune.bt_subcycles_per_launch : 0);
+                                     std::max(knob, 0));
+  ctx->bt_subcycles_used = 0;
   const KDom &d = ctx->kd;
   const size_t P2 = (size_t)d.P2;
   BtBuf b;
@@ -1332,9 +1335,8 @@ int launch_barotropic_ensemble(mom_gpu_ensemble *e, const mom_gpu_bt_params_t *p
                                const mom_gpu_bt_fields_t *f) {
   const int nd = (int)e->ctx.size();
   if (nd > BT_MAXDOM) return mom_fail(e->lead, MOM_GPU_ERR_ARG, "ensemble: too many domains");
-  const auto &tune = e->lead->tune;
-  int hsub = !tune.bt_subcycles_set ? 0
-             : tune.bt_subcycles_per_launch > 0 ? tune.bt_subcycles_per_launch : 4;
+  const int knob = e->lead->tune.bt_subcycles_per_launch;
+  int hsub = knob < 0 ? 0 : knob > 0 ? knob : 4;
   std::vector<BtDom> doms(nd);
   std::vector<BtTail> tails(nd);
   std::vector<BtPrep> preps(nd);
@@ -1350,6 +1352,7 @@ int launch_barotropic_ensemble(mom_gpu_ensemble *e, const mom_gpu_bt_params_t *p
   }
   const BtPlan plan = bt_plan(kds.data(), nd, rows, hsub);
   hsub = plan.hsub;
+  for (mom_gpu_ctx *c : e->ctx) c->bt_subcycles_used = hsub;
   for (int k = 0; k < nd; ++k) {
     mom_gpu_ctx *ctx = e->ctx[k];
     const KDom &d = ctx->kd;

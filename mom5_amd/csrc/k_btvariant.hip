@@ -26,6 +26,8 @@
 // (-ffp-contract=off), so the results equal the CPU restatement bit for bit.
 #include "mom_internal.h"
 
+#include <algorithm>
+
 namespace {
 
 constexpr double kEpsln = 1.0e-40;   // shared/constants/constants.F90:123
@@ -662,17 +664,13 @@ __global__ __launch_bounds__((VX * btv_nw<CG, PR>(UNI)), 4) void k_btv_block(Btv
 template <bool CG, bool PR>
 int btv_tiles(const KDom &d, bool uni, int h) {
   const int TX = btv_tx(h, d.cyclic_x != 0), TY = btv_ty(h, btv_ry<CG, PR>(uni));
-  return TY < 1 ? 1 << 30 : ((d.NI + TX - 1) / TX) * ((d.NJ + TY - 1) / TY);
+  return ((d.NI + TX - 1) / TX) * ((d.NJ + TY - 1) / TY);
 }
 
-// Rows of scalar constants, where the grid allows it and the lower region of three
-// rows a wavefront keeps enough of an interior (1440x1080 C-grid pressure, 8
-// subcycles a launch: 2.32 ms, 64 x 32 regions 2.45; 10: 5.1 and 3.1; a domain
-// in one round does not mind: 90x60, 10: 186 and 214 us).
-template <bool CG, bool PR>
-bool rows_uniform(const mom_gpu_ctx *ctx, int hsub) {
-  if (!(CG ? ctx->btv_rows_ok : ctx->bt_rows_ok)) return false;
-  return btv_r<CG, PR>(true) == 2 || hsub <= 8 || btv_tiles<CG, PR>(ctx->kd, true, hsub) <= 256;
+// Rows of scalar constants, where the grid allows it.
+template <bool CG>
+bool rows_uniform(const mom_gpu_ctx *ctx) {
+  return CG ? ctx->btv_rows_ok : ctx->bt_rows_ok;
 }
 
 // nsub = hsub subcycles a launch; the state alternates between two sets of
@@ -686,7 +684,7 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
   unsigned char *mask = (unsigned char *)(w + 7 * P2);    // the place of cori1
   double *xb[2] = {w, w + P2}, *ub[2] = {w + 2 * P2, w + 4 * P2};
   double *fb[2] = {w + 8 * P2, w + 18 * P2};              // 4 planes each: 8-11, 18-21
-  const bool uni = rows_uniform<CG, PR>(ctx, hsub);
+  const bool uni = rows_uniform<CG>(ctx);
   double *rowc = uni ? w + 7 * P2 + (P2 + 7) / 8 : nullptr;   // behind the masks
   hipLaunchKernelGGL((k_btv_sfmask<CG, PR>), dim3((d.NI + 255) / 256, d.NJ), dim3(256), 0, s, a,
                      mask, rowc);
@@ -718,8 +716,10 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
   return MOM_GPU_OK;
 }
 
-// Subcycles a launch: as set, otherwise the most with one round of regions, when a
-// launch's time is its latency, and 5 or 6 above.  80 subcycles, us alone: scalar
+// Subcycles a launch: the most with one round of regions, when a launch's time is its
+// latency, and 5 or 6 above; no more than the knob, where it is set (it is
+// tuned on pred_corr_tropic_depth_bgrid's own kernel, whose regions hold more
+// subcycles: 10 a launch at 1440x1080 C-grid pressure are 5.1 ms, 8 2.32).  80 subcycles, us alone: scalar
 // rows (two blocks a CU, at most 256 regions, at most 10) 90x60 C-grid pressure 254
 // at 5, 186 at 10; 360x240 256 at 5, 221 at 7, 285 at 8; 517x389 388 at 5, 326
 // at 7, but among three states in turn 184 and 211; 1440x1080 1709 at 5, 1748 at
@@ -728,12 +728,12 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
 // not depend on it.
 template <bool CG, bool PR>
 int blocked_depth(const mom_gpu_ctx *ctx) {
-  if (ctx->tune.bt_subcycles_set) return ctx->tune.bt_subcycles_per_launch;
-  const bool uni = (CG ? ctx->btv_rows_ok : ctx->bt_rows_ok) && btv_r<CG, PR>(true) == 3;
+  const int knob = ctx->tune.bt_subcycles_per_launch;
+  const bool uni = rows_uniform<CG>(ctx) && btv_r<CG, PR>(true) == 3;
   const int most = uni ? 256 : 128, least = uni ? 5 : 6;
   int h = uni ? 10 : 12;
   while (h > least && btv_tiles<CG, PR>(ctx->kd, uni, h) > most) --h;
-  return h;
+  return knob < 0 ? h : std::min(h, knob);
 }
 
 // Tail (:2846-2894): the time means, each halo-updated, and
@@ -831,7 +831,9 @@ int run_variant(mom_gpu_ctx *ctx, const mom_gpu_bt_params_t *p, const mom_gpu_bt
   hipStream_t s = ctx->stream;
   const dim3 grid((d.NI + 63) / 64, d.NJ), block(64);
   const int nts = p->nts, hsub = blocked_depth<CG, PR>(ctx);
-  if (hsub > 0 && !d.cyclic_y && (!d.cyclic_x || d.ni >= MIN_NI)) {
+  const bool blocked = hsub > 0 && !d.cyclic_y && (!d.cyclic_x || d.ni >= MIN_NI);
+  ctx->bt_subcycles_used = blocked ? hsub : 0;
+  if (blocked) {
     const int rc = run_blocked(ctx, a, nts, p->stepping_a, hsub);
     if (rc) return rc;
   } else {

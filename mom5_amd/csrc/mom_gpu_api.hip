@@ -85,9 +85,10 @@ int mom_gpu_memset(void *ptr, int value, size_t bytes) {
 static int *tuning_slot(mom_gpu_ctx *ctx, const char *knob, int *lo, int *hi) {
   if (!knob) return nullptr;
   if (!std::strcmp(knob, "barotropic_subcycles_per_launch")) {
-    *lo = 0; *hi = 12;
+    *lo = -1; *hi = 12;
     return &ctx->tune.bt_subcycles_per_launch;
   }
+  if (!std::strcmp(knob, "barotropic_subcycles_used")) return &ctx->bt_subcycles_used;
   if (!std::strcmp(knob, "mdfl_rows_per_wave")) {
     *lo = 1; *hi = 4;
     return &ctx->tune.mdfl_rows_per_wave;
@@ -148,6 +149,7 @@ int mom_gpu_set_tuning(mom_gpu_ctx_t *ctx, const char *knob, int value) {
   int lo = 0, hi = 0;
   int *slot = tuning_slot(ctx, knob, &lo, &hi);
   REQUIRE(ctx, slot, "mom_gpu_set_tuning: unknown knob '%s'", knob ? knob : "(null)");
+  REQUIRE(ctx, slot != &ctx->bt_subcycles_used, "mom_gpu_set_tuning: %s can only be read", knob);
   REQUIRE(ctx, value >= lo && value <= hi, "mom_gpu_set_tuning: %s=%d outside [%d,%d]", knob,
           value, lo, hi);
   REQUIRE(ctx, slot != &ctx->tune.mdfl_rows_per_wave || value == 1 || value == 2 || value == 4,
@@ -167,7 +169,6 @@ int mom_gpu_set_tuning(mom_gpu_ctx_t *ctx, const char *knob, int value) {
                    value == 5 || value == 6 || value == 8 || value == 10,
           "mom_gpu_set_tuning: step_group_f32 must be 1, 2, 4, 5, 6, 8 or 10");
   *slot = value;
-  if (slot == &ctx->tune.bt_subcycles_per_launch) ctx->tune.bt_subcycles_set = 1;
   return MOM_GPU_OK;
 }
 
@@ -349,8 +350,8 @@ int mom_gpu_create(const mom_gpu_domain_t *dom, const mom_gpu_grid_t *grid, mom_
   k.P2 = k.NI * k.NJ;
   k.cyclic_x = dom->cyclic_x ? 1 : 0;
   k.cyclic_y = dom->cyclic_y ? 1 : 0;
-  c->tune.bt_subcycles_per_launch = 5;
-  c->tune.bt_subcycles_set = 0;
+  c->tune.bt_subcycles_per_launch = -1;
+  c->bt_subcycles_used = -1;
   c->tune.mdfl_rows_per_wave = 1;
   c->tune.step_group_f64 = 2;
   c->tune.step_group_f32 = 10;

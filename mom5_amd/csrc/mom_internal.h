@@ -204,8 +204,7 @@ struct mom_gpu_ctx {
   int red_n;
   // launch-shape knobs (mom_gpu_set_tuning)
   struct {
-    int bt_subcycles_per_launch;   // 0: one launch per phase per subcycle
-    int bt_subcycles_set;          // 1 once mom_gpu_set_tuning gave it; else chosen per call
+    int bt_subcycles_per_launch;   // -1: chosen per call; 0: one launch per phase per subcycle
     int mdfl_rows_per_wave;        // 2 or 4 region rows per wavefront
     int step_group_f64;            // FP64 tracers per pass of the batched step (1, 2)
     int step_group_f32;            // FP32 tracers per pass (1, 2, 4)
@@ -220,6 +219,7 @@ struct mom_gpu_ctx {
     int step_streams;              // 2: a step's FP32 tracers on the second stream
     int bt_land_tiles;             // blocked barotropic: all-land tiles take the short path (0, 1)
   } tune;
+  int bt_subcycles_used;           // of the last barotropic call (-1: none yet)
   char err[512];
 };
 

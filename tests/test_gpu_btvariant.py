@@ -178,3 +178,28 @@ def test_variant_blocked_uniform_rows(ni, nj, cyclic, cgrid, press, uniform):
         want = want or got
         for name, a, b in zip(("x_bar", "udrho", "conv_rho_ud_t"), got, want):
             assert np.array_equal(_bits(a), _bits(b)), (name, hsub)
+
+
+def test_variants_take_no_deeper_launches_than_they_would_choose():
+    """A depth pinned for the depth-based B-grid's kernel bounds the variants' own
+    choice and does not replace it (their regions lose their interior sooner)."""
+    from mom5_amd import DeviceArray, OceanGPU
+    from mom5_amd.synth import make_case
+    c = make_case(700, 500, 2, seed=65, land_frac=0.3, barotropic=True)
+    fl = _inputs(c, True, True, seed=13)
+    H, sh = DeviceArray.from_host, fl["patm"].shape
+    kw = {k: H(v) for k, v in fl.items() if v is not None and k not in ("udrho", "xbar_tau")}
+    xbar, ud = H(fl["xbar_tau"]), H(fl["udrho"])
+    g = OceanGPU(c.dom, c.grid)
+    out = DeviceArray(sh), DeviceArray((2,) + sh), DeviceArray(sh)
+    used = []
+    for n in (-1, 12, 10, 3, 0):
+        print(f"[C-grid pressure 700x500, knob {n}]", flush=True)
+        g.set_tuning("barotropic_subcycles_per_launch", n)
+        g.update_ocean_barotropic_variant(
+            cgrid=True, pressure_based=True, nts=13, dtbt=c.dtbt, x_bar_tau=xbar, udrho_tau=ud,
+            x_bar_taup1=out[0], udrho_taup1=out[1], conv_rho_ud_t=out[2], **kw)
+        g.sync()
+        used.append(g.get_tuning("barotropic_subcycles_used"))
+    assert used[0] in range(4, 9) and used == [used[0]] * 3 + [3, 0]
+    g.close()

@@ -573,3 +573,56 @@ def test_tmask_limit_levels_a_thread(oracle_lib, ni, nj, nk):
     for a, b in zip(outs, orc.tmask_limit(Ts, lo, hi, 0, 1, True)):
         same(a.to_host(), b)
     gpu.close()
+
+
+def test_automatic_subcycles_are_a_value_of_the_knob():
+    """barotropic_subcycles_per_launch reads -1 (chosen by size) until set, can be
+    read, changed and put back, and the depth a call used can be read."""
+    from mom5_amd import DeviceArray, MomGpuError, OceanGPU
+    from mom5_amd.synth import make_case
+    print("[automatic subcycles]", flush=True)
+    case = make_case(90, 60, 2, land_frac=0.3, nts=24, seed=6)
+    f = {k: DeviceArray.from_host(v) for k, v in case.fields.items() if isinstance(v, np.ndarray)}
+    gpu, knob, used = OceanGPU(case.dom, case.grid), "barotropic_subcycles_per_launch", \
+        "barotropic_subcycles_used"
+    shp = case.grid["dxu"].shape
+    out = DeviceArray(shp), DeviceArray((2,) + shp), DeviceArray(shp)
+
+    def call():
+        gpu.update_ocean_barotropic(
+            nts=case.nts, dtbt=case.dtbt, eta_t_bar_tau=f["eta_t_bar"], udrho_tau=f["udrho"],
+            forcing_bt=f["forcing_bt"], thicku=f["thicku"], patm=f["patm"], pme=f["pme"],
+            river=f["river"], source=f["source"], eta_smooth=f["eta_smooth"], rho_g=f["rho_g"],
+            eta_t_bar_taup1=out[0], udrho_taup1=out[1], conv_rho_ud_t=out[2])
+        gpu.sync()
+        return gpu.get_tuning(used)
+
+    saved = gpu.get_tuning(knob)
+    assert saved == -1 and gpu.get_tuning(used) == -1
+    chosen = call()
+    assert chosen > 5                # a domain of a few tiles takes deep launches
+    for n in (3, 12, 0):
+        gpu.set_tuning(knob, n)
+        assert gpu.get_tuning(knob) == n and call() == n
+    gpu.set_tuning(knob, saved)
+    assert gpu.get_tuning(knob) == -1 and call() == chosen
+    for k, n in ((knob, -2), (knob, 13), (used, 5), (used, -1)):
+        with pytest.raises(MomGpuError):
+            gpu.set_tuning(k, n)
+    assert call() == chosen
+    gpu.close()
+
+
+def test_autotune_tries_the_automatic_subcycles():
+    from mom5_amd.step import BatchedStep
+    from mom5_amd.synth import make_case
+    from mom5_amd.tune import autotune
+    print("[autotune, automatic subcycles]", flush=True)
+    case = make_case(60, 40, 4, land_frac=0.3, nts=24, seed=6, stf_scale=1e-3)
+    st = BatchedStep(case)
+    knob = "barotropic_subcycles_per_launch"
+    rep = autotune(st, reps=1)["barotropic"]
+    assert rep["default"] == {knob: -1}
+    assert sorted(t[knob] for t in rep["tried"]) == list(range(-1, 13))
+    assert st.gpu.get_tuning(knob) == rep["best"][knob]
+    st.gpu.close()
