@@ -115,15 +115,15 @@ __global__ __launch_bounds__(RX *NW) void k_quick_step(QStepJob J, int per_xcd) 
   if (xface) {
     const double *w = J.qw + ox;
     qx0 = w[0]; qx1 = w[P2];
-    cxp0 = w[4 * P2]; cxp1 = w[5 * P2]; cxp2 = w[6 * P2];
-    cxn0 = w[7 * P2]; cxn1 = w[8 * P2]; cxn2 = w[9 * P2];
+    cxp0 = w[plane_at(4, P2)]; cxp1 = w[plane_at(5, P2)]; cxp2 = w[plane_at(6, P2)];
+    cxn0 = w[plane_at(7, P2)]; cxn1 = w[plane_at(8, P2)]; cxn2 = w[plane_at(9, P2)];
     dyte = J.dyte[ox];
   }
   if (yface) {
     const double *w = J.qw + oy;
-    qy0 = w[2 * P2]; qy1 = w[3 * P2];
-    cyp0 = w[10 * P2]; cyp1 = w[11 * P2]; cyp2 = w[12 * P2];
-    cyn0 = w[13 * P2]; cyn1 = w[14 * P2]; cyn2 = w[15 * P2];
+    qy0 = w[plane_at(2, P2)]; qy1 = w[plane_at(3, P2)];
+    cyp0 = w[plane_at(10, P2)]; cyp1 = w[plane_at(11, P2)]; cyp2 = w[plane_at(12, P2)];
+    cyn0 = w[plane_at(13, P2)]; cyn1 = w[plane_at(14, P2)]; cyn2 = w[plane_at(15, P2)];
     dxtn = J.dxtn[oy];
   }
   const double datr = cell ? J.datr[off] : 0.0;

@@ -60,7 +60,7 @@ __global__ void k_quicker_init(KDom d, const double *__restrict__ dxt,
     v[15] = y0 * y1 / ((y0 + 2.0 * y1 + y2) * (y0 + y1));
   }
 #pragma unroll
-  for (int n = 0; n < 16; ++n) qw[o + n * P2] = v[n];
+  for (int n = 0; n < 16; ++n) qw[o + plane_at(n, P2)] = v[n];
 }
 
 __global__ void k_quicker_init_z(int nk, const double *__restrict__ dzt, double *__restrict__ qz) {
@@ -158,15 +158,15 @@ __global__ __launch_bounds__(QRX *NW) void k_quicker_horz(
   if (xface) {
     const double *w = qw + raw;
     qx0 = w[0]; qx1 = w[P2];
-    cxp0 = w[4 * P2]; cxp1 = w[5 * P2]; cxp2 = w[6 * P2];
-    cxn0 = w[7 * P2]; cxn1 = w[8 * P2]; cxn2 = w[9 * P2];
+    cxp0 = w[plane_at(4, P2)]; cxp1 = w[plane_at(5, P2)]; cxp2 = w[plane_at(6, P2)];
+    cxn0 = w[plane_at(7, P2)]; cxn1 = w[plane_at(8, P2)]; cxn2 = w[plane_at(9, P2)];
     dyte = dyte_a[raw];
   }
   if (yface) {
     const double *w = qw + raw;
-    qy0 = w[2 * P2]; qy1 = w[3 * P2];
-    cyp0 = w[10 * P2]; cyp1 = w[11 * P2]; cyp2 = w[12 * P2];
-    cyn0 = w[13 * P2]; cyn1 = w[14 * P2]; cyn2 = w[15 * P2];
+    qy0 = w[plane_at(2, P2)]; qy1 = w[plane_at(3, P2)];
+    cyp0 = w[plane_at(10, P2)]; cyp1 = w[plane_at(11, P2)]; cyp2 = w[plane_at(12, P2)];
+    cyn0 = w[plane_at(13, P2)]; cyn1 = w[plane_at(14, P2)]; cyn2 = w[plane_at(15, P2)];
     dxtn = dxtn_a[raw];
   }
   const double datr = cell ? datr_a[raw] : 0.0;

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "mom5_gpu.h"
+#include "planes.h"
 #include "table_cache.h"
 
 // Compact domain description passed to kernels by value.  Compute-domain
