@@ -334,6 +334,10 @@ int mom_gpu_create(const mom_gpu_domain_t *dom, const mom_gpu_grid_t *grid, mom_
   const long long cells = (long long)(ni + 2) * (nj + 2) * (dom->nk + 1);
   if (cells >= (1LL << 31))
     return mom_fail(nullptr, MOM_GPU_ERR_ARG, "mom_gpu_create: domain too large for 32-bit offsets");
+  if (!level_fits((long long)(ni + 2) * (nj + 2)))
+    return mom_fail(nullptr, MOM_GPU_ERR_ARG,
+                    "mom_gpu_create: a level of %d x %d points does not fit 32-bit byte offsets",
+                    ni + 2, nj + 2);
   const double *need[] = {grid->dxt, grid->dyt, grid->dat, grid->datr, grid->dxte, grid->dyte,
                           grid->dxtn, grid->dytn, grid->dxu, grid->dyu, grid->dxur, grid->dyur,
                           grid->f, grid->dzt};

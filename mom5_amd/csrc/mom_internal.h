@@ -118,8 +118,8 @@ __host__ __device__ inline float fmxf(float a, float b) { return (b > a) ? b : a
 
 // Level-sliced addressing: a buffer descriptor of the level (the array plus
 // the level's offset, in scalar registers) and a 32-bit byte offset of the
-// point within the level, so that no lane carries a 64-bit address.  A level
-// of the largest domain is far below 4 GiB.
+// point within the level, so that no lane carries a 64-bit address.  A level is
+// below 4 GiB: mom_gpu_create refuses others (level_fits).
 __device__ inline __amdgpu_buffer_rsrc_t lvl_rsrc(const void *p) {
   // raw buffer: stride 0, 4 GiB of records, 32-bit data format (CDNA)
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, -1, 0x00020000);

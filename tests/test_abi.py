@@ -66,3 +66,22 @@ def test_product_has_no_cpu_fallback():
             if fn.endswith((".py", ".hip", ".h", ".F90", ".cpp")):
                 txt = open(os.path.join(dirpath, fn)).read()
                 assert "oracle" not in txt.replace("Oracle", ""), fn
+
+
+def test_create_rejects_levels_past_32_bit_byte_offsets():
+    """Two levels of 23171 x 23171 points (4 GiB of FP64 and more) pass the check of
+    all levels' points but not that of a level's bytes; of 23170 x 23170 both
+    (the call then misses its grid).  Nothing reaches the GPU."""
+    from mom5_amd import _lib
+    lib = _lib.load()
+
+    def create(n):
+        dom = _lib.Domain(isd=0, ied=n - 1, jsd=0, jed=n - 1, isc=1, iec=n - 2, jsc=1, jec=n - 2,
+                          nk=2, cyclic_x=1, cyclic_y=0)
+        ctx = C.c_void_p()
+        assert lib.mom_gpu_create(C.byref(dom), C.byref(_lib.Grid()), C.byref(ctx)) == -1
+        return lib.mom_gpu_last_error(None)
+
+    assert 23170 ** 2 < 2 ** 29 <= 23171 ** 2
+    assert b"32-bit byte offsets" in create(23171)
+    assert b"a grid field is NULL" in create(23170)
