@@ -446,7 +446,7 @@ def run_mixed(args, w):
         if twin:
             idx = [n for n in range(ntr) if not is64[n]]
             h = -(-nk // 2)
-            h = next(v for v in (8, 16, 24, 32, 40) if v >= h)
+            h = next(v for v in (8, 12, 16, 20, 23, 26, 29, 32, 35, 38, 40) if v >= h)
             key = f"k_vdiff_twin<{h}>"
             what = ("implicit vertical diffusion of the FP32 tracers, two wavefronts per "
                     "column, levels in registers")
@@ -661,7 +661,8 @@ def run_plain(args, w):
     achieved = kb / (k_ms / 1e3) / 1e9
     roof = dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                 frac=round(achieved / HBM_PEAK_GBS, 4), traffic=None,
-                kernel="k_mdfl (MDFL-Sweby advection, one tracer)",
+                kernel=("k_step<double, 1, 1, 16>" if g.get_tuning("mdfl_rows_per_wave") == 1
+                        else "k_mdfl") + " (MDFL-Sweby tendency of one tracer)",
                 kernel_ms=round(k_ms, 4), bytes_per_launch=kb)
     log(f"step {ms:.3f} ms; mdfl launch {k_ms:.4f} ms")
     cfg = {"workload": w["name"], "grid": [case.ni, case.nj, case.nk], "tracers": ntr,
