@@ -570,7 +570,10 @@ __global__ __launch_bounds__(256) void k_bt_land(KDom d, const unsigned char *__
 
 // bt_tile for a domain whose dxu, dyu, datr, dxur, dyur and f are the same, bit for
 // bit, along every row (spherical grids: launch_check_recip).  A row's constants
-// are then wavefront-uniform and lie in scalar registers, x neighbours come by
+// are then wavefront-uniform and need no vector register a lane: they lie in scalar
+// registers, as far as those reach (the compiler keeps 35 of them in lanes of vector
+// registers with three rows a wavefront and 109 with four, whose instance
+// also has 12 B of scratch).  x neighbours come by
 // lane shifts, y neighbours from the thread's own rows but for one row a
 // wavefront each way (LDS).  What bounds it: memory a launch (18 planes once, the
 // nine of them that regions share up to twice) against 54 FP64 instructions a
@@ -581,7 +584,8 @@ __global__ __launch_bounds__(256) void k_bt_land(KDom d, const unsigned char *__
 // block of 16 wavefronts, 2 rows 9.8 (6), 3 rows 8.2 (7), 4 rows 8.1 (10); 12
 // wavefronts of 2 rows 11.6 (5), 10 of 3 rows 11.0 (6); 8 of 3 rows 8.4 (6), 8 of
 // 4 rows 8.0 (6), 7.8 with every other launch backwards.  517 x 389, 80
-// subcycles, three states in turn: 241 us (bt_tile) to 121.
+// subcycles: 286 us (bt_tile) to 254 alone, 241 to 121 among three states in turn
+// (bt_plan).
 // The same values as bt_tile, instructions saved:
 // - tmask into datr and umask into thicku: x*m is x or a zero of x's sign, as is
 //   the product's (a NaN stays one); the pressure force's zero loses its sign in
@@ -1150,9 +1154,11 @@ struct BtBufs {
 // not depend on either.  rows: every domain's rows are uniform; h: subcycles asked
 // for, 0 to choose.
 // - While the tiles leave CUs idle a launch's time is its latency, so the deepest
-//   launches win: 90 x 60, 80 subcycles, 5 / 10 a launch: 165 / 120 us (alone),
-//   63 / 50 (three states in turn); 360 x 240, 5 / 7: 178 / 159, 83 / 81; above
-//   one tile a CU, 517 x 389, 5 / 7: 254 / 228 but 126 / 144.  The general tile,
+//   launches win: 90 x 60, 80 subcycles, 5 / 10 a launch: 165 / 120 us alone (one
+//   call, waited for), 63 / 50 among three states in turn (calls queued on the
+//   streams of three contexts, so that one fills what another leaves idle); 360 x
+//   240, 5 / 7: 178 / 159, 83 / 81; above one tile a CU, 517 x 389, 5 / 7: 254 / 228
+//   but 126 / 144 (a deeper launch does more work a point).  The general tile,
 //   one block a CU: 90 x 60, 5 / 12: 256 / 186 and 95 / 69, 360 x 240, 5 / 8:
 //   268 / 214 and 122 / 120, past 128 tiles 517 x 389, 5 / 7: 286 / 255, 241 / 240.
 // - Three rows a wavefront have the shorter chain (90 x 60, 10 a launch: 120 us

@@ -260,8 +260,9 @@ __global__ void k_btv_corrector(BtvArgs<CG, PR> a, int fstau, int fstaup1, doubl
 // row a wavefront and quantity.  The forcing and the thickness are read once a
 // subcycle and lie in LDS too.
 //
-// Grids that do not change along a row (checked at creation) keep a row's
-// constants in scalar registers, so 8 wavefronts of three rows (64 x 24) take at
+// Grids that do not change along a row (checked at creation) take a row's constants
+// by scalar loads (the C-grid pressure instance keeps 75 scalars in lanes of vector
+// registers and has 20 B of scratch), so 8 wavefronts of three rows (64 x 24) take at
 // most 128 registers and two blocks share a CU: one loads while the other steps.
 // Other grids, and the C-grid depth scheme (whose LDS holds two more planes), take
 // 16 wavefronts of two rows (64 x 32), one block a CU.  A subcycle is bound by
@@ -719,13 +720,13 @@ int run_blocked(mom_gpu_ctx *ctx, const BtvArgs<CG, PR> &a, int nts, int step_a,
 // Subcycles a launch: the most with one round of regions, when a launch's time is its
 // latency, and 5 or 6 above; no more than the knob, where it is set (it is
 // tuned on pred_corr_tropic_depth_bgrid's own kernel, whose regions hold more
-// subcycles: 10 a launch at 1440x1080 C-grid pressure are 5.1 ms, 8 2.32).  80 subcycles, us alone: scalar
-// rows (two blocks a CU, at most 256 regions, at most 10) 90x60 C-grid pressure 254
-// at 5, 186 at 10; 360x240 256 at 5, 221 at 7, 285 at 8; 517x389 388 at 5, 326
-// at 7, but among three states in turn 184 and 211; 1440x1080 1709 at 5, 1748 at
-// 6.  Other regions (one block a CU, at most 128, at most 12) 90x60 C-grid depth
-// 291 at 5, 203 at 12; 1440x1080 2167 at 5, 1993 at 6, 2119 at 7.  Results do
-// not depend on it.
+// subcycles: 10 a launch at 1440x1080 C-grid pressure are 5.1 ms, 8 2.32).
+// 80 subcycles, us alone: scalar rows (two blocks a CU, at most 256 regions, at most
+// 10) 90x60 C-grid pressure 254 at 5, 186 at 10; 360x240 256 at 5, 221 at 7, 285 at 8;
+// 517x389 388 at 5, 326 at 7, but among the calls of three contexts queued on their
+// streams 184 and 211; 1440x1080 1709 at 5, 1748 at 6.  Other regions (one block a
+// CU, at most 128, at most 12) 90x60 C-grid depth 291 at 5, 203 at 12; 1440x1080 2167
+// at 5, 1993 at 6, 2119 at 7.  Results do not depend on it.
 template <bool CG, bool PR>
 int blocked_depth(const mom_gpu_ctx *ctx) {
   const int knob = ctx->tune.bt_subcycles_per_launch;

@@ -2013,8 +2013,8 @@ static void launch_twin64(mom_gpu_ctx *ctx, VdJob<double> J, bool kk) {
   const KDom &d = J.d;
   const int per_xcd = ((J.nblocks + 1) / 2 + 7) / 8;   // tile pairs per XCD
   // A small domain's tracers go to blocks of their own while all take one round (two
-  // blocks a CU): step of T and S at 90x60x25 alone 151 us, so 144; among three
-  // states 56.1 and 53.2
+  // blocks a CU): step of T and S at 90x60x25 alone 151 us, so 144; among the
+  // calls of three contexts queued on their streams 56.1 and 53.2
   const int ny = 8 * per_xcd * J.g.n <= 512 ? J.g.n : 1;
   const dim3 grid(8 * per_xcd, ny), block(256);
   with_slots(twin_slots(d.nk), [&](auto H) {

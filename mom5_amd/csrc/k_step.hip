@@ -176,8 +176,9 @@ __device__ __forceinline__ void step_tile(const StepJob<TT> &J, int tile, int ka
   // and y faces read different rows (CY).
   // With the loads at the level's start two FP64 tracers took 1.75 ms at
   // 1440x1080x50; so, and without branches, 1.50 ms, now bound by vector
-  // instructions: 340 a level and wavefront, issued 82% of the time (ten FP32
-  // tracers: 687).  The tracers' loads take no branch: a point outside the
+  // instructions: 340 in a level's code, of which 307 run on average at 3600x2700x75
+  // and issue in 80% of the vector ALUs' cycles (ten FP32 tracers: 687, 636 and
+  // 88%).  The tracers' loads take no branch: a point outside the
   // domain reads past the level's end, a 0 (with the branch, and a window kept as
   // four tracers instead of three and a difference, FP32 took 752 instructions
   // and waited for the loads where the loop closes: pass of T, S and six FP32
@@ -984,7 +985,9 @@ static void add_th_f32(hipStream_t s, const KDom &d, float *out, const double *t
 
 // Level chunks a tile is split into: as many as still take one round of the 256
 // CUs (a tile fills one), at least four levels each (a chunk costs about 1.2
-// levels more).  us of a step or pass alone / among three states in turn:
+// levels more).  us of a step or pass alone (one call, waited for) / among three
+// states in turn (calls queued on the streams of three contexts, so that one fills
+// what another leaves idle):
 //   90x60x25, 10 tiles: one chunk 208 / 83, 6 chunks 154 / 67
 //   240x180x40, T, S and four FP32, 60 tiles: 273 / 135, 4 chunks 136 / 126
 //   360x240x40, T, S and six FP32, 120 tiles: 381 / 264, 2 chunks 269 / 274
